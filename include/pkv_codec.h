@@ -574,11 +574,14 @@ int pkv_blake3(pkv_ctx* ctx, const void* data, uint64_t len, uint8_t out[32]);
  * Host builds of the exact scalar routines the kernels use (test hooks):
  * angle bins of (a[i], b[i]) for pbits, the encode kernels' octant fast path
  * (3-bit bin and whether the pair is safe for it, i.e. kept from the exact
- * formula), and logf / expf over arrays. */
+ * formula), logf / expf over arrays, and the lossy decodes' short forms of
+ * expf (|x| <= 32.5) and of u / 255 (u = 0 .. 255). */
 void pkv_host_angle_bins(const float* a, const float* b, uint64_t n, uint32_t pbits, uint32_t* out);
 void pkv_host_octant_bins(const float* a, const float* b, uint64_t n, uint32_t* bins, uint8_t* safe);
 void pkv_host_logf(const float* x, uint64_t n, float* out);
 void pkv_host_expf(const float* x, uint64_t n, float* out);
+void pkv_host_expf_fused(const float* x, uint64_t n, float* out);
+void pkv_host_div255(const float* u, uint64_t n, float* out);
 /* The fib encode redo's test that f32 rounds every value within |v| 2^-50
  * of v[i] like v[i] (1) or that the exact division must decide (0). */
 void pkv_host_f32_stable_rel50(const double* v, uint64_t n, uint8_t* out);

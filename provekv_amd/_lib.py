@@ -55,7 +55,7 @@ EXPORTS = (
     "pkv_radii_log_bound", "pkv_fb2_n_blocks", "pkv_lloyd_refine", "pkv_blake3_ranges", "pkv_blake3_layer_digests",
     "pkv_blake3_tier_digests", "pkv_blake3",
     "pkv_host_angle_bins", "pkv_host_octant_bins", "pkv_host_logf",
-    "pkv_host_expf", "pkv_host_f32_stable_rel50", "pkv_code_from_json", "pkv_fib_digests", "pkv_host_blake3",
+    "pkv_host_expf", "pkv_host_expf_fused", "pkv_host_div255", "pkv_host_f32_stable_rel50", "pkv_code_from_json", "pkv_fib_digests", "pkv_host_blake3",
 )
 
 
@@ -182,6 +182,8 @@ def _declare(L):
         "pkv_host_logf": ([P, U64, P], None),
         "pkv_host_f32_stable_rel50": ([P, U64, P], None),
         "pkv_host_expf": ([P, U64, P], None),
+        "pkv_host_expf_fused": ([P, U64, P], None),
+        "pkv_host_div255": ([P, U64, P], None),
         "pkv_code_from_json": ([P, P, U64, P, U64, P, P], I32),
         "pkv_fib_digests": ([P, P, P, P], I32),
         "pkv_host_blake3": ([P, U64, P], None),

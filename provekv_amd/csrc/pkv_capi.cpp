@@ -2120,6 +2120,15 @@ void pkv_host_expf(const float* x, uint64_t n, float* out) {
     for (uint64_t i = 0; i < n; ++i) out[i] = og_expf(x[i], tab);
 }
 
+void pkv_host_expf_fused(const float* x, uint64_t n, float* out) {
+    static const uint64_t tab[32] = {PKV_EXP2F_TABLE};
+    for (uint64_t i = 0; i < n; ++i) out[i] = og_expf_fused(x[i], tab);
+}
+
+void pkv_host_div255(const float* u, uint64_t n, float* out) {
+    for (uint64_t i = 0; i < n; ++i) out[i] = div255_f(u[i]);
+}
+
 void pkv_host_f32_stable_rel50(const double* v, uint64_t n, uint8_t* out) {
     for (uint64_t i = 0; i < n; ++i) out[i] = f32_rounding_stable_rel50(v[i]) ? 1 : 0;
 }

@@ -46,16 +46,6 @@ typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 __constant__ LogfEntry c_logf_tab[16] = {PKV_LOGF_TABLE};
 __constant__ uint64_t c_exp2f_tab[32] = {PKV_EXP2F_TABLE};
 
-// u / 255.0f for every u8 code u (radius.rs:139-143), correctly rounded by the
-// compiler at build time: the decode reads it instead of dividing per radius.
-struct Div255 {
-    float v[256];
-    constexpr Div255() : v() {
-        for (int u = 0; u < 256; ++u) v[u] = static_cast<float>(u) / 255.0f;
-    }
-};
-__constant__ Div255 c_div255 = Div255();
-
 // Gap between cheap_logf (below) and logf, per magnitude of the result:
 // g_logb[e] = the largest |cheap_logf(v) - logf(v)| over every normal positive
 // float v whose logf(v) has biased exponent <= e, rounded up to f32.  Measured
@@ -82,8 +72,9 @@ __device__ __forceinline__ uint32_t segment_of(const uint32_t* __restrict__ tile
     return tile_seg ? tile_seg[blk] : find_segment(tile_start, nseg, blk);
 }
 
-__device__ __forceinline__ uint64_t vec_elem_offset(const SegDev& s, uint64_t i) {
-    return s.elem_offset + (i / s.group) * s.stride_outer + (i % s.group) * s.stride_inner;
+__device__ __forceinline__ uint64_t vec_elem_offset(const SegDev& s, uint32_t i) {
+    const uint32_t o = i / s.group;
+    return s.elem_offset + o * s.stride_outer + (i - o * s.group) * s.stride_inner;
 }
 
 __device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int src) {
@@ -148,6 +139,30 @@ __device__ void global_to_lds(uint32_t* lds, const uint8_t* __restrict__ src, ui
             const uint32_t k = k0 + j * WAVE + static_cast<uint32_t>(lane);
             if (k < ndw) lds[k] = sh ? __builtin_amdgcn_alignbyte(w1[j], w0[j], sh) : w0[j];
         }
+    }
+}
+
+// Move nbytes (>= 16, a multiple of 4) from global memory at any byte alignment
+// into LDS (LDS byte 0 == src byte 0, 4-byte aligned), 16 bytes per lane and
+// load; the last load starts early enough to end with the range, so only the
+// range's own bytes are read.  All MAXK loads are issued before the first is
+// waited for.  (Dword loads shifted into place by v_alignbyte took two loads
+// and an extra instruction per 4 bytes.)
+typedef uint32_t v4u_a4 __attribute__((ext_vector_type(4), aligned(4)));
+template <uint32_t MAXK>
+__device__ __forceinline__ void global_to_lds16(uint32_t* lds, const uint8_t* __restrict__ src, uint32_t nbytes,
+                                                int lane) {
+    v4u v[MAXK];
+    const uint32_t last = nbytes - 16u;
+#pragma unroll
+    for (uint32_t k = 0; k < MAXK; ++k) {
+        const uint32_t o = 16u * (k * WAVE + static_cast<uint32_t>(lane));
+        if (o < nbytes) __builtin_memcpy(&v[k], src + min(o, last), 16);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < MAXK; ++k) {
+        const uint32_t o = 16u * (k * WAVE + static_cast<uint32_t>(lane));
+        if (o < nbytes) *reinterpret_cast<v4u_a4*>(lds + (min(o, last) >> 2)) = v[k];
     }
 }
 
@@ -268,6 +283,23 @@ __device__ void stage_rows_out(void* __restrict__ out, const LaunchCommon& lc, c
         if (skip) continue;
         uint64_t off = vec_elem_offset(s, v0 + r);
         store_out4<true>(out, lc, off + 4 * c, *reinterpret_cast<const float4*>(stage + r * PITCH + 4 * c));
+    }
+}
+
+// The same for nv <= 16 rows whose element offsets lane r holds in my_off, rows
+// with a clear bit in `wmask` skipped.
+template <int DIM>
+__device__ __forceinline__ void stage_rows_out_at(void* __restrict__ out, const LaunchCommon& lc, const float* stage,
+                                                  uint64_t my_off, uint32_t nv, uint32_t wmask, int lane) {
+    constexpr int PITCH = DIM + 4;
+    constexpr int Q = DIM / 4;
+    constexpr int RPI = WAVE / Q;
+#pragma unroll
+    for (int k = 0; k < 16 / RPI; ++k) {
+        const uint32_t r = static_cast<uint32_t>(RPI * k + lane / Q), c = static_cast<uint32_t>(lane) % Q;
+        const uint64_t off = shfl_u64(my_off, static_cast<int>(r));
+        if (r < nv && ((wmask >> r) & 1u))
+            store_out4<true>(out, lc, off + 4 * c, *reinterpret_cast<const float4*>(stage + r * PITCH + 4 * c));
     }
 }
 
@@ -1665,6 +1697,47 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
 }
 
 // ------------------------------------------------------------ turbo decode
+// BlockLogU8 radii (turbo-quant/src/radius.rs:128-145) of the NC codes in the
+// words q: r = expf(mn + (mx - mn) * fl(code / 255)).  `ok` gathers the
+// decoder's checks (radius.rs:171-177, polar.rs:127-133).  While every lane
+// of the wave has |mn|, |mx| <= 32 (every radius within e^+-32) each exponent
+// lies within a rounding of [mn, mx], so og_expf_fused gives expf's bits, the
+// radii are finite and positive and only mn <= mx is left to check: 17 VALU
+// operations per radius against about 35 of the general form, which any other
+// wave takes.  The exponentials were most of a lossy decode's arithmetic:
+// 0.36 M head_dim-64 vectors into a bf16 cache 40.3 -> 36.2 us, 4.2 M
+// head_dim-128 vectors to f32 723 -> 610 us (3.55 -> 4.2 TB/s; with the
+// payload loads, row offsets and three-swap transform of
+// turbo_decode_split128_kernel).
+template <int NC>
+__device__ __forceinline__ void radii_u8(const uint32_t (&q)[NC / 4], float mn, float mx, const uint64_t* exp_tab,
+                                         float (&r)[NC], bool& ok) {
+    const float span = mx - mn;
+    const bool narrow = __builtin_fabsf(mn) <= 32.0f && __builtin_fabsf(mx) <= 32.0f;
+    ok &= isfinite_f(mn) && isfinite_f(mx) && !(mn > mx);
+    if (__ballot(!narrow) == 0ull) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const float u = static_cast<float>((q[i >> 2] >> (8 * (i & 3))) & 0xffu);   // v_cvt_f32_ubyte
+            r[i] = og_expf_fused(mn + span * div255_f(u), exp_tab);
+        }
+    } else {
+#pragma unroll 1
+        for (int w = 0; w < NC / 4; ++w) {
+            uint32_t qw = q[0];   // q[w] by selects (a dynamic index would go through scratch)
+#pragma unroll
+            for (int k = 1; k < NC / 4; ++k) qw = k == w ? q[k] : qw;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const float v = og_expf(mn + span * div255_f(static_cast<float>((qw >> (8 * t)) & 0xffu)), exp_tab);
+                ok &= isfinite_f(v) && !(v < 0.0f);
+#pragma unroll
+                for (int k = 0; k < NC / 4; ++k) r[4 * k + t] = k == w ? v : r[4 * k + t];
+            }
+        }
+    }
+}
+
 template <int DIM, int PB>
 __global__ __launch_bounds__(TILE) void turbo_decode_kernel(
     LaunchCommon lc, const uint8_t* __restrict__ wire, void* __restrict__ out,
@@ -1676,13 +1749,11 @@ __global__ __launch_bounds__(TILE) void turbo_decode_kernel(
     extern __shared__ float smem[];
     __shared__ float cs_lds[512];
     __shared__ uint64_t exp_lds[32];
-    __shared__ float div255_lds[256];
 
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
-    for (uint32_t t = threadIdx.x; t < 256; t += blockDim.x) div255_lds[t] = c_div255.v[t];
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1732,7 +1803,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_kernel(
 #pragma unroll
             for (int i = 0; i < PAIRS; ++i) {
                 const uint32_t u = (q[i >> 2] >> (8 * (i & 3))) & 0xffu;
-                r[i] = og_expf(mn + span * div255_lds[u], exp_lds);   // radius.rs:128-145
+                r[i] = og_expf(mn + span * div255_f(static_cast<float>(u)), exp_lds);   // radius.rs:128-145
                 ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);     // polar.rs:127-133
             }
         }
@@ -1808,13 +1879,11 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split_kernel(
     extern __shared__ uint32_t smem_u[];   // per wave: two buffers of turbo_split_buf_words
     __shared__ float cs_lds[32];           // levels <= 16
     __shared__ uint64_t exp_lds[32];
-    __shared__ float div255_lds[256];
 
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
-    for (uint32_t t = threadIdx.x; t < 256; t += blockDim.x) div255_lds[t] = c_div255.v[t];
     __syncthreads();
 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -1914,20 +1983,10 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split_kernel(
                 ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);   // radius.rs:88-104
             }
         } else {
-            const float mn = u2f(pword(8)), mx = u2f(pword(9));
-            ok &= isfinite_f(mn) && isfinite_f(mx) && !(mn > mx);   // radius.rs:171-177
-            const float span = mx - mn;
+            uint32_t q[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t q = pword(4 * h + k);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const uint32_t u = (q >> (8 * t)) & 0xffu;
-                    const int i = 4 * k + t;
-                    r[i] = og_expf(mn + span * div255_lds[u], exp_lds);   // radius.rs:128-145
-                    ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);             // polar.rs:127-133
-                }
-            }
+            for (int k = 0; k < 4; ++k) q[k] = pword(4 * h + k);
+            radii_u8<HP>(q, u2f(pword(8)), u2f(pword(9)), exp_lds, r, ok);
         }
         // this half's 16 angle indices: bits 16 pbits h .. (pbits <= 4: <= 64 bits)
         const uint32_t bit0 = 16u * pbits * static_cast<uint32_t>(h);
@@ -1991,7 +2050,9 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split_kernel(
 
 // Turbo decode at head_dim 128: four lanes per vector as in
 // turbo_encode_qjl128_kernel, one 16-vector group per wave, four workgroups
-// per tile; rows leave through LDS, 512 B contiguous per row.
+// per tile.  Lane q reads the pairs of layout F (8q .. 8q + 7 and 32 + 8q ..
+// 32 + 8q + 7), so the transform is fwht128_inv's three lane swaps per element
+// pair and ends in layout G; the rows leave through LDS, 512 B contiguous each.
 __host__ __device__ constexpr uint32_t turbo_split128_wave_words(uint32_t pwd) {
     return (16 * pwd + 4 > 16 * (128 + 4) + 4) ? 16 * pwd + 4 : 16 * (128 + 4) + 4;
 }
@@ -2007,13 +2068,11 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     extern __shared__ uint32_t smem_u[];   // per wave: 16 payloads, then 16 decoded rows
     __shared__ float cs_lds[512];
     __shared__ uint64_t exp_lds[32];
-    __shared__ float div255_lds[256];
 
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
-    for (uint32_t t = threadIdx.x; t < 256; t += blockDim.x) div255_lds[t] = c_div255.v[t];
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -2037,11 +2096,13 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     if (t0 >= seg.n_vectors) return;
     const uint32_t nv = min(static_cast<uint32_t>(GV), seg.n_vectors - t0);
     uint32_t* sw = smem_u + wave * turbo_split128_wave_words(pwd);
-    global_to_lds(sw, blob + 38 + static_cast<uint64_t>(t0) * plen, nv * plen, lane);
+    global_to_lds16<5>(sw, blob + 38 + static_cast<uint64_t>(t0) * plen, nv * plen, lane);   // <= 16 * 296 B
     wave_sync();
 
     const bool active = static_cast<uint32_t>(n) < nv;
-    const uint32_t* pw = sw + min(static_cast<uint32_t>(n), nv - 1) * pwd;
+    const uint32_t mine = min(static_cast<uint32_t>(n), nv - 1);
+    const uint32_t* pw = sw + mine * pwd;
+    const uint64_t my_off = vec_elem_offset(seg, t0 + mine);
     const bool f32r = lc.radii == PKV_RADII_F32;
     const uint32_t rwords = f32r ? 64u : 64u / 4 + 2;
     bool ok = true;
@@ -2049,32 +2110,30 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     if (f32r) {
 #pragma unroll
         for (int i = 0; i < HP; ++i) {
-            r[i] = u2f(pw[16 * q + i]);
+            r[i] = u2f(pw[(i < 8 ? 8 * q : 24 + 8 * q) + i]);
             ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);   // radius.rs:88-104
         }
     } else {
-        const float mn = u2f(pw[16]), mx = u2f(pw[17]);
-        ok &= isfinite_f(mn) && isfinite_f(mx) && !(mn > mx);   // radius.rs:171-177
-        const float span = mx - mn;
+        uint32_t w[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t w = pw[4 * q + k];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const uint32_t u = (w >> (8 * t)) & 0xffu;
-                const int i = 4 * k + t;
-                r[i] = og_expf(mn + span * div255_lds[u], exp_lds);   // radius.rs:128-145
-                ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);             // polar.rs:127-133
-            }
-        }
+        for (int k = 0; k < 4; ++k) w[k] = pw[(k < 2 ? 2 * q : 6 + 2 * q) + k];
+        radii_u8<HP>(w, u2f(pw[16]), u2f(pw[17]), exp_lds, r, ok);
     }
-    // this quarter's 16 angle indices: bits 16 pbits q .. (pbits <= 4: <= 64 bits)
-    const uint32_t bit0 = 16u * pbits * static_cast<uint32_t>(q);
-    const uint32_t* aw = pw + rwords + (bit0 >> 5);
-    const uint32_t sh = bit0 & 31u;
-    const uint64_t lo64 = static_cast<uint64_t>(aw[0]) | static_cast<uint64_t>(aw[1]) << 32;
-    uint64_t pk = lo64 >> sh;
-    if (sh) pk |= static_cast<uint64_t>(aw[2]) << (64 - sh);
+    // this lane's two runs of 8 angle indices, 8 pbits (<= 32) bits each, at
+    // bits 8 pbits q and 8 pbits (4 + q)
+    uint64_t pk;
+    {
+        const uint32_t nb = 8u * pbits;
+        uint64_t run[2];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const uint32_t bit0 = nb * (static_cast<uint32_t>(q) + 4u * half);
+            const uint32_t* aw = pw + rwords + (bit0 >> 5);
+            const uint64_t v = static_cast<uint64_t>(aw[0]) | static_cast<uint64_t>(aw[1]) << 32;
+            run[half] = (v >> (bit0 & 31u)) & ((1ull << nb) - 1u);
+        }
+        pk = run[0] | run[1] << nb;
+    }
     // the angle field is 64 * pbits bits, a whole number of words: no padding
     // bits to check (bitpack.rs:88-109); nor in the 32/64-bit QJL field
 
@@ -2085,7 +2144,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
         y[2 * i] = r[i] * cs_lds[2 * bin];
         y[2 * i + 1] = r[i] * cs_lds[2 * bin + 1];
     }
-    fwht_quarter(y, q);
+    fwht128_inv(y);   // layout F -> layout G
     const float scale = fwht_scale<DIM>();
     const bool vok = or_quarters(ok ? 0u : 1u, q) == 0u;
     if (active && q == 0 && !vok) status_fail(lc.status, sidx, 1, t0 + n, KIND_CORRUPT);
@@ -2093,19 +2152,19 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     wave_sync();
     float* stage = reinterpret_cast<float*>(sw);
     {
-        float* srow = stage + n * (DIM + 4) + 32 * q;
-        const float4* sp = reinterpret_cast<const float4*>(signs + 32 * q);
+        const uint32_t g0 = 16u * static_cast<uint32_t>(((q & 1) << 1) | (q >> 1)), g1 = 64u + g0;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const float4 sg = sp[k];
-            *reinterpret_cast<float4*>(srow + 4 * k) =
+            const uint32_t e = (k < 4 ? g0 : g1) + 4u * (k & 3);
+            const float4 sg = *reinterpret_cast<const float4*>(signs + e);
+            *reinterpret_cast<float4*>(stage + n * (DIM + 4) + e) =
                 make_float4((y[4 * k] * scale) * sg.x, (y[4 * k + 1] * scale) * sg.y, (y[4 * k + 2] * scale) * sg.z,
                             (y[4 * k + 3] * scale) * sg.w);
         }
     }
-    const uint64_t badm = __ballot(active && q == 0 && !vok);
+    const uint32_t wmask = static_cast<uint32_t>(__ballot(active && q == 0 && vok));
     wave_sync();
-    stage_rows_out<DIM>(out, lc, stage, seg, t0, nv, static_cast<uint32_t>(badm), 0u, lane);
+    stage_rows_out_at<DIM>(out, lc, stage, my_off, nv, wmask, lane);
 }
 
 // ------------------------------------------------------------ scoring on codes
@@ -2209,13 +2268,11 @@ __global__ __launch_bounds__(TILE) void turbo_score_kernel(
     extern __shared__ uint32_t smem_u[];  // per wave: 64 payloads
     __shared__ float2 cs_lds[256];
     __shared__ uint64_t exp_lds[32];
-    __shared__ float div255_lds[256];
 
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < levels; t += blockDim.x)
         cs_lds[t] = make_float2(cs_tab[2 * t], cs_tab[2 * t + 1]);
     if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
-    for (uint32_t t = threadIdx.x; t < 256; t += blockDim.x) div255_lds[t] = c_div255.v[t];
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -2260,7 +2317,7 @@ __global__ __launch_bounds__(TILE) void turbo_score_kernel(
 #pragma unroll
         for (int i = 0; i < PAIRS; ++i) {
             const uint32_t u = (pw[i >> 2] >> (8 * (i & 3))) & 0xffu;
-            r[i] = og_expf(mn + span * div255_lds[u], exp_lds);
+            r[i] = og_expf(mn + span * div255_f(static_cast<float>(u)), exp_lds);
             ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);
         }
         w = QW + 2;
@@ -2360,7 +2417,6 @@ turbo_score_lut_kernel(
     extern __shared__ uint32_t smem_u[];
     __shared__ float2 cs_lds[16];
     __shared__ uint64_t exp_lds[32];
-    __shared__ float div255_lds[256];
 
     constexpr uint32_t levels = 1u << pbits;
     if (threadIdx.x < 16)
@@ -2368,8 +2424,7 @@ turbo_score_lut_kernel(
                                                    : make_float2(0.0f, 0.0f);
     if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
     if (LOSSY)
-        for (uint32_t t = threadIdx.x; t < 256; t += blockDim.x) div255_lds[t] = c_div255.v[t];
-    __syncthreads();   // the tables are read by every wave (radii below, the (cos, sin) terms later)
+        __syncthreads();   // the tables are read by every wave (radii below, the (cos, sin) terms later)
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t blk = blockIdx.x;
@@ -2428,7 +2483,7 @@ turbo_score_lut_kernel(
 #pragma unroll
         for (int i = 0; i < PAIRS; ++i) {
             const uint32_t u = (rw[i >> 2] >> (8 * (i & 3))) & 0xffu;
-            r[i] = og_expf(mn + span * div255_lds[u], exp_lds);
+            r[i] = og_expf(mn + span * div255_f(static_cast<float>(u)), exp_lds);
             ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);
         }
     }

@@ -300,3 +300,22 @@ def test_redo_xhat_stability_test_is_sufficient():
     # random rotated components: refused about 17 times in 2^29
     r = rng.standard_normal(200_000) / 8.0
     assert _stable_rel50(r).mean() > 0.9999
+
+
+def test_lossy_decode_short_forms():
+    """The lossy decodes' fused expf equals the restated expf for |x| <= 32.5
+    (a stride through every such float of both signs, and every float near
+    the kernels' bound of 32), and their u / 255 the quotient of every code."""
+    def same(bits):
+        x = np.ascontiguousarray(bits.astype(np.uint32)).view(np.float32)
+        out = np.zeros_like(x)
+        L.lib().pkv_host_expf_fused(x.ctypes.data, x.size, out.ctypes.data)
+        return np.array_equal(out.view(np.uint32), _host_expf(x).view(np.uint32))
+    edge = int(np.float32(32.5).view(np.uint32))
+    for sign in (0, 1 << 31):
+        assert same(np.arange(0, edge + 1, 211, dtype=np.int64) | sign)
+        assert same(np.arange(int(np.float32(31.9).view(np.uint32)), edge + 1, dtype=np.int64) | sign)
+    u = np.arange(256, dtype=np.float32)
+    q = np.zeros_like(u)
+    L.lib().pkv_host_div255(u.ctypes.data, u.size, q.ctypes.data)
+    assert np.array_equal(q, u / np.float32(255.0))
