@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 #include "pkv_internal.h"
@@ -147,22 +148,25 @@ __device__ void global_to_lds(uint32_t* lds, const uint8_t* __restrict__ src, ui
 // load; the last load starts early enough to end with the range, so only the
 // range's own bytes are read.  All MAXK loads are issued before the first is
 // waited for.  (Dword loads shifted into place by v_alignbyte took two loads
-// and an extra instruction per 4 bytes.)
+// and an extra instruction per 4 bytes.)  SKIP: loads wholly past the range
+// are left out (for callers whose usual range is well below MAXK loads;
+// otherwise the test costs more than the rare repeat).
 typedef uint32_t v4u_a4 __attribute__((ext_vector_type(4), aligned(4)));
-template <uint32_t MAXK>
+template <uint32_t MAXK, bool SKIP>
 __device__ __forceinline__ void global_to_lds16(uint32_t* lds, const uint8_t* __restrict__ src, uint32_t nbytes,
                                                 int lane) {
     v4u v[MAXK];
-    const uint32_t last = nbytes - 16u;
+    uint32_t o[MAXK];
 #pragma unroll
-    for (uint32_t k = 0; k < MAXK; ++k) {
-        const uint32_t o = 16u * (k * WAVE + static_cast<uint32_t>(lane));
-        if (o < nbytes) __builtin_memcpy(&v[k], src + min(o, last), 16);
+    for (uint32_t k = 0; k < MAXK; ++k) {   // lanes past the end repeat the last 16 bytes
+        if (SKIP && 16u * k * WAVE >= nbytes) break;   // wave-uniform
+        o[k] = min(16u * (k * WAVE + static_cast<uint32_t>(lane)), nbytes - 16u);
+        __builtin_memcpy(&v[k], src + o[k], 16);
     }
 #pragma unroll
     for (uint32_t k = 0; k < MAXK; ++k) {
-        const uint32_t o = 16u * (k * WAVE + static_cast<uint32_t>(lane));
-        if (o < nbytes) *reinterpret_cast<v4u_a4*>(lds + (min(o, last) >> 2)) = v[k];
+        if (SKIP && 16u * k * WAVE >= nbytes) break;
+        *reinterpret_cast<v4u_a4*>(lds + (o[k] >> 2)) = v[k];
     }
 }
 
@@ -1706,7 +1710,7 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
 // operations per radius against about 35 of the general form, which any other
 // wave takes.  The exponentials were most of a lossy decode's arithmetic:
 // 0.36 M head_dim-64 vectors into a bf16 cache 40.3 -> 36.2 us, 4.2 M
-// head_dim-128 vectors to f32 723 -> 610 us (3.55 -> 4.2 TB/s; with the
+// head_dim-128 vectors to f32 720 -> 605 us (3.55 -> 4.2 TB/s; with the
 // payload loads, row offsets and three-swap transform of
 // turbo_decode_split128_kernel).
 template <int NC>
@@ -2096,7 +2100,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     if (t0 >= seg.n_vectors) return;
     const uint32_t nv = min(static_cast<uint32_t>(GV), seg.n_vectors - t0);
     uint32_t* sw = smem_u + wave * turbo_split128_wave_words(pwd);
-    global_to_lds16<5>(sw, blob + 38 + static_cast<uint64_t>(t0) * plen, nv * plen, lane);   // <= 16 * 296 B
+    global_to_lds16<5, true>(sw, blob + 38 + static_cast<uint64_t>(t0) * plen, nv * plen, lane);   // <= 16 * 296 B
     wave_sync();
 
     const bool active = static_cast<uint32_t>(n) < nv;
@@ -2180,52 +2184,69 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
 //         of Rust's f32 Sum (an all-zero sum keeps the sign of its terms).
 // A query with a non-finite input, rotated or projected value marks status
 // word 0 of segment 0 with its index (turbo.rs:330, polar.rs:341, qjl.rs:280).
+// The call is one latency chain, so the two parts run on two waves of the
+// query's workgroup, and a lane loads its whole row of G before the fold
+// starts (5.5 us with both on one wave and the row loaded 16 values at a
+// time, 256 queries at DIM 128; 3.8 us so).
 template <int DIM>
-__global__ __launch_bounds__(WAVE) void turbo_prepare_kernel(const float* __restrict__ q, uint32_t nq,
-                                                             float* __restrict__ out, const float* __restrict__ signs,
-                                                             const float* __restrict__ G, uint32_t proj,
-                                                             uint32_t mode, float rscale, uint32_t* status) {
-    __shared__ float v[DIM];
-    __shared__ float raw[DIM];
-    const uint32_t qi = blockIdx.x, lane = threadIdx.x;
+__global__ __launch_bounds__(2 * WAVE) void turbo_prepare_kernel(const float* __restrict__ q, uint32_t nq,
+                                                                 float* __restrict__ out,
+                                                                 const float* __restrict__ signs,
+                                                                 const float* __restrict__ G, uint32_t proj,
+                                                                 uint32_t mode, float rscale, uint32_t* status) {
+    __shared__ __align__(16) float buf[2][DIM];
+    const uint32_t qi = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     if (qi >= nq) return;
+    float* v = buf[wave];   // wave 0: the vector under rotation; wave 1: the raw query
     const float* src = q + static_cast<uint64_t>(qi) * DIM;
     const uint32_t W = DIM + (mode ? proj : 0u);
     float* dst = out + static_cast<uint64_t>(qi) * W;
     bool bad = false;
+    if (wave == 0) {
 #pragma unroll
-    for (int c = lane; c < DIM; c += WAVE) {
-        const float x = src[c];
-        raw[c] = x;
-        v[c] = x * signs[c];
-        bad |= !isfinite_f(x);
-    }
-    wave_sync();
-#pragma unroll
-    for (int step = 1; step < DIM; step *= 2) {
-#pragma unroll
-        for (int bf = lane; bf < DIM / 2; bf += WAVE) {
-            const int i = (bf / step) * 2 * step + bf % step, j = i + step;
-            const float a = v[i], b = v[j];
-            v[i] = a + b;
-            v[j] = a - b;
+        for (int c = lane; c < DIM; c += WAVE) {
+            const float x = src[c];
+            v[c] = x * signs[c];
+            bad |= !isfinite_f(x);
         }
         wave_sync();
-    }
 #pragma unroll
-    for (int c = lane; c < DIM; c += WAVE) {
-        const float y = v[c] * rscale;
-        dst[c] = y;
-        bad |= !isfinite_f(y);
-    }
-    if (mode) {
-        for (uint32_t j = lane; j < proj; j += WAVE) {
-            const float* g = G + static_cast<uint64_t>(j) * DIM;
-            float acc = -0.0f;
-#pragma unroll 16
-            for (int c = 0; c < DIM; ++c) acc = acc + g[c] * raw[c];
-            dst[DIM + j] = acc;
-            bad |= !isfinite_f(acc);
+        for (int step = 1; step < DIM; step *= 2) {
+#pragma unroll
+            for (int bf = lane; bf < DIM / 2; bf += WAVE) {
+                const int i = (bf / step) * 2 * step + bf % step, j = i + step;
+                const float a = v[i], b = v[j];
+                v[i] = a + b;
+                v[j] = a - b;
+            }
+            wave_sync();
+        }
+#pragma unroll
+        for (int c = lane; c < DIM; c += WAVE) {
+            const float y = v[c] * rscale;
+            dst[c] = y;
+            bad |= !isfinite_f(y);
+        }
+    } else {   // launched only with QJL
+        const uint32_t j = lane < proj ? lane : 0u;   // proj is 32 or 64
+        float4 g[DIM / 4];
+#pragma unroll
+        for (int c = 0; c < DIM / 4; ++c) g[c] = reinterpret_cast<const float4*>(G + static_cast<uint64_t>(j) * DIM)[c];
+#pragma unroll
+        for (int c = lane; c < DIM; c += WAVE) v[c] = src[c];
+        wave_sync();
+        float acc = -0.0f;
+#pragma unroll
+        for (int c = 0; c < DIM / 4; ++c) {
+            const float4 x = reinterpret_cast<const float4*>(v)[c];
+            acc = acc + g[c].x * x.x;
+            acc = acc + g[c].y * x.y;
+            acc = acc + g[c].z * x.z;
+            acc = acc + g[c].w * x.w;
+        }
+        if (lane < proj) {
+            dst[DIM + lane] = acc;
+            bad = !isfinite_f(acc);
         }
     }
     if (__ballot(bad) != 0ull && lane == 0 && status) status_fail(status, 0, 0, qi, KIND_NONFINITE_INPUT);
@@ -2391,192 +2412,239 @@ __global__ __launch_bounds__(TILE) void turbo_score_kernel(
     if (store && !fin) status_fail(lc.status, sidx, 1, v0 + lane, KIND_SCORE_NONFINITE);
 }
 
-// The same scores for profiles with at most 16 angle bins (pbits <= 4), with
-// the per-pair term looked up instead of recomputed: for a chunk of up to
-// four queries the block first tabulates, in LDS,
-//   T[q][i][b] = qa_i * cos(theta_b) + qb_i * sin(theta_b)
+// The same scores for profiles with 3- or 4-bit angles, with the per-pair term
+// looked up instead of recomputed: for a group of G = 4 queries (2 or 1 for
+// the rest) the block first tabulates, in LDS,
+//   T[i][b][g] = qa_i * cos(theta_b) + qb_i * sin(theta_b) of query g
 // -- the parenthesised sum of polar.rs:361, the same two products and add --
-// so each (code, query, pair) costs one LDS read, a multiply by r_i and the
-// sequential add: est = est + r_i * T[q][i][bin_i], bit for bit the
-// reference's expression.  Payloads are staged through LDS 32 lanes at a
-// time (raw words into registers), and the staging space is then reused for
-// the table, which keeps four workgroups per CU at head_dim 128.
+// so each (code, pair) costs one table address and one G-wide LDS read for
+// the whole group and each (code, query, pair) a multiply by r_i and the
+// sequential add: est = est + r_i * T[i][bin_i][g], bit for bit the
+// reference's expression, G independent chains at a time.  The angle bins stay
+// packed as the payload has them; a table address is a shift and a mask.
+//
+// What bounds it is VALU issue: per 64-code wave at head_dim 128 about 64 x
+// (2 + 2G) operations per group, 32 G for the sketch fold, and with
+// BlockLogU8 radii 64 exponentials (radii_u8), about 2,100 operations for one
+// group of four.  2.1 M head_dim-128 codes x 4 queries, prepare included:
+// BlockLogU8 271 -> 120 us (243 MB, 2.0 TB/s), f32 radii 237 -> 157 us
+// (3.9 TB/s, near what a copy reaches); the one-query table with a separate
+// shift, mask and read per query was the start of both.
 template <int DIM, int PROJ, bool LOSSY, int PB>
-__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(DIM == 128 && PROJ ? 3 : 4))) void
-turbo_score_lut_kernel(
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void turbo_score_lut_kernel(
     LaunchCommon lc, const uint8_t* __restrict__ wire, const float* __restrict__ prepared, uint32_t nq,
     uint64_t qstride, float* __restrict__ scores, uint64_t ld, const float* __restrict__ cs_tab, uint64_t seed,
     uint32_t hproj, float qscale, float post) {
-    constexpr uint32_t pbits = PB;
     constexpr int PAIRS = DIM / 2;
-    constexpr int LUTQ = PAIRS * 16;             // floats per query: [pair][bin]
+    constexpr int LV = 1 << PB;                         // angle bins
     constexpr int W = DIM + PROJ;
     constexpr int RW = LOSSY ? PAIRS / 4 + 2 : PAIRS;   // radii words
-    constexpr int AWMAX = (PAIRS * PB + 31) / 32;       // angle words
+    constexpr int AW = (PAIRS * PB + 31) / 32;          // angle words
     constexpr int SW = PROJ / 32;                       // sign words
-    extern __shared__ uint32_t smem_u[];
-    __shared__ float2 cs_lds[16];
+    constexpr int PWD = RW + AW + SW;                   // payload words
+    constexpr int LANES = LOSSY ? 64 : 32;              // payloads staged per round (four workgroups fit a CU)
+    constexpr int STAGE = WAVES * (LANES * PWD + 4), TABLE = PAIRS * LV * 4;
+    // staged payloads, then the table (a fixed array: its address folds into
+    // the lookups' offsets)
+    __shared__ __align__(16) uint32_t smem_u[STAGE > TABLE ? STAGE : TABLE];
     __shared__ uint64_t exp_lds[32];
-
-    constexpr uint32_t levels = 1u << pbits;
-    if (threadIdx.x < 16)
-        cs_lds[threadIdx.x] = threadIdx.x < levels ? make_float2(cs_tab[2 * threadIdx.x], cs_tab[2 * threadIdx.x + 1])
-                                                   : make_float2(0.0f, 0.0f);
     if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
-    if (LOSSY)
-        __syncthreads();   // the tables are read by every wave (radii below, the (cos, sin) terms later)
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t blk = blockIdx.x;
-    const uint32_t sidx = segment_of(lc.tile_seg, lc.tile_start, lc.nseg, blk);
+    const uint32_t sidx =
+        __builtin_amdgcn_readfirstlane(segment_of(lc.tile_seg, lc.tile_start, lc.nseg, blk));   // block-uniform
     const SegDev seg = lc.segs[sidx];
     const uint32_t tile = blk - lc.tile_start[sidx];
-    const uint32_t plen = lc.plen, pwd = plen >> 2;
+    const uint32_t plen = lc.plen;   // 4 * PWD
     const uint8_t* blob = wire + seg.wire_offset;
     const uint32_t hb = lane < 38 ? blob[lane] : 0u;   // checked once the payloads are staged
     const uint32_t v0 = tile * TILE + static_cast<uint32_t>(wave) * WAVE;
     const uint32_t nv = v0 < seg.n_vectors ? min(static_cast<uint32_t>(WAVE), seg.n_vectors - v0) : 0u;
     const bool active = static_cast<uint32_t>(lane) < nv;
+    const float* pseg = prepared + static_cast<uint64_t>(sidx) * qstride * W;
 
-    // raw payload words, 32 lanes per round through this wave's staging area
-    uint32_t rw[RW], aw[AWMAX], sgw[SW ? SW : 1];
+    // Table entries of this thread: bin threadIdx % LV of pairs i0 + k * TILE / LV
+    constexpr int PER = PAIRS * LV / TILE;
+    static_assert(PAIRS * LV % TILE == 0 && TILE % LV == 0, "table fill");
+    const uint32_t i0 = threadIdx.x / LV;
+    const float tc = cs_tab[2 * (threadIdx.x % LV)], ts = cs_tab[2 * (threadIdx.x % LV) + 1];
+
+    // raw payload words, LANES lanes per round through this wave's staging area
+    uint32_t rw[RW], aw[AW], sgw[SW ? SW : 1];
     {
-        uint32_t* sw = smem_u + wave * (32 * pwd + 4);
-        constexpr uint32_t nwa = AWMAX;
+        uint32_t* sw = smem_u + wave * (LANES * PWD + 4);
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const uint32_t h0 = 32u * half;
-            const uint32_t hn = nv > h0 ? min(32u, nv - h0) : 0u;
-            if (hn) global_to_lds<16>(sw, blob + 38 + static_cast<uint64_t>(v0 + h0) * plen, hn * plen, lane);
+        for (int half = 0; half < WAVE / LANES; ++half) {
+            const uint32_t h0 = static_cast<uint32_t>(LANES * half);
+            const uint32_t hn = nv > h0 ? min(static_cast<uint32_t>(LANES), nv - h0) : 0u;
+            if (hn)
+                global_to_lds16<(LANES * PWD * 4 + 1023) / 1024, false>(
+                    sw, blob + 38 + static_cast<uint64_t>(v0 + h0) * plen, hn * plen, lane);
             wave_sync();
-            if ((lane >> 5) == half) {
-                const uint32_t* pw = sw + min(static_cast<uint32_t>(lane & 31), hn ? hn - 1 : 0u) * pwd;
+            if (lane / LANES == half) {
+                const uint32_t* pw = sw + min(static_cast<uint32_t>(lane % LANES), hn ? hn - 1 : 0u) * PWD;
 #pragma unroll
                 for (int k = 0; k < RW; ++k) rw[k] = pw[k];
 #pragma unroll
-                for (int k = 0; k < AWMAX; ++k) aw[k] = pw[RW + k];
+                for (int k = 0; k < AW; ++k) aw[k] = pw[RW + k];
 #pragma unroll
-                for (int k = 0; k < SW; ++k) sgw[k] = pw[RW + nwa + k];
+                for (int k = 0; k < SW; ++k) sgw[k] = pw[RW + AW + k];
             }
             wave_sync();
         }
     }
     const bool hbad = lane < 38 && tqb1_checked(lane) &&
-                      hb != tqb1_byte(lane, DIM, pbits, lc.radii, hproj, seed, seg.n_vectors, plen);
+                      hb != tqb1_byte(lane, DIM, PB, lc.radii, hproj, seed, seg.n_vectors, plen);
     if (__ballot(hbad) != 0ull) {   // the same header for every wave of the block: all leave
         if (lane == 0 && wave == 0) status_fail(lc.status, sidx, 0, 0u, KIND_HEADER);
         return;
     }
+    __syncthreads();   // exp_lds
     // radii with the decoder's checks (radius.rs:88-104, 128-145, 171-177; polar.rs:127-133)
     float r[PAIRS];
     bool ok = true;
     if constexpr (!LOSSY) {
+        // finite and non-negative: bits below +inf's, or -0
+        uint32_t top = 0;
 #pragma unroll
         for (int i = 0; i < PAIRS; ++i) {
             r[i] = u2f(rw[i]);
-            ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);
+            top = max(top, rw[i]);
         }
+        if (top >= 0x7f800000u)
+#pragma unroll
+            for (int i = 0; i < PAIRS; ++i) ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);
     } else {
-        const float mn = u2f(rw[PAIRS / 4]), mx = u2f(rw[PAIRS / 4 + 1]);
-        ok &= isfinite_f(mn) && isfinite_f(mx) && !(mn > mx);
-        const float span = mx - mn;
+        uint32_t q[PAIRS / 4];
 #pragma unroll
-        for (int i = 0; i < PAIRS; ++i) {
-            const uint32_t u = (rw[i >> 2] >> (8 * (i & 3))) & 0xffu;
-            r[i] = og_expf(mn + span * div255_f(static_cast<float>(u)), exp_lds);
-            ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);
-        }
+        for (int k = 0; k < PAIRS / 4; ++k) q[k] = rw[k];
+        radii_u8<PAIRS>(q, u2f(rw[PAIRS / 4]), u2f(rw[PAIRS / 4 + 1]), exp_lds, r, ok);
     }
-    // byte offsets bin * 4 of every pair, four per word
-    uint32_t boff[PAIRS / 4];
+    // sketch signs, one word per 32: the complements of the even bits in the
+    // low half, of the odd bits in the high half, so that one shift and one
+    // mask give the pair (2k, 2k + 1) as f16 +-1.0 halves
+    uint32_t sgp[SW ? SW : 1];
 #pragma unroll
-    for (int i = 0; i < PAIRS / 4; ++i) boff[i] = 0u;
-#pragma unroll
-    for (int i = 0; i < PAIRS; ++i) {
-        constexpr uint32_t M = levels - 1u;
-        const int bit = i * PB, wd = bit >> 5, sh = bit & 31;
-        uint32_t b = aw[wd] >> sh;
-        if (sh + PB > 32) b |= aw[wd + 1] << (32 - sh);
-        boff[i >> 2] |= ((b & M) * 4u) << (8 * (i & 3));
-    }
-    // sketch signs as f16 +-1.0, two per register, folded in by a mixed FMA
-    // whose product (+-1 times p) is exact: e2 + s_j * p_j rounds once, as the
-    // reference's add of sign as f32 * p (qjl.rs:316-321)
-    uint32_t sgh[PROJ ? PROJ / 2 : 1];
-#pragma unroll
-    for (int j2 = 0; j2 < PROJ / 2; ++j2) {
-        const uint32_t w = sgw[(2 * j2) >> 5] >> ((2 * j2) & 31);
-        sgh[j2] = ((w & 1u) ? 0x3c00u : 0xbc00u) | (((w & 2u) ? 0x3c00u : 0xbc00u) << 16);
+    for (int k = 0; k < SW; ++k) {
+        uint32_t x = ~sgw[k];
+        x = (x & 0x99999999u) | ((x >> 1) & 0x22222222u) | ((x & 0x22222222u) << 1);   // gather even and odd bits
+        x = (x & 0xc3c3c3c3u) | ((x >> 2) & 0x0c0c0c0cu) | ((x & 0x0c0c0c0cu) << 2);
+        x = (x & 0xf00ff00fu) | ((x >> 4) & 0x00f000f0u) | ((x & 0x00f000f0u) << 4);
+        x = (x & 0xff0000ffu) | ((x >> 8) & 0x0000ff00u) | ((x & 0x0000ff00u) << 8);
+        sgp[k] = x;
     }
     if (active && !ok) status_fail(lc.status, sidx, 0, v0 + lane, KIND_CORRUPT);
     const uint64_t col = vec_elem_offset(seg, v0 + min(static_cast<uint32_t>(lane), nv ? nv - 1 : 0u));
     const bool store = active && ok;
-    const float* pseg = prepared + static_cast<uint64_t>(sidx) * qstride * W;
-    float* lut = reinterpret_cast<float*>(smem_u);
-    constexpr int PER = LUTQ / TILE;   // table entries per thread and query
-    static_assert(LUTQ % TILE == 0, "table fill");
-    float qa[PER], qb[PER];           // the next query's rotated pairs this thread tabulates
-    auto fetch = [&](uint32_t q) {
-        const float* pq = pseg + static_cast<uint64_t>(q) * W;
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const uint32_t i = (threadIdx.x + k * TILE) / 16;
-            qa[k] = pq[2 * i];
-            qb[k] = pq[2 * i + 1];
-        }
-    };
-    if (nq) fetch(0);
     bool fin = true;
-    for (uint32_t q = 0; q < nq; ++q) {
-        __syncthreads();   // staging / the previous query's table is no longer read
+
+    // scores of queries q0 .. q0 + G - 1
+    auto group = [&](auto gc, uint32_t q0) __attribute__((always_inline)) {
+        constexpr int G = decltype(gc)::value;
+        constexpr int LOGB = G == 4 ? 4 : G == 2 ? 3 : 2;   // log2 of a table entry's bytes
+        typedef float vg __attribute__((ext_vector_type(G)));
+        const float* pq = pseg + static_cast<uint64_t>(q0) * W;
+        float* lut = reinterpret_cast<float*>(smem_u);
+        float qa[PER][G], qb[PER][G];
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const float* src = pq + g * W + 2 * (i0 + k * (TILE / LV));
+                qa[k][g] = src[0];
+                qb[k][g] = src[1];
+            }
+        __syncthreads();   // staging / the previous group's table is no longer read
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const uint32_t e = threadIdx.x + k * TILE;
-            const float2 c = cs_lds[e % 16];
-            lut[e] = qa[k] * c.x + qb[k] * c.y;
+            vg e;
+#pragma unroll
+            for (int g = 0; g < G; ++g) e[g] = qa[k][g] * tc + qb[k][g] * ts;
+            reinterpret_cast<vg*>(lut)[threadIdx.x + k * TILE] = e;
         }
         __syncthreads();
-        if (q + 1 < nq) fetch(q + 1);   // in flight while this query is scored
-        // keep the per-pair offsets and the signs packed: unpacked per query, not hoisted
-        // out of the loop into one register each
+        // keep the angle bins and the signs packed: unpacked per group, not
+        // hoisted out of the query loop into one register each
 #pragma unroll
-        for (int k = 0; k < PAIRS / 4; ++k) asm volatile("" : "+v"(boff[k]));
+        for (int k = 0; k < AW; ++k) asm volatile("" : "+v"(aw[k]));
 #pragma unroll
-        for (int k = 0; k < (PROJ ? PROJ / 2 : 1); ++k) asm volatile("" : "+v"(sgh[k]));
+        for (int k = 0; k < SW; ++k) asm volatile("" : "+v"(sgp[k]));
         const char* lb = reinterpret_cast<const char*>(lut);
-        auto tab = [&](int i) {
-            const uint32_t off = (boff[i >> 2] >> (8 * (i & 3))) & 0xffu;
-            return *reinterpret_cast<const float*>(lb + off + 4 * (i * 16));
+        auto tab = [&](int i) -> vg {
+            const int bit = i * PB, wd = bit >> 5, sh = bit & 31;
+            uint32_t off;   // bin i << LOGB
+            if (sh + PB > 32) off = (__builtin_amdgcn_alignbit(aw[wd + 1 < AW ? wd + 1 : wd], aw[wd], sh) << LOGB);
+            else if (sh >= LOGB) off = aw[wd] >> (sh - LOGB);
+            else off = aw[wd] << (LOGB - sh);
+            off &= static_cast<uint32_t>(LV - 1) << LOGB;
+            return *reinterpret_cast<const vg*>(lb + off + (i * LV << LOGB));
         };
-        constexpr int DEPTH = 4;   // table reads in flight ahead of the sequential sum
-        float ring[DEPTH];
+        constexpr int STEP = 2;   // pairs per scheduling step: their table reads are a step ahead of the sums
+        vg cur[STEP], nxt[STEP];
 #pragma unroll
-        for (int k = 0; k < DEPTH; ++k) ring[k] = tab(k);
-        float est = 0.0f;
+        for (int k = 0; k < STEP; ++k) nxt[k] = tab(k);
+        float est[G];
 #pragma unroll
-        for (int i = 0; i < PAIRS; ++i) {
-            const float t = ring[i % DEPTH];
-            if (i + DEPTH < PAIRS) ring[i % DEPTH] = tab(i + DEPTH);
-            est = est + r[i] * t;
-        }
-        bool f = isfinite_f(est);
-        float total = est;
-        if constexpr (PROJ != 0) {
-            const float* pq = pseg + static_cast<uint64_t>(q) * W;
-            float e2 = -0.0f;
+        for (int g = 0; g < G; ++g) est[g] = 0.0f;
 #pragma unroll
-            for (int j = 0; j < PROJ; ++j) {
-                const _Float16 h = __builtin_bit_cast(_Float16, static_cast<uint16_t>(sgh[j >> 1] >> (16 * (j & 1))));
-                e2 = __builtin_fmaf(static_cast<float>(h), pq[DIM + j], e2);
+        for (int i = 0; i < PAIRS; i += STEP) {
+#pragma unroll
+            for (int k = 0; k < STEP; ++k) {
+                cur[k] = nxt[k];
+                if (i + STEP < PAIRS) nxt[k] = tab(i + STEP + k);
             }
-            const float qj = qscale * e2;
-            f &= isfinite_f(qj);
-            total = est + qj;
+            __builtin_amdgcn_sched_barrier(0);   // no reads further ahead: they would spill the radii
+#pragma unroll
+            for (int k = 0; k < STEP; ++k)
+#pragma unroll
+                for (int g = 0; g < G; ++g) est[g] = est[g] + r[i + k] * cur[k][g];
+#pragma unroll
+            for (int g = 0; g < G; ++g) asm volatile("" : "+v"(est[g]));   // every chain advances here, none is sunk
+            __builtin_amdgcn_sched_barrier(0);
         }
-        f &= isfinite_f(total);
-        fin &= f;
-        if (store) scores[static_cast<uint64_t>(q) * ld + col] = total * post;
+        float e2[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) e2[g] = -0.0f;
+        if constexpr (PROJ != 0) {
+#pragma unroll
+            for (int j = 0; j < PROJ; j += 2) {
+                // (s_j, s_j+1) folded in by mixed FMAs whose products (+-1 times
+                // p) are exact: e2 + s_j * p_j rounds once, as the reference's
+                // add of sign as f32 * p (qjl.rs:316-321)
+                const int k = (j >> 1) & 15;
+                const uint32_t h = ((sgp[j >> 5] << (15 - k)) & 0x80008000u) ^ 0x3c003c00u;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const _Float16 sj = __builtin_bit_cast(_Float16, static_cast<uint16_t>(h >> (16 * t)));
+#pragma unroll
+                    for (int g = 0; g < G; ++g)
+                        e2[g] = __builtin_fmaf(static_cast<float>(sj), pq[g * W + DIM + j + t], e2[g]);
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            bool f = isfinite_f(est[g]);
+            float total = est[g];
+            if constexpr (PROJ != 0) {
+                const float qj = qscale * e2[g];
+                f &= isfinite_f(qj);
+                total = est[g] + qj;
+            }
+            f &= isfinite_f(total);
+            fin &= f;
+            if (store) scores[static_cast<uint64_t>(q0 + g) * ld + col] = total * post;
+        }
+    };
+    uint32_t q = 0;
+#pragma unroll 1
+    for (; q + 4 <= nq; q += 4) group(std::integral_constant<int, 4>{}, q);
+    if (nq - q >= 2) {
+        group(std::integral_constant<int, 2>{}, q);
+        q += 2;
     }
+    if (q < nq) group(std::integral_constant<int, 1>{}, q);
     if (store && !fin) status_fail(lc.status, sidx, 1, v0 + lane, KIND_SCORE_NONFINITE);
 }
 
@@ -3784,11 +3852,12 @@ int launch_turbo_prepare(const TurboDev& td, const float* q, uint32_t nq, float*
                          uint32_t* status, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (nq == 0) return hipSuccess;
+    const dim3 threads(td.mode ? 2 * WAVE : WAVE);   // the second wave projects onto G
     if (td.dim == 64)
-        hipLaunchKernelGGL(turbo_prepare_kernel<64>, dim3(nq), dim3(WAVE), 0, st, q, nq, out, td.signs, td.qjl,
+        hipLaunchKernelGGL(turbo_prepare_kernel<64>, dim3(nq), threads, 0, st, q, nq, out, td.signs, td.qjl,
                            td.proj, td.mode, rscale, status);
     else if (td.dim == 128)
-        hipLaunchKernelGGL(turbo_prepare_kernel<128>, dim3(nq), dim3(WAVE), 0, st, q, nq, out, td.signs, td.qjl,
+        hipLaunchKernelGGL(turbo_prepare_kernel<128>, dim3(nq), threads, 0, st, q, nq, out, td.signs, td.qjl,
                            td.proj, td.mode, rscale, status);
     else
         return hipErrorInvalidValue;
@@ -3809,14 +3878,11 @@ int launch_turbo_score(const LaunchCommon& lc, const TurboDev& td, const uint8_t
     (lc.radii == PKV_RADII_F32 ? (narrow ? PKV_SCORE(D, P, false, true) : PKV_SCORE(D, P, false, false))        \
                                : (narrow ? PKV_SCORE(D, P, true, true) : PKV_SCORE(D, P, true, false)))
     if ((td.pbits == 3 || td.pbits == 4) && proj <= 32) {   // table path: [pair][bin] terms in LDS
-        const size_t stage = static_cast<size_t>(WAVES) * (32 * (lc.plen >> 2) + 4) * sizeof(uint32_t);
-        const size_t table = static_cast<size_t>(td.dim / 2) * 16 * sizeof(float);
-        const size_t llds = std::max(stage, table);
 #define PKV_LUT(D, P, PB)                                                                                      \
     (lc.radii == PKV_RADII_F32                                                                                 \
-         ? launch_big_lds(turbo_score_lut_kernel<D, P, false, PB>, nblocks, llds, st, lc, wire, prepared, nq,   \
+         ? launch_big_lds(turbo_score_lut_kernel<D, P, false, PB>, nblocks, 0, st, lc, wire, prepared, nq,   \
                           qstride, scores, ld, td.cs, td.seed, td.proj, qscale, post)                           \
-         : launch_big_lds(turbo_score_lut_kernel<D, P, true, PB>, nblocks, llds, st, lc, wire, prepared, nq,    \
+         : launch_big_lds(turbo_score_lut_kernel<D, P, true, PB>, nblocks, 0, st, lc, wire, prepared, nq,    \
                           qstride, scores, ld, td.cs, td.seed, td.proj, qscale, post))
         if (td.dim == 64)
             return td.pbits == 3 ? (proj ? PKV_LUT(64, 32, 3) : PKV_LUT(64, 0, 3))

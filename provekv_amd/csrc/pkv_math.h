@@ -345,7 +345,7 @@ PKV_HD float og_expf(float x, const uint64_t* tab) {
     return (float)y;
 }
 
-// og_expf for |x| <= 32.5 with the multiply-adds fused (8 f64 operations
+// og_expf for |x| <= 32.5 with the multiply-adds fused (7 f64 operations
 // instead of 13, no range checks): the same f32 for every such x -- the two
 // finite floats on which the forms differ are 0x1.04845ep+5 and
 // -0x1.f8cbb2p+5 (every float below 88 in magnitude was compared).
@@ -363,10 +363,8 @@ PKV_HD float og_expf_fused(float x, const uint64_t* tab) {
     const uint64_t e = tab[ki % 32];
     // + (ki << 47): only the high word changes
     const double s = u2d((uint64_t)((uint32_t)(e >> 32) + (ki << 15)) << 32 | (uint32_t)e);
-    const double zz = __builtin_fma(C0, r, C1);
-    double y = __builtin_fma(C2, r, 1.0);
-    y = __builtin_fma(zz, r * r, y);
-    return (float)(y * s);
+    const double q = __builtin_fma(__builtin_fma(C0, r, C1), r, C2);
+    return (float)(__builtin_fma(q, r, 1.0) * s);
 }
 
 // fl(u / 255) for u = 0 .. 255 (exact integers): 1/255 as two floats, the low
