@@ -127,6 +127,7 @@ struct pkv_profile {
     double* d_rot64 = nullptr;   // row-major f64 rotation (encode's exact redo)
     float* d_rot32t = nullptr;
     float* d_rot32 = nullptr;
+    float* d_prefix = nullptr;   // decode partial sums (matrix-core decode only)
     int mfma_decode = 0;
     uint32_t* d_mf = nullptr;
     float thr = 0.0f;
@@ -450,6 +451,7 @@ FibDev fib_dev(const pkv_profile* p) {
     f.rot64 = p->d_rot64;
     f.rot32t = p->d_rot32t;
     f.rot32 = p->d_rot32;
+    f.prefix = p->d_prefix;
     f.mfma_decode = p->mfma_decode;
     f.mf = p->d_mf;
     f.thr = p->thr;
@@ -1006,6 +1008,16 @@ static int fib_verify_mfma_products(pkv_ctx* ctx, pkv_profile* p) {
     return PKV_OK;
 }
 
+// The matrix-core decode's table of partial sums (ready when this returns).
+static int fib_build_prefix(pkv_ctx* ctx, pkv_profile* p) {
+    if (!p->mfma_decode) return PKV_OK;
+    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&p->d_prefix),
+                      (sizeof(float) * p->dim) << (5 * FIB_PREFIX_BLOCKS)));
+    const hipError_t e = static_cast<hipError_t>(launch_fib_prefix(p->d_rot32, p->d_cb, p->d_prefix, ctx->own_stream));
+    const hipError_t se = hipStreamSynchronize(ctx->own_stream);
+    return hip_status(e == hipSuccess ? se : e);
+}
+
 static int fib_profile_common(pkv_ctx* ctx, uint32_t dim, uint32_t k, uint32_t n, std::vector<float> cb,
                               std::vector<double> rot, pkv_profile** out) {
     pkv_profile* p = new (std::nothrow) pkv_profile();
@@ -1039,6 +1051,7 @@ static int fib_profile_common(pkv_ctx* ctx, uint32_t dim, uint32_t k, uint32_t n
     if (!rc) rc = upload(&p->d_mf, p->mf);
     if (!rc) rc = upload(&p->d_rot32, p->rot32);
     if (!rc) rc = fib_verify_mfma_products(ctx, p);
+    if (!rc) rc = fib_build_prefix(ctx, p);
     if (rc) { pkv_profile_destroy(p); return rc; }
     *out = p;
     return PKV_OK;
@@ -1187,7 +1200,8 @@ void pkv_profile_destroy(pkv_profile* p) {
                     static_cast<void*>(p->d_qa), static_cast<void*>(p->d_qb),
                     static_cast<void*>(p->d_cb), static_cast<void*>(p->d_rot_t), static_cast<void*>(p->d_rot64),
                     static_cast<void*>(p->d_rot32t),
-                    static_cast<void*>(p->d_mf), static_cast<void*>(p->d_rot32), static_cast<void*>(p->d_cb64)})
+                    static_cast<void*>(p->d_mf), static_cast<void*>(p->d_rot32), static_cast<void*>(p->d_cb64),
+                    static_cast<void*>(p->d_prefix)})
         if (d) (void)hipFree(d);
     delete p;
 }

@@ -72,6 +72,11 @@ constexpr uint32_t fib_mfma_row(uint32_t t, uint32_t m) {
     return 4 * (8 * t + (4 * (m >> 3) + (m & 3)) / 2) + 2 * ((4 * (m >> 3) + (m & 3)) % 2) + ((m >> 2) & 1);
 }
 
+// Leading blocks of a vector whose decode sums come from a table of every index
+// combination: 3 blocks = 32,768 rows of 256 bytes, 8 MB a profile (2 would
+// save two thirds as many rows of the sum; 4 would take 256 MB).
+constexpr int FIB_PREFIX_BLOCKS = 3;
+
 struct FibDev {
     const float* codebook;  // n * k
     const double* codebook64;  // n * k, the same values widened (per-vector f64 decode)
@@ -79,6 +84,7 @@ struct FibDev {
     const double* rot64;    // dim * dim, row-major (the encode's exact redo)
     const float* rot32t;    // dim * dim, f32(rot) transposed: [col][row] (VALU decode)
     const float* rot32;     // dim * dim, f32(rot) row-major (MFMA decode)
+    const float* prefix;    // 32^FIB_PREFIX_BLOCKS * dim partial sums (MFMA decode)
     int mfma_decode;        // matrix-core products verified bit-exact for this profile
     const uint32_t* mf;     // MF_WORDS (encode MFMA operands)
     float thr;              // argmin acceptance margin for the approximate keys
@@ -178,6 +184,7 @@ int launch_logf_bound(void* stream);
 int launch_f16_subnormal_probe(float* out, void* stream);
 int launch_logf_bound_read(float* out, void* stream);
 int launch_sqrt_check(uint32_t* bad, void* stream);
+int launch_fib_prefix(const float* rot32, const float* cb, float* out, void* stream);
 int launch_fib_product_check(const float* rot32, const float* cb, uint32_t* bad, void* stream);
 
 // Legacy per-vector records (pkv_records.hip).  Records are rec_hdr header

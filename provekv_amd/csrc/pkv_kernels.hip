@@ -3437,13 +3437,27 @@ __global__ __launch_bounds__(TILE) void fib_decode_kernel(LaunchCommon lc, const
 // fib_product_check_kernel checks every product this kernel can form
 // (64 rows x 64 columns x 32 codewords) when a profile is created, and the
 // profile falls back to fib_decode_kernel on any difference.
+//
+// What bounds one copy is that arithmetic: per 32 vectors and row 32 adds of 4
+// cycles and 64 matrix-core cycles, which do not overlap on f32 operands.  The
+// sum after the first FIB_PREFIX_BLOCKS blocks depends only on their indices,
+// so it is read from a table built with the profile (fib_prefix_kernel: the
+// same products and sums, 32,768 rows of 256 bytes, 8 MB, mostly L2 and
+// Infinity Cache) instead of being formed: 12 of the 64 rows less (1.23 M
+// vectors to f32: 190 -> 164 us, 1.7 -> 2.0 TB/s; PREFIX at launch_fib_decode).
+//
+// A wave takes 32 vectors, a workgroup a half-tile of 128, so a small launch
+// spreads over twice the waves it did with 64 per wave and its latency is one
+// sub-tile's (48 blobs of 185 vectors: 20.6 -> 13.1 us a call, 150 k vectors
+// 38 -> 28 us).
 typedef float v32f __attribute__((ext_vector_type(32)));
 
-template <int DIM, bool STAGED>
+template <int DIM, bool STAGED, bool PREFIX>
 __global__ __launch_bounds__(TILE) void fib_decode_mfma_kernel(LaunchCommon lc, const uint8_t* __restrict__ wire,
                                                                void* __restrict__ out,
                                                                const float* __restrict__ rot32,
                                                                const float* __restrict__ cb,
+                                                               const float* __restrict__ prefix,
                                                                const SegDev* __restrict__ segs,
                                                                const uint32_t* __restrict__ tile_start,
                                                                const uint32_t* __restrict__ tile_seg) {
@@ -3452,97 +3466,110 @@ __global__ __launch_bounds__(TILE) void fib_decode_mfma_kernel(LaunchCommon lc, 
     static_assert(DIM == 64, "two 32-column MFMA blocks");
     constexpr int BLOCKS = DIM / 4;
     constexpr uint32_t PLEN = 2 + (BLOCKS * 5 + 7) / 8;   // 12
-    constexpr int PAY_WORDS = WAVE * PLEN / 4 + 4;
-    constexpr int RPITCH = DIM + 4;      // one staged row per vector, padded
-    __shared__ float rot_s[DIM * DIM];   // f32(Pi), row-major
+    constexpr int RPITCH = DIM + 4;                       // one staged row per vector, padded
+    constexpr int PRE = PREFIX ? FIB_PREFIX_BLOCKS : 0;   // blocks summed in the table
+    constexpr int ROW0 = 4 * PRE;                         // first row summed here
+    constexpr uint32_t ROT4 = (DIM - ROW0) * DIM / 4;
+    __shared__ __align__(16) float rot_s[(DIM - ROW0) * DIM];   // f32(Pi) from row ROW0, row-major
     __shared__ float4 cb_s[32];
-    __shared__ uint32_t pay_s[WAVES][PAY_WORDS];
-    __shared__ float half_s[STAGED ? WAVES : 1][STAGED ? 16 * RPITCH : 4];   // output staging: 16 rows
+    __shared__ __align__(16) float half_s[STAGED ? WAVES : 1][STAGED ? 16 * RPITCH : 4];   // output staging: 16 rows
     {
-        const float4* src = reinterpret_cast<const float4*>(rot32);
+        const float4* src = reinterpret_cast<const float4*>(rot32 + ROW0 * DIM);
         float4* dst = reinterpret_cast<float4*>(rot_s);
-        float4 t[DIM * DIM / 4 / TILE];
+        constexpr int N = (ROT4 + TILE - 1) / TILE;
+        float4 t[N];
 #pragma unroll
-        for (int k = 0; k < DIM * DIM / 4 / TILE; ++k) t[k] = src[threadIdx.x + k * TILE];
+        for (int k = 0; k < N; ++k) t[k] = src[min(static_cast<uint32_t>(threadIdx.x + k * TILE), ROT4 - 1u)];
 #pragma unroll
-        for (int k = 0; k < DIM * DIM / 4 / TILE; ++k) dst[threadIdx.x + k * TILE] = t[k];
+        for (int k = 0; k < N; ++k) dst[min(static_cast<uint32_t>(threadIdx.x + k * TILE), ROT4 - 1u)] = t[k];
         if (threadIdx.x < 32) cb_s[threadIdx.x] = reinterpret_cast<const float4*>(cb)[threadIdx.x];
     }
     __syncthreads();
 
-    const int wave = threadIdx.x >> 6;
-    // one tile per workgroup, or (grid capped) a workgroup walks the tiles
-    // blockIdx.x, blockIdx.x + gridDim.x, ... with the tables loaded once
-    const uint32_t nblk = tile_start[lc.nseg];
-    for (uint32_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-    wave_sync();   // the previous tile's LDS reads are done
-    // opaque per tile: the loop must not keep lane-derived addresses or table
-    // reads live across tiles (register pressure)
-    int zoff = 0, lane = threadIdx.x & 63;
-    asm volatile("" : "+s"(zoff), "+v"(lane));
-    const int h = lane >> 5, n = lane & 31;
-    const uint32_t sidx = segment_of(tile_seg, tile_start, lc.nseg, blk);
-    const SegDev seg = segs[sidx];
-    const uint32_t tile = blk - tile_start[sidx];
-    const uint32_t v0 = tile * TILE + wave * WAVE;
-    const uint8_t* blob = wire + seg.wire_offset;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t nhalf = 2u * tile_start[lc.nseg];
+    for (uint32_t hb = blockIdx.x; hb < nhalf; hb += gridDim.x) {
+        // opaque per half-tile: the loop must not keep lane-derived addresses or
+        // table reads live across half-tiles (register pressure)
+        int zoff = 0, lane = threadIdx.x & 63;
+        asm volatile("" : "+s"(zoff), "+v"(lane));
+        const int h = lane >> 5, n = lane & 31;
+        const uint32_t sidx = segment_of(tile_seg, tile_start, lc.nseg, hb >> 1);
+        const SegDev seg = segs[sidx];
+        const uint8_t* blob = wire + seg.wire_offset;
+        // Lane n's vector: two runs of 16, 32 apart -- when a blob holds 32 heads
+        // (vector = token * H + head) the same 16 heads at consecutive tokens,
+        // so the staged stores below write two adjacent rows per run.  Any
+        // other layout is just another order.
+        const uint32_t r0 = ((hb >> 1) - tile_start[sidx]) * TILE + (hb & 1u) * (TILE / 2) + 64u * (wave >> 1) +
+                            16u * (wave & 1u);
+        const uint32_t vi = r0 + (static_cast<uint32_t>(n) & 15u) + 32u * (static_cast<uint32_t>(n) >> 4);
+        const bool some = r0 < seg.n_vectors;   // wave-uniform
+        const bool active = vi < seg.n_vectors;
+        // header bytes and this lane's payload (lanes past the end: the last vector's)
+        const uint32_t hb0 = lane < 19 ? blob[lane] : 0u;
+        uint32_t q[3] = {0u, 0u, 0u};
+        if (some)
+            __builtin_memcpy(q, blob + 19 + static_cast<uint64_t>(min(vi, seg.n_vectors - 1u)) * PLEN, PLEN);
+        bool bad = lane < 19 && fb2_checked(lane, seg.n_vectors) &&
+                   hb0 != fb2_byte(lane, 5u, BLOCKS, seg.n_vectors, PLEN - 2);
+        if (lane == 14 && hb0 != 0u) bad = true;   // norm format must be Fp16Paper
+        if (__ballot(bad) != 0ull) {
+            if (lane == 0) status_fail(lc.status, sidx, 0, 0u, KIND_HEADER);
+            continue;
+        }
+        if (!some) continue;
 
-    uint32_t hb = lane < 19 ? blob[lane] : 0u;
-    bool bad = lane < 19 && fb2_checked(lane, seg.n_vectors) &&
-               hb != fb2_byte(lane, 5u, BLOCKS, seg.n_vectors, PLEN - 2);
-    if (lane == 14 && hb != 0u) bad = true;   // norm format must be Fp16Paper
-    if (__ballot(bad) != 0ull) {
-        if (lane == 0) status_fail(lc.status, sidx, 0, 0u, KIND_HEADER);
-        continue;
-    }
-    if (v0 >= seg.n_vectors) continue;
-    const uint32_t nv = min(static_cast<uint32_t>(WAVE), seg.n_vectors - v0);
-    uint32_t* sw = pay_s[wave];
-    global_to_lds(sw, blob + 19 + static_cast<uint64_t>(v0) * PLEN, nv * PLEN, lane);
-    wave_sync();
-
-    // Sub-tile s, lane n: wave vector w = (n % 16) + 16 s + 32 (n / 16) -- vectors
-    // w and w + 32 are the same head at consecutive tokens when a blob holds
-    // 32 heads (vector = token * H + head), so the staged stores below write
-    // two adjacent rows per run.  Any other layout is just another order.
-    for (uint32_t sub = 0; sub < 2; ++sub) {
-        if (sub == 1 && nv <= 16) break;
-        const uint32_t w = (static_cast<uint32_t>(n) & 15u) + 16u * sub + 32u * (static_cast<uint32_t>(n) >> 4);
-        const uint32_t my = min(w, nv - 1);   // lanes past the end repeat the last
-        const uint32_t q0 = sw[3 * my], q1 = sw[3 * my + 1], q2 = sw[3 * my + 2];
-        const uint64_t lo = (static_cast<uint64_t>(q0) >> 16) | (static_cast<uint64_t>(q1) << 16) |
-                            (static_cast<uint64_t>(q2) << 48);
-        const uint32_t hi = q2 >> 16;
+        // the 16 x 5-bit indices, LSB-first from payload byte 2, as 80 bits
+        // shifted down by one index per block
+        uint32_t f0 = __builtin_amdgcn_alignbit(q[1], q[0], 16), f1 = __builtin_amdgcn_alignbit(q[2], q[1], 16),
+                 f2 = q[2] >> 16;
+        v32f acc = {};   // columns 32bb + 8g + 4h + i in register 16bb + 4g + i
+        if constexpr (PREFIX) {
+            const float* row = prefix + static_cast<size_t>(f0 & ((1u << (5 * PRE)) - 1u)) * DIM + 4 * h;
+#pragma unroll
+            for (int bb = 0; bb < 2; ++bb)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 v = *reinterpret_cast<const float4*>(row + 32 * bb + 8 * g);
+                    acc[16 * bb + 4 * g] = v.x;
+                    acc[16 * bb + 4 * g + 1] = v.y;
+                    acc[16 * bb + 4 * g + 2] = v.z;
+                    acc[16 * bb + 4 * g + 3] = v.w;
+                }
+        }
         const v32f zero = {};
-        v32f acc = {};
-#pragma unroll 2
-        for (int b = 0; b < BLOCKS; ++b) {
-            const int bit = 5 * b;
-            // 5-bit index b, LSB-first from payload byte 2 (bit may straddle the 64-bit word)
-            const uint32_t w = static_cast<uint32_t>(bit < 64 ? (lo >> bit) | (bit > 59 ? static_cast<uint64_t>(hi) << (64 - bit) : 0ull)
-                                                             : static_cast<uint64_t>(hi >> (bit - 64))) & 31u;
-            const float4 c = cb_s[w];
+        if constexpr (PREFIX) {
+            f0 = __builtin_amdgcn_alignbit(f1, f0, 5 * PRE);
+            f1 = __builtin_amdgcn_alignbit(f2, f1, 5 * PRE);
+            f2 >>= 5 * PRE;
+        }
+        const float* rp = rot_s + lane + zoff;
+#pragma unroll 1
+        for (int b = PRE; b < BLOCKS; ++b, rp += 4 * DIM) {
+            const float4 c = cb_s[f0 & 31u];
+            f0 = __builtin_amdgcn_alignbit(f1, f0, 5);
+            f1 = __builtin_amdgcn_alignbit(f2, f1, 5);
+            f2 >>= 5;
             const float cr[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(rot_s[(4 * b + t) * DIM + lane + zoff], cr[t], zero, 0, 0, 0);
+                const v32f p = __builtin_amdgcn_mfma_f32_32x32x1f32(rp[t * DIM], cr[t], zero, 0, 0, 0);
 #pragma unroll
-                for (int q = 0; q < 32; ++q) acc[q] = acc[q] + p[q];
+                for (int k = 0; k < 32; ++k) acc[k] = acc[k] + p[k];
             }
         }
-        const float nrm = f16_to_f32(static_cast<uint16_t>(q0 & 0xffffu));
+        const float nrm = f16_to_f32(static_cast<uint16_t>(q[0] & 0xffffu));
         const bool ok = isfinite_f(nrm) && nrm > 0.0f;
         bool fin = true;
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            acc[q] = acc[q] * nrm;
-            fin &= isfinite_f(acc[q]);
+        for (int k = 0; k < 32; ++k) {
+            acc[k] = acc[k] * nrm;
+            fin &= isfinite_f(acc[k]);
         }
         // a vector is bad if either half-wave saw a bad value
         const uint64_t badm = __ballot(!(ok && fin));
         const bool vbad = ((badm >> n) | (badm >> (n + 32))) & 1ull;
-        const bool active = w < nv;
-        const uint32_t vi = v0 + w;
         if (active && h == 0 && vbad) status_fail(lc.status, sidx, 1, vi, ok ? KIND_DECODE_NONFINITE : KIND_CORRUPT);
         if constexpr (!STAGED) {
             if (active && !vbad) {
@@ -3550,10 +3577,10 @@ __global__ __launch_bounds__(TILE) void fib_decode_mfma_kernel(LaunchCommon lc, 
 #pragma unroll
                 for (int bb = 0; bb < 2; ++bb)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) {   // registers q .. q + 3: columns 32bb + 8g + 4h .. + 3
-                        const int q = 16 * bb + 4 * g;
+                    for (int g = 0; g < 4; ++g) {   // registers k .. k + 3: columns 32bb + 8g + 4h .. + 3
+                        const int k = 16 * bb + 4 * g;
                         store_out4(out, lc, orow + 32 * bb + 8 * g + 4 * h,
-                                   make_float4(acc[q], acc[q + 1], acc[q + 2], acc[q + 3]));
+                                   make_float4(acc[k], acc[k + 1], acc[k + 2], acc[k + 3]));
                     }
             }
             continue;
@@ -3575,10 +3602,10 @@ __global__ __launch_bounds__(TILE) void fib_decode_mfma_kernel(LaunchCommon lc, 
 #pragma unroll
                 for (int bb = 0; bb < 2; ++bb)
 #pragma unroll
-                    for (int g = 0; g < 4; ++g) {   // registers q .. q + 3: columns 32bb + 8g + 4h .. + 3
-                        const int q = 16 * bb + 4 * g;
+                    for (int g = 0; g < 4; ++g) {   // registers k .. k + 3: columns 32bb + 8g + 4h .. + 3
+                        const int k = 16 * bb + 4 * g;
                         *reinterpret_cast<float4*>(hs + row * RPITCH + 32 * bb + 8 * g + 4 * h) =
-                            make_float4(acc[q], acc[q + 1], acc[q + 2], acc[q + 3]);
+                            make_float4(acc[k], acc[k + 1], acc[k + 2], acc[k + 3]);
                     }
             }
             wave_sync();
@@ -3595,7 +3622,22 @@ __global__ __launch_bounds__(TILE) void fib_decode_mfma_kernel(LaunchCommon lc, 
             wave_sync();   // the next pass overwrites the staging rows
         }
     }
+}
+
+// The decode's partial sums after the first FIB_PREFIX_BLOCKS blocks, one row of
+// 64 columns per index combination (block 0's index lowest): the reference's
+// sequential f32 products and sums (rotation.rs:136-149) from 0.
+__global__ __launch_bounds__(256) void fib_prefix_kernel(const float* __restrict__ rot32, const float* __restrict__ cb,
+                                                         float* __restrict__ out) {
+    const uint32_t w = blockIdx.x * 4u + (threadIdx.x >> 6), col = threadIdx.x & 63u;
+    float s = 0.0f;
+#pragma unroll
+    for (int b = 0; b < FIB_PREFIX_BLOCKS; ++b) {
+        const float* c = cb + 4u * ((w >> (5 * b)) & 31u);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s = s + rot32[(4 * b + t) * 64 + col] * c[t];
     }
+    out[static_cast<size_t>(w) * 64u + col] = s;
 }
 
 // Counts the products of (f32(Pi)[r][col], codeword component c[j][r % 4])
@@ -3953,18 +3995,35 @@ int launch_fib_encode(const LaunchCommon& lc, const FibDev& fd, const void* in, 
 
 int launch_fib_decode(const LaunchCommon& lc, const FibDev& fd, const uint8_t* wire, void* out, uint32_t nblocks,
                       void* stream) {
-    const uint32_t grid = lc.grid_cap ? std::min(nblocks, lc.grid_cap) : nblocks;
-    if (fd.mfma_decode && lc.fanout > 1)
-        hipLaunchKernelGGL((fib_decode_mfma_kernel<64, true>), dim3(grid), dim3(TILE), 0,
-                           static_cast<hipStream_t>(stream), lc, wire, out, fd.rot32, fd.codebook, lc.segs,
-                           lc.tile_start, lc.tile_seg);
-    else if (fd.mfma_decode)
-        hipLaunchKernelGGL((fib_decode_mfma_kernel<64, false>), dim3(grid), dim3(TILE), 0,
-                           static_cast<hipStream_t>(stream), lc, wire, out, fd.rot32, fd.codebook, lc.segs,
-                           lc.tile_start, lc.tile_seg);
-    else
-        hipLaunchKernelGGL(fib_decode_kernel<64>, dim3(nblocks), dim3(TILE), 0, static_cast<hipStream_t>(stream), lc,
-                           wire, out, fd.rot32t, fd.codebook);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (!fd.mfma_decode) {
+        hipLaunchKernelGGL(fib_decode_kernel<64>, dim3(nblocks), dim3(TILE), 0, st, lc, wire, out, fd.rot32t,
+                           fd.codebook);
+        return hipGetLastError();
+    }
+    if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 half-tiles per tile
+    // The table of partial sums pays while the arithmetic is the bound; past
+    // 12 output bytes per value the decode is bound by its writes and the
+    // table's reads slow them down (config-3 step, table against none: 2 f32
+    // copies 425 / 439 us, 3 474 / 476, 4 527 / 520, 8 798 / 778; 4 bf16 copies
+    // 441 / 460, 8 544 / 527).
+    const bool table = lc.fanout <= (lc.out_dtype == PKV_F32 ? 3u : 6u);
+    auto kern = lc.fanout == 1 ? fib_decode_mfma_kernel<64, false, true>
+                : table        ? fib_decode_mfma_kernel<64, true, true>
+                               : fib_decode_mfma_kernel<64, true, false>;
+    // one half-tile per workgroup (a resident grid walking them was slower: one
+    // copy 172 against 164 us, 8 copies 830 against 778 us for the step) unless
+    // the caller bounds its share of the GPU
+    uint32_t grid = std::min(2 * nblocks, 1u << 23);
+    if (lc.grid_cap) grid = std::min(grid, lc.grid_cap);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(TILE), 0, st, lc, wire, out, fd.rot32, fd.codebook, fd.prefix, lc.segs,
+                       lc.tile_start, lc.tile_seg);
+    return hipGetLastError();
+}
+
+int launch_fib_prefix(const float* rot32, const float* cb, float* out, void* stream) {
+    hipLaunchKernelGGL(fib_prefix_kernel, dim3((1u << (5 * FIB_PREFIX_BLOCKS)) / 4), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), rot32, cb, out);
     return hipGetLastError();
 }
 
