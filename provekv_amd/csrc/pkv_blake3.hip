@@ -145,10 +145,16 @@ __device__ __forceinline__ QuadMsgIdx quad_msg_idx(uint32_t i) {
 }
 
 // One compression on the quad.  (cv_lo, cv_hi) = chaining value words
-// (i, 4 + i) in and out; message word k is word(k), read from LDS.
+// (i, 4 + i) in and out; message word k is word(k), read from LDS -- all 28
+// before the first round, so no round waits for LDS.
 template <typename Word>
 __device__ __forceinline__ void quad_compress(uint32_t& cv_lo, uint32_t& cv_hi, uint32_t i, const QuadMsgIdx& q,
                                               Word word, uint64_t counter, uint32_t block_len, uint32_t flags) {
+    uint32_t m[7][4];
+#pragma unroll
+    for (int r = 0; r < 7; ++r)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[r][k] = word(q.w[r][k]);
     uint32_t a = cv_lo, b = cv_hi;
     uint32_t c = i == 0 ? PKV_B3_IV0 : i == 1 ? PKV_B3_IV1 : i == 2 ? PKV_B3_IV2 : PKV_B3_IV3;
     uint32_t d = i == 0 ? static_cast<uint32_t>(counter)
@@ -157,13 +163,11 @@ __device__ __forceinline__ void quad_compress(uint32_t& cv_lo, uint32_t& cv_hi, 
                         : flags;
 #pragma unroll
     for (int r = 0; r < 7; ++r) {
-        const uint32_t mx = word(q.w[r][0]), my = word(q.w[r][1]);
-        const uint32_t nx = word(q.w[r][2]), ny = word(q.w[r][3]);
-        g1(a, b, c, d, mx, my);
+        g1(a, b, c, d, m[r][0], m[r][1]);
         b = qrot1(b);
         c = qrot2(c);
         d = qrot3(d);
-        g1(a, b, c, d, nx, ny);
+        g1(a, b, c, d, m[r][2], m[r][3]);
         b = qrot3(b);
         c = qrot2(c);
         d = qrot1(d);
@@ -171,6 +175,10 @@ __device__ __forceinline__ void quad_compress(uint32_t& cv_lo, uint32_t& cv_hi, 
     cv_lo = a ^ c;
     cv_hi = b ^ d;
 }
+
+// A quad's block in LDS: 16 words at a pitch of 20, so that the 16 quads of a
+// wave reading the same word fall on 16 different banks.
+constexpr uint32_t QPITCH = 20;
 
 }  // namespace
 
@@ -221,12 +229,18 @@ __global__ __launch_bounds__(256) void blake3_tree_kernel(const uint8_t* __restr
 // Pass 0 with four lanes per chunk: 16 chunks per wave (one per quad), then
 // the wave merges its 16 chaining values over four levels, one parent per
 // active quad.  Tiles are 16 chunks; a range of at most 16 chunks ends here.
+// A small wire leaves a wave or two per SIMD, so latency is what counts: the
+// blocks are loaded four ahead (with each loaded only when its turn came, 16
+// memory round trips were most of the pass) and a block's 28 message words
+// are read from LDS before its rounds: 14.4 Ki chunks 30 -> 22.8 us.  What is
+// left is the rounds' dependent chain, about 13 cycles per instruction at a wave
+// per SIMD.
 __global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restrict__ buf,
                                                           const B3Range* __restrict__ ranges,
                                                           const B3Pass* __restrict__ pass, uint32_t nr,
                                                           uint32_t* __restrict__ cv_out, uint32_t* __restrict__ out) {
-    __shared__ uint32_t blk_s[4][16][16];   // per wave, per quad: the current 64-byte block
-    __shared__ uint32_t cv_s[4][16][8];     // per wave, per quad: its chaining value
+    __shared__ __align__(16) uint32_t blk_s[4][16][QPITCH];   // per wave, per quad: the current 64-byte block
+    __shared__ uint32_t cv_s[4][16][8];                       // per wave, per quad: its chaining value
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t quad = lane >> 2, i = lane & 3u;
     const uint32_t tile = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + wave);
@@ -244,7 +258,7 @@ __global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restr
     const uint32_t nq = ps.count - first < 16u ? ps.count - first : 16u;   // quads with a chunk
     const bool root_group = ps.count <= 16u;
     const QuadMsgIdx qi = quad_msg_idx(i);
-    const uint32_t* my_blk = blk_s[wave][quad];
+    uint32_t* my_blk = blk_s[wave][quad];
 
     uint32_t cv_lo = i == 0 ? PKV_B3_IV0 : i == 1 ? PKV_B3_IV1 : i == 2 ? PKV_B3_IV2 : PKV_B3_IV3;
     uint32_t cv_hi = i == 0 ? PKV_B3_IV4 : i == 1 ? PKV_B3_IV5 : i == 2 ? PKV_B3_IV6 : PKV_B3_IV7;
@@ -255,43 +269,56 @@ __global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restr
         const uint64_t left = rg.len - start;
         const uint32_t clen = left < b3::CHUNK_BYTES ? static_cast<uint32_t>(left) : b3::CHUNK_BYTES;
         // the wave runs as many blocks as its longest chunk (every chunk but
-        // a range's last is whole: 16 blocks); quads past nq and a shorter
-        // last chunk idle through the rest
+        // a range's last is whole: 16 blocks); a shorter last chunk idles
+        // through the rest (quads past nq repeat chunk `first`, unused)
         const uint32_t nblk = clen == 0 ? 1u : (clen + 63u) / 64u;
         const uint32_t wblk = nq > 1u ? 16u : __builtin_amdgcn_readfirstlane(nblk);
-        const uint8_t* base = buf + rg.offset + start;
-        const uint32_t sh = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(base) & 3u);
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(base - sh);
+        const uint8_t* base = buf + rg.offset + start + 16u * i;   // this lane's 16 bytes of block 0
         const bool root = ps.count == 1u;
-        for (uint32_t b = 0; b < wblk; ++b) {
-            const bool live = quad < nq && b < nblk;
-            const uint32_t blen = clen - 64u * b < 64u ? clen - 64u * b : 64u;
-            // lane i: message words 4i .. 4i + 3 from dwords 4i .. 4i + 4 of the block
-            uint32_t dw[5] = {0u, 0u, 0u, 0u, 0u};
-            if (live) {
-                const uint32_t nd = blen ? (sh + blen + 3u) >> 2 : 0u;
-#pragma unroll
-                for (uint32_t k = 0; k < 5; ++k)
-                    if (4u * i + k < nd) dw[k] = p[16u * b + 4u * i + k];
-            }
-            uint32_t w[4];
+        // whole 16-byte pieces, at any byte alignment; zeros past the chunk
+        auto load4 = [&](uint32_t b0, uint4 (&v)[4]) {
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) {
-                w[j] = __builtin_amdgcn_alignbyte(dw[j + 1], dw[j], sh);
-                const int rem = static_cast<int>(blen) - static_cast<int>(4u * (4u * i + j));
-                w[j] = rem >= 4 ? w[j] : rem <= 0 ? 0u : (w[j] & ((1u << (8 * rem)) - 1u));
+                v[j] = make_uint4(0u, 0u, 0u, 0u);
+                if (64u * (b0 + j) + 16u * i + 16u <= clen) __builtin_memcpy(&v[j], base + 64u * (b0 + j), 16);
             }
-            *reinterpret_cast<uint4*>(&blk_s[wave][quad][4u * i]) = make_uint4(w[0], w[1], w[2], w[3]);
-            wave_sync_lds();
-            uint32_t flags = b == 0 ? b3::CHUNK_START : 0u;
-            if (b == nblk - 1) flags |= b3::CHUNK_END | (root ? b3::ROOT : 0u);
-            uint32_t nlo = cv_lo, nhi = cv_hi;
-            quad_compress(nlo, nhi, i, qi, [&](uint32_t k) { return my_blk[k]; }, chunk, blen, flags);
-            if (live) {
-                cv_lo = nlo;
-                cv_hi = nhi;
+        };
+        uint4 nxt[4];
+        load4(0, nxt);
+        // the piece that ends inside the chunk's last 16 bytes, byte by byte
+        const uint32_t tb = clen >> 6, trem = clen & 15u;
+        const bool has_tail = trem != 0u && ((clen >> 4) & 3u) == i;
+        uint32_t tw[4] = {0u, 0u, 0u, 0u};
+        if (has_tail) {
+#pragma unroll
+            for (uint32_t k = 0; k < 15; ++k)
+                if (k < trem) tw[k >> 2] |= static_cast<uint32_t>(base[64u * tb + k]) << (8u * (k & 3u));
+        }
+        for (uint32_t b0 = 0; b0 < wblk; b0 += 4) {
+            uint4 cur[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cur[j] = nxt[j];
+            if (b0 + 4 < wblk) load4(b0 + 4, nxt);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t b = b0 + j;
+                if (b < wblk) {   // wave-uniform
+                    uint4 w = cur[j];
+                    if (has_tail && b == tb) w = make_uint4(tw[0], tw[1], tw[2], tw[3]);
+                    *reinterpret_cast<uint4*>(my_blk + 4u * i) = w;
+                    wave_sync_lds();
+                    const uint32_t blen = clen - 64u * b < 64u ? clen - 64u * b : 64u;
+                    uint32_t flags = b == 0 ? b3::CHUNK_START : 0u;
+                    if (b == nblk - 1) flags |= b3::CHUNK_END | (root ? b3::ROOT : 0u);
+                    uint32_t nlo = cv_lo, nhi = cv_hi;
+                    quad_compress(nlo, nhi, i, qi, [&](uint32_t k) { return my_blk[k]; }, chunk, blen, flags);
+                    if (b < nblk) {
+                        cv_lo = nlo;
+                        cv_hi = nhi;
+                    }
+                    wave_sync_lds();   // every quad has read its block before the next one lands
+                }
             }
-            wave_sync_lds();   // every quad has read its block before the next one lands
         }
     }
     // merge the quads' chaining values: level s pairs quads q, q + s
@@ -407,64 +434,150 @@ __global__ __launch_bounds__(256) void blake3_merge4_kernel(const B3Pass* __rest
     }
 }
 
-// Layer digests: entry i holds the payload digests of layer i % layers, key
-// then value (16 words); out[i] = blake3 of serde_json's compact text of
+// The last pass of a tier together with its layer digests: one workgroup per
+// layer entry, waves 0-3 on its key range and 4-7 on its value range.  A range
+// with values left (count > 0, at most 64 in a last pass) is merged as
+// blake3_merge4_kernel does; one that ended earlier (and every range when
+// `pass` is null) has its payload digest in `digests` already.  Then
+// layer_out[i] = blake3 of serde_json's compact text of
 // json!({"layer_index", "key_digests": [k], "value_digests": [v]}) -- a
 // BTreeMap (serde_json without preserve_order), so the keys print sorted:
 //   {"key_digests":["<64 hex>"],"layer_index":<decimal>,"value_digests":["<64 hex>"]}
-// At most 194 bytes: one chunk of four blocks, hashed by one lane.
-__global__ __launch_bounds__(64) void blake3_layer_kernel(const uint32_t* __restrict__ kv, uint32_t n,
-                                                          uint32_t layers, uint32_t* __restrict__ out) {
-    __shared__ uint32_t text[64][65];   // one 256-byte row per lane (+1 word: no bank conflicts)
-    const uint32_t i = blockIdx.x * 64u + threadIdx.x;
-    if (i >= n) return;
-    uint32_t* row = text[threadIdx.x];
-    for (int w = 0; w < 64; ++w) row[w] = 0u;
-    uint32_t pos = 0;
-    auto put = [&](uint32_t byte) {
-        row[pos >> 2] |= byte << (8u * (pos & 3u));
-        ++pos;
-    };
-    auto put_str = [&](const char* s) {
-        for (; *s; ++s) put(static_cast<uint8_t>(*s));
-    };
-    auto put_hex = [&](const uint32_t* d) {
-        for (int j = 0; j < 32; ++j) {
-            const uint32_t byte = (d[j >> 2] >> (8 * (j & 3))) & 255u;
-            const uint32_t hi = byte >> 4, lo = byte & 15u;
-            put(hi < 10u ? '0' + hi : 'a' + hi - 10u);
-            put(lo < 10u ? '0' + lo : 'a' + lo - 10u);
+// with layer i % layers; at most 194 bytes, one chunk of four blocks: each lane
+// of wave 0 forms four bytes of the text and the blocks are chained on quads
+// (one lane building and hashing the text alone took 10-12 us in a launch of
+// its own after a 9 us merge; the two together take 12.8 us at config 3's pool,
+// 48 workgroups, 10.7 us at its shells).
+struct LayerText {
+    char key[18] = "{\"key_digests\":[\"";
+    char index[18] = "\"],\"layer_index\":";
+    char value[20] = ",\"value_digests\":[\"";
+    char end[4] = "\"]}";
+};
+__constant__ LayerText c_layer_text = LayerText();
+
+__global__ __launch_bounds__(512) void blake3_layer_kernel(const B3Pass* __restrict__ pass,
+                                                           const uint32_t* __restrict__ cv_in, uint32_t* digests,
+                                                           uint32_t n, uint32_t layers,
+                                                           uint32_t* __restrict__ layer_out) {
+    __shared__ uint32_t cv_s[8][16][8];   // per wave, per quad: a chaining value
+    __shared__ uint32_t dig_s[2][8];
+    __shared__ uint32_t text_s[64];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t side = wave >> 2, wv = wave & 3u, quad = lane >> 2, i = lane & 3u;
+    const QuadMsgIdx qi = quad_msg_idx(i);
+    auto merge = [&](uint32_t w, uint32_t n, bool last) {   // as in blake3_merge4_kernel
+        for (uint32_t s = 1; s < n; s <<= 1) {
+            const uint32_t c = (n + s - 1u) / s;
+            const bool act = (quad & (2u * s - 1u)) == 0u && quad / s + 1u < c;
+            const uint32_t partner = act ? quad + s : quad;
+            uint32_t plo = i == 0 ? PKV_B3_IV0 : i == 1 ? PKV_B3_IV1 : i == 2 ? PKV_B3_IV2 : PKV_B3_IV3;
+            uint32_t phi = i == 0 ? PKV_B3_IV4 : i == 1 ? PKV_B3_IV5 : i == 2 ? PKV_B3_IV6 : PKV_B3_IV7;
+            const uint32_t* left = cv_s[w][quad];
+            const uint32_t* right = cv_s[w][partner];
+            quad_compress(plo, phi, i, qi, [&](uint32_t k) { return k < 8u ? left[k] : right[k - 8u]; }, 0,
+                          b3::BLOCK_BYTES, b3::PARENT | (last && c == 2u ? b3::ROOT : 0u));
+            wave_sync_lds();   // all reads of this level done
+            if (act) {
+                cv_s[w][quad][i] = plo;
+                cv_s[w][quad][4u + i] = phi;
+            }
+            wave_sync_lds();
         }
     };
-    uint32_t d[16];
+    for (uint32_t entry = blockIdx.x; entry < n; entry += gridDim.x) {   // one each but for millions of layers
+        const uint64_t r = 2ull * entry + side;
+        const uint32_t nw = pass ? pass[r].count : 0u;   // values of this range (<= 64)
+        const uint32_t base = 16u * wv;
+        const uint32_t nq = nw > base ? (nw - base < 16u ? nw - base : 16u) : 0u;   // this wave's values
+        if (quad < nq) {
+            const uint32_t* src = cv_in + 8ull * (pass[r].in_base + base + quad);
+            cv_s[wave][quad][i] = src[i];
+            cv_s[wave][quad][4u + i] = src[4u + i];
+        }
+        wave_sync_lds();
+        if (nq > 1) merge(wave, nq, nw <= 16u);
+        __syncthreads();
+        if (wv == 0) {
+            const uint32_t ng = (nw + 15u) / 16u;   // waves that held values
+            if (ng > 1) {
+                // the waves' results become quads 0 .. ng - 1 of this side's first wave
+                uint32_t wlo = 0, whi = 0;
+                if (quad < ng) {
+                    wlo = cv_s[wave + quad][0][i];
+                    whi = cv_s[wave + quad][0][4u + i];
+                }
+                wave_sync_lds();
+                if (quad < ng) {
+                    cv_s[wave][quad][i] = wlo;
+                    cv_s[wave][quad][4u + i] = whi;
+                }
+                wave_sync_lds();
+                merge(wave, ng, true);
+            }
+            if (lane < 8u) {
+                uint32_t* dst = digests + 8ull * r;   // only 4-byte aligned
+                uint32_t v;
+                if (nw) {
+                    v = cv_s[wave][0][lane];
+                    dst[lane] = v;
+                } else {
+                    v = dst[lane];
+                }
+                dig_s[side][lane] = v;
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const uint32_t li = entry % layers;
+            uint32_t nd = 1, top = 1;   // decimal digits of li, 10^(nd - 1)
+            for (uint32_t v = li; v >= 10u; v /= 10u) {
+                ++nd;
+                top *= 10u;
+            }
+            const uint32_t p1 = 17u, p2 = p1 + 64u, p3 = p2 + 17u, p4 = p3 + nd, p5 = p4 + 19u, p6 = p5 + 64u;
+            const uint32_t len = p6 + 3u;
+            uint32_t word = 0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) d[w] = kv[16ull * i + w];
-    put_str("{\"key_digests\":[\"");
-    put_hex(d);
-    put_str("\"],\"layer_index\":");
-    uint32_t li = i % layers, digits[10], nd = 0;
-    do {
-        digits[nd++] = li % 10u;
-        li /= 10u;
-    } while (li);
-    while (nd) put('0' + digits[--nd]);
-    put_str(",\"value_digests\":[\"");
-    put_hex(d + 8);
-    put_str("\"]}");
-    const uint32_t len = pos, nblk = (len + 63u) / 64u;
-    uint32_t cv[8];
-    b3::set_iv(cv);
-    for (uint32_t b = 0; b < nblk; ++b) {
-        uint32_t m[16];
-#pragma unroll
-        for (int w = 0; w < 16; ++w) m[w] = row[16 * b + w];
-        uint32_t flags = b == 0 ? b3::CHUNK_START : 0u;
-        if (b == nblk - 1) flags |= b3::CHUNK_END | b3::ROOT;
-        b3::compress(cv, m, 0, b == nblk - 1 ? len - 64u * b : 64u, flags);
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint32_t p = 4u * lane + k;
+                uint32_t ch = 0;
+                if ((p >= p1 && p < p2) || (p >= p5 && p < p6)) {
+                    const uint32_t s = p >= p5 ? 1u : 0u, j = p - (s ? p5 : p1);
+                    const uint32_t nib = (dig_s[s][j >> 3] >> (8u * ((j >> 1) & 3u) + (j & 1u ? 0u : 4u))) & 15u;
+                    ch = nib < 10u ? '0' + nib : 'a' + nib - 10u;
+                } else if (p >= p3 && p < p4) {
+                    uint32_t d = top;
+                    for (uint32_t q = p3; q < p; ++q) d /= 10u;
+                    ch = '0' + li / d % 10u;
+                } else if (p < len) {
+                    ch = static_cast<uint8_t>(p < p1   ? c_layer_text.key[p]
+                                              : p < p3 ? c_layer_text.index[p - p2]
+                                              : p < p5 ? c_layer_text.value[p - p4]
+                                                       : c_layer_text.end[p - p6]);
+                }
+                word |= ch << (8u * k);
+            }
+            text_s[lane] = word;
+            wave_sync_lds();
+            uint32_t cv_lo = i == 0 ? PKV_B3_IV0 : i == 1 ? PKV_B3_IV1 : i == 2 ? PKV_B3_IV2 : PKV_B3_IV3;
+            uint32_t cv_hi = i == 0 ? PKV_B3_IV4 : i == 1 ? PKV_B3_IV5 : i == 2 ? PKV_B3_IV6 : PKV_B3_IV7;
+            const uint32_t nblk = (len + 63u) / 64u;
+#pragma unroll 1
+            for (uint32_t b = 0; b < nblk; ++b) {   // every quad the same
+                uint32_t flags = b == 0 ? b3::CHUNK_START : 0u;
+                if (b == nblk - 1) flags |= b3::CHUNK_END | b3::ROOT;
+                quad_compress(cv_lo, cv_hi, i, qi, [&](uint32_t k) { return text_s[16u * b + k]; }, 0,
+                              b == nblk - 1 ? len - 64u * b : 64u, flags);
+            }
+            if (quad == 0) {
+                uint32_t* dst = layer_out + 8ull * entry;
+                dst[i] = cv_lo;
+                dst[4u + i] = cv_hi;
+            }
+        }
+        __syncthreads();   // the next entry rewrites the values and digests
     }
-    uint32_t* dst = out + 8ull * i;
-#pragma unroll
-    for (int w = 0; w < 8; ++w) dst[w] = cv[w];
 }
 
 int launch_blake3_pass(const uint8_t* buf, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
@@ -492,10 +605,11 @@ int launch_blake3_merge4(const B3Pass* pass, uint32_t nr, uint32_t tiles, const 
     return hipGetLastError();
 }
 
-int launch_blake3_layers(const uint32_t* kv, uint32_t n, uint32_t layers, uint32_t* out, void* stream) {
+int launch_blake3_layers(const B3Pass* pass, const uint32_t* cv_in, uint32_t* digests, uint32_t n, uint32_t layers,
+                         uint32_t* out, void* stream) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(blake3_layer_kernel, dim3((n + 63u) / 64u), dim3(64), 0, static_cast<hipStream_t>(stream), kv,
-                       n, layers, out);
+    hipLaunchKernelGGL(blake3_layer_kernel, dim3(n < (1u << 20) ? n : 1u << 20), dim3(512), 0,
+                       static_cast<hipStream_t>(stream), pass, cv_in, digests, n, layers, out);
     return hipGetLastError();
 }
 

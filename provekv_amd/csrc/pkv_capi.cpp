@@ -1404,8 +1404,9 @@ struct B3Plan {
 
 // Chunks below which pass 0 puts four lanes on a chunk (16 chunks per wave,
 // ~1.4x the instructions, a quarter of the latency): one lane per chunk would
-// leave the GPU with fewer than half a wave per SIMD.  Measured at config 3:
-// the pool's 14.4 Ki chunks 47 -> 31 us, the shells' 48 Ki chunks 43 -> 50 us.
+// leave the GPU with fewer than half a wave per SIMD.  Measured (both passes of
+// a call, one lane / four): config 3's pool, 14.4 Ki chunks, 47 / 30 us; its
+// shells, 48 Ki chunks, 51 / 50 us; 64 Ki chunks 50 / 61 us.
 constexpr uint64_t kB3QuadBelow = 32ull * 1024;
 
 int plan_blake3(const pkv_range* ranges, uint32_t nr, uint64_t buf_bytes, B3Plan* plan) {
@@ -1450,9 +1451,12 @@ int plan_blake3(const pkv_range* ranges, uint32_t nr, uint64_t buf_bytes, B3Plan
     return PKV_OK;
 }
 
-// Caller holds ctx->mu and has made the device current.
+// Caller holds ctx->mu and has made the device current.  With d_layers (nr
+// even: key and value ranges in turn) the last pass also forms the nr / 2
+// layer digests.
 int blake3_ranges_locked(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_bytes, const pkv_range* ranges,
-                         uint32_t nr, uint8_t* d_out, hipStream_t stream) {
+                         uint32_t nr, uint8_t* d_out, hipStream_t stream, uint8_t* d_layers = nullptr,
+                         uint32_t layers = 0) {
     B3Plan plan;
     int rc = plan_blake3(ranges, nr, buf_bytes, &plan);
     if (rc) return rc;
@@ -1495,8 +1499,13 @@ int blake3_ranges_locked(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_bytes,
         if (p == 0)
             e = plan.quad ? launch_blake3_quad(d_buf, d_ranges, d_pass, nr, plan.tiles[p], d_cv, out, stream)
                           : launch_blake3_pass(d_buf, d_ranges, d_pass, nr, plan.tiles[p], d_cv, out, stream);
-        else
+        else if (!d_layers || p + 1 < plan.tiles.size())
             e = launch_blake3_merge4(d_pass, nr, plan.tiles[p], d_cv, d_cv, out, stream);
+    }
+    if (d_layers && !e) {
+        const size_t last = plan.tiles.size() - 1;   // a single pass ended every range itself
+        const auto* d_pass = last ? reinterpret_cast<const B3Pass*>(d + pass_off) + last * (nr + 1) : nullptr;
+        e = launch_blake3_layers(d_pass, d_cv, out, nr / 2, layers, reinterpret_cast<uint32_t*>(d_layers), stream);
     }
     const int rc2 = finish_slot(sl, stream);
     if (e) return hip_status(static_cast<hipError_t>(e));
@@ -1525,8 +1534,9 @@ int pkv_blake3_layer_digests(pkv_ctx* ctx, const uint8_t* d_kv_digests, uint32_t
         return PKV_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
-    const int e = launch_blake3_layers(reinterpret_cast<const uint32_t*>(d_kv_digests), n, layers,
-                                       reinterpret_cast<uint32_t*>(d_out), stream);
+    const int e = launch_blake3_layers(nullptr, nullptr,
+                                       reinterpret_cast<uint32_t*>(const_cast<uint8_t*>(d_kv_digests)), n, layers,
+                                       reinterpret_cast<uint32_t*>(d_out), stream);   // reads the digests only
     return e ? hip_status(static_cast<hipError_t>(e)) : PKV_OK;
 }
 
@@ -1540,12 +1550,8 @@ int pkv_blake3_tier_digests(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_byt
         return PKV_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    const int rc = blake3_ranges_locked(ctx, d_buf, buf_bytes, ranges, 2 * n, d_blob_digests, st);
-    if (rc) return rc;
-    const int e = launch_blake3_layers(reinterpret_cast<const uint32_t*>(d_blob_digests), n, layers,
-                                       reinterpret_cast<uint32_t*>(d_layer_digests), st);
-    return e ? hip_status(static_cast<hipError_t>(e)) : PKV_OK;
+    return blake3_ranges_locked(ctx, d_buf, buf_bytes, ranges, 2 * n, d_blob_digests, static_cast<hipStream_t>(stream),
+                                d_layer_digests, layers);
 }
 
 int pkv_blake3(pkv_ctx* ctx, const void* data, uint64_t len, uint8_t out[32]) {

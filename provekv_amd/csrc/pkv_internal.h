@@ -236,6 +236,8 @@ int launch_blake3_quad(const uint8_t* buf, const B3Range* ranges, const B3Pass* 
 // compression, one workgroup per tile.
 int launch_blake3_merge4(const B3Pass* pass, uint32_t nr, uint32_t tiles, const uint32_t* cv_in, uint32_t* cv_out,
                          uint32_t* out, void* stream);
-int launch_blake3_layers(const uint32_t* kv, uint32_t n, uint32_t layers, uint32_t* out, void* stream);
+// A tier's last pass (null: every range of it has ended) and its n layer digests.
+int launch_blake3_layers(const B3Pass* pass, const uint32_t* cv_in, uint32_t* digests, uint32_t n, uint32_t layers,
+                         uint32_t* out, void* stream);
 
 }  // namespace pkv
