@@ -265,6 +265,38 @@ int pkv_decode_segments_bounded(pkv_ctx* ctx, const pkv_profile* prof, int radii
                                 uint32_t fanout, uint64_t fanout_stride, uint32_t max_workgroups,
                                 uint32_t* d_status, void* stream);
 
+/* The status words of several calls cleared (all ones) by one launch: buffer i
+ * holds 2 * nsegs[i] words.  For a step of several pkv_run_segments calls with
+ * PKV_STATUS_CLEARED, each of which would otherwise clear its own words in a
+ * launch before its kernel.  n <= PKV_STATUS_BUFFERS_MAX. */
+#define PKV_STATUS_BUFFERS_MAX 8u
+int pkv_status_clear(pkv_ctx* ctx, uint32_t* const* d_status, const uint32_t* nsegs, uint32_t n, void* stream);
+
+/* One encode or decode of a segment table, every option in a struct:
+ * pkv_encode_segments_bounded (encode != 0; fanout 1) or
+ * pkv_decode_segments_bounded.  PKV_STATUS_CLEARED: d_status (required) holds
+ * cleared words by the time the call's kernel runs -- pkv_status_clear earlier
+ * on `stream`, or ordered before it by an event -- and is not cleared again. */
+#define PKV_STATUS_CLEARED 1u
+typedef struct pkv_segments_op {
+    int32_t encode;
+    int32_t radii_codec;
+    int32_t dtype;            /* of the tensor: encode input or decode output */
+    uint32_t flags;
+    void* d_tensor;           /* read by an encode, written by a decode */
+    uint64_t elems;
+    const pkv_seg* segs;
+    uint8_t* d_wire;
+    uint64_t wire_bytes;
+    uint64_t fanout_stride;
+    uint32_t nseg;
+    uint32_t fanout;
+    uint32_t max_workgroups;  /* 0: no bound */
+    uint32_t reserved;        /* 0 */
+    uint32_t* d_status;
+} pkv_segments_op;
+int pkv_run_segments(pkv_ctx* ctx, const pkv_profile* prof, const pkv_segments_op* op, void* stream);
+
 /* pkv_decode_segments_ex without any allocation: no hipMalloc, hipFree or
  * other allocating call, here or in the kernels.  No counterpart in the
  * reference; for callers that cannot allocate device memory (tight serving

@@ -47,7 +47,7 @@ EXPORTS = (
     "pkv_fib_constants", "pkv_profile_constants", "pkv_payload_len", "pkv_header_len", "pkv_blob_len",
     "pkv_write_header",
     "pkv_segments_status", "pkv_encode_segments", "pkv_encode_segments_bounded", "pkv_decode_segments", "pkv_decode_segments_ex",
-    "pkv_decode_segments_bounded", "pkv_decode_segments_noalloc",
+    "pkv_decode_segments_bounded", "pkv_decode_segments_noalloc", "pkv_status_clear", "pkv_run_segments",
     "pkv_encode_batch_compact",
     "pkv_decode_batch_compact", "pkv_parse_header", "pkv_record_len", "pkv_encode_vectors", "pkv_decode_vectors",
     "pkv_constants_cache_stats", "pkv_constants_cache_clear", "pkv_prepared_len", "pkv_turbo_prepare_queries",
@@ -57,6 +57,18 @@ EXPORTS = (
     "pkv_host_angle_bins", "pkv_host_octant_bins", "pkv_host_logf",
     "pkv_host_expf", "pkv_host_expf_fused", "pkv_host_div255", "pkv_host_f32_stable_rel50", "pkv_code_from_json", "pkv_fib_digests", "pkv_host_blake3",
 )
+
+
+class SegmentsOp(C.Structure):
+    """pkv_segments_op"""
+    _fields_ = [("encode", C.c_int32), ("radii_codec", C.c_int32), ("dtype", C.c_int32), ("flags", C.c_uint32),
+                ("d_tensor", C.c_void_p), ("elems", C.c_uint64), ("segs", C.c_void_p), ("d_wire", C.c_void_p),
+                ("wire_bytes", C.c_uint64), ("fanout_stride", C.c_uint64), ("nseg", C.c_uint32),
+                ("fanout", C.c_uint32), ("max_workgroups", C.c_uint32), ("reserved", C.c_uint32),
+                ("d_status", C.c_void_p)]
+
+
+STATUS_CLEARED = 1
 
 
 class Seg(C.Structure):
@@ -155,6 +167,8 @@ def _declare(L):
         "pkv_decode_segments_ex": ([P, P, I32, P, U64, P, U32, P, I32, U64, U32, U64, P, P], I32),
         "pkv_decode_segments_bounded": ([P, P, I32, P, U64, P, U32, P, I32, U64, U32, U64, U32, P, P], I32),
         "pkv_decode_segments_noalloc": ([P, P, I32, P, U64, P, U32, P, I32, U64, U32, U64, P, P], I32),
+        "pkv_status_clear": ([P, P, P, U32, P], I32),
+        "pkv_run_segments": ([P, P, P, P], I32),
         "pkv_encode_batch_compact": ([P, P, I32, P, U64, P, U64, P, P], I32),
         "pkv_decode_batch_compact": ([P, P, P, U64, P, U64, P, P], I32),
         "pkv_parse_header": ([P, P, U64, P, P], I32),

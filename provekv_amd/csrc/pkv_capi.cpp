@@ -462,15 +462,18 @@ FibDev fib_dev(const pkv_profile* p) {
     return f;
 }
 
-// Clears the status words and launches the encode or decode kernel of the
+// Clears the status words (unless the caller has) and launches the encode or decode kernel of the
 // profile over a device-resident segment table (dsegs, dtiles: nseg + 1 tile
 // prefix, nblocks tiles in all).  Returns a hipError_t as int.
 int launch_segments(const pkv_profile* prof, int radii, bool encode, int dtype, const void* d_f32,
                     const uint8_t* d_wire, const SegDev* dsegs, const uint32_t* dtiles, uint32_t nseg,
                     uint32_t nblocks, uint32_t* status, bool per_vector, uint32_t fanout, uint64_t fanout_stride,
-                    uint32_t grid_cap, hipStream_t stream, float* diag = nullptr, const uint32_t* dmap = nullptr) {
-    int e = launch_fill_u32(status, STATUS_NONE, 2ull * nseg, stream);
-    if (e) return e;
+                    uint32_t grid_cap, hipStream_t stream, float* diag = nullptr, const uint32_t* dmap = nullptr,
+                    bool cleared = false) {
+    if (!cleared) {
+        const int e = launch_fill_u32(status, STATUS_NONE, 2ull * nseg, stream);
+        if (e) return e;
+    }
     LaunchCommon lc;
     lc.segs = dsegs;
     lc.tile_start = dtiles;
@@ -502,7 +505,7 @@ int run_segments_locked(pkv_ctx* ctx, const pkv_profile* prof, int radii, bool e
                         const void* d_f32, uint64_t f32_elems, const pkv_seg* segs, uint32_t nseg,
                         const uint8_t* d_wire, uint64_t wire_bytes, uint32_t* d_status, hipStream_t stream,
                         bool per_vector = false, uint32_t fanout = 1, uint64_t fanout_stride = 0,
-                        uint32_t grid_cap = 0, float* diag = nullptr) {
+                        uint32_t grid_cap = 0, float* diag = nullptr, bool cleared = false) {
     if (!ctx || !prof) return PKV_ERR_INVALID_ARG;
     if (prof->kind == PKV_CODEC_TURBO && radii != PKV_RADII_F32 && radii != PKV_RADII_LOG_U8)
         return PKV_ERR_INVALID_ARG;
@@ -530,7 +533,7 @@ int run_segments_locked(pkv_ctx* ctx, const pkv_profile* prof, int radii, bool e
     if (rc) return rc;
     uint32_t* status = d_status ? d_status : dstat;
     const int e = launch_segments(prof, radii, encode, dtype, d_f32, d_wire, dsegs, dtiles, nseg, tiles[nseg], status,
-                                  per_vector, fanout, fanout_stride, grid_cap, stream, diag, dmap);
+                                  per_vector, fanout, fanout_stride, grid_cap, stream, diag, dmap, cleared);
     int rc2 = finish_slot(sl, stream);
     if (e) return hip_status(static_cast<hipError_t>(e));
     if (rc2 || d_status) return rc2;
@@ -1303,6 +1306,31 @@ int pkv_decode_segments_bounded(pkv_ctx* ctx, const pkv_profile* prof, int radii
     return run_segments_locked(ctx, prof, radii_codec, false, out_dtype, d_out, out_elems, segs, nseg, d_wire,
                                wire_bytes, d_status, static_cast<hipStream_t>(stream), false, fanout, fanout_stride,
                                max_workgroups);
+}
+
+int pkv_status_clear(pkv_ctx* ctx, uint32_t* const* d_status, const uint32_t* nsegs, uint32_t n, void* stream) {
+    if (!ctx || n > PKV_STATUS_BUFFERS_MAX || (n && (!d_status || !nsegs))) return PKV_ERR_INVALID_ARG;
+    FillList list{};
+    list.count = n;
+    for (uint32_t i = 0; i < n; ++i) {
+        if (nsegs[i] && (!d_status[i] || reinterpret_cast<uintptr_t>(d_status[i]) % 4)) return PKV_ERR_INVALID_ARG;
+        list.p[i] = d_status[i];
+        list.n[i] = 2ull * nsegs[i];
+    }
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    HIP_TRY(hipSetDevice(ctx->device));
+    return hip_status(static_cast<hipError_t>(launch_fill_list(list, STATUS_NONE, stream)));
+}
+
+int pkv_run_segments(pkv_ctx* ctx, const pkv_profile* prof, const pkv_segments_op* op, void* stream) {
+    if (!ctx || !op || (op->flags & ~PKV_STATUS_CLEARED) || op->reserved) return PKV_ERR_INVALID_ARG;
+    const bool cleared = (op->flags & PKV_STATUS_CLEARED) != 0;
+    if (cleared && !op->d_status) return PKV_ERR_INVALID_ARG;
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    return run_segments_locked(ctx, prof, op->radii_codec, op->encode != 0, op->dtype, op->d_tensor, op->elems,
+                               op->segs, op->nseg, op->d_wire, op->wire_bytes, op->d_status,
+                               static_cast<hipStream_t>(stream), false, op->fanout, op->fanout_stride,
+                               op->max_workgroups, nullptr, cleared);
 }
 
 // pkv_decode_segments_ex with the table and its tile prefix in this device's

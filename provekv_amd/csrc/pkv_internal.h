@@ -176,6 +176,13 @@ int launch_fib_encode(const LaunchCommon& lc, const FibDev& fd, const void* in, 
                       void* stream);
 int launch_fib_decode(const LaunchCommon& lc, const FibDev& fd, const uint8_t* wire, void* out,
                       uint32_t nblocks, void* stream);
+// Up to PKV_STATUS_BUFFERS_MAX arrays filled with one value by one launch.
+struct FillList {
+    uint32_t* p[PKV_STATUS_BUFFERS_MAX];
+    uint64_t n[PKV_STATUS_BUFFERS_MAX];
+    uint32_t count;
+};
+int launch_fill_list(const FillList& list, uint32_t value, void* stream);
 int launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, void* stream);
 // Measure the cheap-log bound table the BlockLogU8 encodes read (once per
 // device, before any encode there); copy it (256 floats) to device memory.

@@ -3666,6 +3666,15 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t value, uint64_t n) {
     if (i < n) p[i] = value;
 }
 
+// One row of workgroups per array.
+__global__ void fill_list_kernel(FillList list, uint32_t value) {
+    uint32_t* p = list.p[blockIdx.y];
+    const uint64_t n = list.n[blockIdx.y];
+    for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < n;
+         i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
+        p[i] = value;
+}
+
 // g_logb measurement: every normal positive float v in [2^-126, 2^128), a
 // contiguous run of `per` per thread.  The running maximum of
 // |cheap_logf(v) - logf(v)| (exact in f64, rounded up to f32) goes to
@@ -3807,6 +3816,16 @@ int launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, void* stream) {
     if (n == 0) return hipSuccess;
     uint32_t blocks = static_cast<uint32_t>((n + 255) / 256);
     hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream), p, value, n);
+    return hipGetLastError();
+}
+
+int launch_fill_list(const FillList& list, uint32_t value, void* stream) {
+    uint64_t most = 0;
+    for (uint32_t k = 0; k < list.count; ++k) most = std::max(most, list.n[k]);
+    if (most == 0) return hipSuccess;
+    const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((most + 255) / 256, 4096));
+    hipLaunchKernelGGL(fill_list_kernel, dim3(blocks, list.count), dim3(256), 0, static_cast<hipStream_t>(stream), list,
+                       value);
     return hipGetLastError();
 }
 

@@ -83,6 +83,15 @@ class Context:
         L.check(L.lib().pkv_radii_log_bound(self.ptr, out.ctypes.data), "pkv_radii_log_bound")
         return out
 
+    def clear_status(self, buffers, stream=None) -> None:
+        """Clear several calls' status words in one launch (pkv_status_clear):
+        rows of (32-bit tensor, segments).  The calls then take
+        status_cleared=True."""
+        ptrs = (C.c_void_p * len(buffers))(*[Profile._status_ptr(st, n) for st, n in buffers])
+        counts = (C.c_uint32 * len(buffers))(*[n for _, n in buffers])
+        L.check(L.lib().pkv_status_clear(self.ptr, ptrs, counts, len(buffers), _stream_ptr(stream)),
+                "pkv_status_clear")
+
     # ------------------------------------------------------------ digests
     def blake3_ranges(self, buf, ranges, out=None, stream=None):
         """BLAKE3 of byte ranges of device uint8 tensor `buf` (rows of
@@ -261,11 +270,23 @@ class Profile:
             raise ValueError(f"status must be a contiguous 32-bit tensor of >= {2 * nseg} elements")
         return status.data_ptr()
 
+    def _run_cleared(self, encode, radii, dtype, tensor, segs, wire, fanout, fanout_stride, max_workgroups, status,
+                     stream) -> None:
+        if status is None:
+            raise ValueError("status_cleared needs the status tensor")
+        op = L.SegmentsOp(int(encode), radii, dtype, L.STATUS_CLEARED, tensor.data_ptr(), tensor.numel(),
+                          segs.ctypes.data, wire.data_ptr(), wire.numel(), fanout_stride, len(segs), fanout,
+                          max_workgroups, 0, self._status_ptr(status, len(segs)))
+        L.check(L.lib().pkv_run_segments(self.ctx.ptr, self._ptr, C.byref(op), _stream_ptr(stream)),
+                "pkv_run_segments")
+
     def encode_segments(self, inp, segs: np.ndarray, wire, radii: int = L.RADII_F32, status=None,
-                        stream=None, max_workgroups: int = 0) -> None:
+                        stream=None, max_workgroups: int = 0, status_cleared: bool = False) -> None:
         """Encode every segment of `segs` from device tensor `inp` (f32 or
         bf16) into device uint8 tensor `wire` in one launch.  max_workgroups
-        > 0 bounds the fib encode's persistent grid (pkv_encode_segments_bounded)."""
+        > 0 bounds the fib encode's persistent grid (pkv_encode_segments_bounded).
+        status_cleared: Context.clear_status cleared `status` earlier in
+        stream order, so this call launches its kernel alone."""
         torch = _torch()
         segs = np.ascontiguousarray(segs, dtype=SEG_DTYPE)
         dtype = L.DT_BF16 if inp.dtype == torch.bfloat16 else L.DT_F32
@@ -275,6 +296,9 @@ class Profile:
             raise TypeError("wire must be uint8")
         if not (inp.is_contiguous() and wire.is_contiguous()):
             raise ValueError("tensors must be contiguous")
+        if status_cleared:
+            self._run_cleared(True, radii, dtype, inp, segs, wire, 1, 0, max_workgroups, status, stream)
+            return
         st = self._status_ptr(status, len(segs))
         if max_workgroups:
             rc = L.lib().pkv_encode_segments_bounded(self.ctx.ptr, self._ptr, radii, dtype, inp.data_ptr(),
@@ -288,11 +312,13 @@ class Profile:
         L.check(rc, "pkv_encode_segments")
 
     def decode_segments(self, wire, segs: np.ndarray, out, radii: int = L.RADII_F32, status=None,
-                        stream=None, fanout: int = 1, fanout_stride: int = 0, max_workgroups: int = 0) -> None:
+                        stream=None, fanout: int = 1, fanout_stride: int = 0, max_workgroups: int = 0,
+                        status_cleared: bool = False) -> None:
         """Decode into `out` (float32, bfloat16 or float16; the latter two are
         the f32 decode rounded to nearest even), each vector written `fanout`
         times `fanout_stride` elements apart.  max_workgroups > 0 bounds the
-        head_dim-64 turbo decode's grid (it then loops over the tiles)."""
+        head_dim-64 turbo decode's grid (it then loops over the tiles).
+        status_cleared as for encode_segments."""
         torch = _torch()
         segs = np.ascontiguousarray(segs, dtype=SEG_DTYPE)
         dts = {torch.float32: L.DT_F32, torch.bfloat16: L.DT_BF16, torch.float16: L.DT_F16}
@@ -300,6 +326,10 @@ class Profile:
             raise TypeError("decode writes float32 / bfloat16 / float16 from a uint8 wire")
         if not (out.is_contiguous() and wire.is_contiguous()):
             raise ValueError("tensors must be contiguous")
+        if status_cleared:
+            self._run_cleared(False, radii, dts[out.dtype], out, segs, wire, fanout, fanout_stride, max_workgroups,
+                              status, stream)
+            return
         st = self._status_ptr(status, len(segs))
         if max_workgroups:
             rc = L.lib().pkv_decode_segments_bounded(self.ctx.ptr, self._ptr, radii, wire.data_ptr(), wire.numel(),

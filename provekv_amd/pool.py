@@ -186,18 +186,35 @@ class TwoTierPlan:
         }
 
     def encode(self, corpus, bufs, stream=None):
-        """Pool build + all shells: two launches (fib, turbo)."""
-        self.fib.encode_segments(corpus, self.pool.enc, bufs["pool_wire"], status=bufs["pool_status"],
-                                 stream=stream)
+        """Pool build + all shells: two launches (fib, turbo), after one that
+        clears both tiers' status words."""
+        self._clear(bufs, ("pool_status", "shell_status"), stream)
+        self._encode_pool(corpus, bufs, stream)
+        self._encode_shells(corpus, bufs, stream)
+
+    def _encode_pool(self, corpus, bufs, stream, max_workgroups: int = 0):
+        self.fib.encode_segments(corpus, self.pool.enc, bufs["pool_wire"], status=bufs["pool_status"], stream=stream,
+                                 max_workgroups=max_workgroups, status_cleared=True)
+
+    def _encode_shells(self, corpus, bufs, stream):
         self.turbo.encode_segments(corpus, self.shells.enc, bufs["shell_wire"], radii=self.radii,
-                                   status=bufs["shell_status"], stream=stream)
+                                   status=bufs["shell_status"], stream=stream, status_cleared=True)
+
+    def _clear(self, bufs, names, stream):
+        """The named status words in one launch: each call of a step would
+        otherwise clear its own in a launch before its kernel (1.4 us and a
+        launch gap each; three of a step's four are saved)."""
+        n = {"pool": len(self.pool.enc), "shell": len(self.shells.enc)}
+        self.ctx.clear_status([(bufs[k], n[k.split("_")[0]]) for k in names], stream)
 
     def decode(self, bufs, stream=None):
-        """Rehydrate the pool once and every shell: two launches."""
+        """Rehydrate the pool once and every shell: two launches, after one
+        that clears both tiers' status words."""
+        self._clear(bufs, ("pool_dstatus", "shell_dstatus"), stream)
         self.fib.decode_segments(bufs["pool_wire"], self.pool.dec, bufs["pool_out"],
-                                 status=bufs["pool_dstatus"], stream=stream)
+                                 status=bufs["pool_dstatus"], stream=stream, status_cleared=True)
         self.turbo.decode_segments(bufs["shell_wire"], self.shells.dec, bufs["shell_out"], radii=self.radii,
-                                   status=bufs["shell_dstatus"], stream=stream)
+                                   status=bufs["shell_dstatus"], stream=stream, status_cleared=True)
 
     def rehydrate(self, bufs, cache: DeviceKVCache, stream=None):
         """Decode the pool and every shell straight into `cache` -- prefix at
@@ -206,6 +223,8 @@ class TwoTierPlan:
         proveKV/scripts/ppl_validate_multi_agent.py:226-272) -- in the cache's
         dtype, once per cache copy: two launches.  Status words land in
         bufs["pool_cstatus"] / bufs["shell_cstatus"]."""
+        self._cache_tables(bufs, cache)
+        self._clear(bufs, ("pool_cstatus", "shell_cstatus"), stream)
         self._rehydrate_tier("pool", bufs, cache, stream)
         self._rehydrate_tier("shells", bufs, cache, stream)
 
@@ -223,18 +242,20 @@ class TwoTierPlan:
         done.  Without `side` the four launches run in order on `stream`."""
         import torch
         main = stream if stream is not None else torch.cuda.current_stream()
+        self._cache_tables(bufs, cache)
+        self._clear(bufs, ("pool_status", "shell_status", "pool_cstatus", "shell_cstatus"), main)
         if side is None:
-            self.encode(corpus, bufs, stream=main)
-            self.rehydrate(bufs, cache, stream=main)
+            self._encode_pool(corpus, bufs, main)
+            self._encode_shells(corpus, bufs, main)
+            self._rehydrate_tier("pool", bufs, cache, main)
+            self._rehydrate_tier("shells", bufs, cache, main)
             return
         shells_encoded, join = torch.cuda.Event(), torch.cuda.Event()
-        self.turbo.encode_segments(corpus, self.shells.enc, bufs["shell_wire"], radii=self.radii,
-                                   status=bufs["shell_status"], stream=main)
+        self._encode_shells(corpus, bufs, main)
         shells_encoded.record(main)
         side.wait_event(shells_encoded)
         self._rehydrate_tier("shells", bufs, cache, side, max_workgroups=side_workgroups)
-        self.fib.encode_segments(corpus, self.pool.enc, bufs["pool_wire"], status=bufs["pool_status"], stream=main,
-                                 max_workgroups=pool_workgroups)
+        self._encode_pool(corpus, bufs, main, max_workgroups=pool_workgroups)
         self._rehydrate_tier("pool", bufs, cache, main)
         join.record(side)
         main.wait_event(join)
@@ -261,16 +282,17 @@ class TwoTierPlan:
                 bufs[name] = torch.empty(2 * n, dtype=torch.int32, device=cache.buf.device)
 
     def _rehydrate_tier(self, tier: str, bufs, cache: DeviceKVCache, stream, max_workgroups: int = 0):
-        self._cache_tables(bufs, cache)
+        """One tier into `cache` (its status words cleared before)."""
         pseg, sseg = self._cache_segs
         out = cache.buf.view(-1)
         if tier == "pool":
             self.fib.decode_segments(bufs["pool_wire"], pseg, out, status=bufs["pool_cstatus"], stream=stream,
-                                     fanout=cache.copies, fanout_stride=cache.copy_stride)
+                                     fanout=cache.copies, fanout_stride=cache.copy_stride, status_cleared=True)
         else:
             self.turbo.decode_segments(bufs["shell_wire"], sseg, out, radii=self.radii,
                                        status=bufs["shell_cstatus"], stream=stream, fanout=cache.copies,
-                                       fanout_stride=cache.copy_stride, max_workgroups=max_workgroups)
+                                       fanout_stride=cache.copy_stride, max_workgroups=max_workgroups,
+                                       status_cleared=True)
             cache.mark_filled(self.tokens)
 
     def check_rehydrate(self, bufs):

@@ -1,0 +1,72 @@
+"""Status words cleared once for a step: failures of each of the step's calls are
+reported at the vector and segment they happened, on a second step over stale
+words too, on one stream and two, and the entry point refuses what it must."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from provekv_amd import _lib as L
+from provekv_amd import synth
+from provekv_amd.pool import DeviceKVCache, TwoTierPlan
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("two_streams", [False, True])
+def test_step_reports_after_one_clear(ctx, two_streams):
+    import torch
+    layers, heads, prefix, agents = 2, 3, 9, [4, 1]
+    plan = TwoTierPlan(ctx, layers, heads, 64, prefix, agents)
+    bufs = plan.alloc()
+    cache = DeviceKVCache(layers, heads, plan.tokens, 64)
+    side = torch.cuda.Stream() if two_streams else None
+    good = synth.corpus_tokens(7, layers, heads, plan.tokens, 64)
+    names = ("pool_status", "shell_status", "pool_cstatus", "shell_cstatus")
+
+    def step(x):
+        plan.build_and_rehydrate(torch.from_numpy(x.reshape(-1).copy()).cuda(), bufs, cache, side=side)
+        torch.cuda.synchronize()
+        return {k: bufs[k].cpu().numpy().view(np.uint32).reshape(-1, 2) for k in names}
+
+    for k, v in step(good).items():
+        assert (v == 0xFFFFFFFF).all(), k
+    bad = good.copy()
+    bad[3, 1, 2, 0, 5] = np.nan              # pool: token 3, layer 1, head 2, K
+    bad[prefix + 4, 0, 1, 1, 0] = np.inf     # agent 1's only token, layer 0, head 1, V
+    st = step(bad)
+    assert (st["pool_status"] != 0xFFFFFFFF).any(1).tolist() == [False, False, True, False]
+    assert st["pool_status"][2, 0] >> 4 == 3 * heads + 2
+    want = [False] * 8
+    want[4 + 1] = True                       # agent 1, layer 0, V
+    assert (st["shell_status"] != 0xFFFFFFFF).any(1).tolist() == want
+    assert st["shell_status"][5].min() >> 4 == 1
+    with pytest.raises(L.PkvError):
+        plan.check(bufs, decode=False)
+    for k, v in step(good).items():          # stale words are cleared again
+        assert (v == 0xFFFFFFFF).all(), k
+
+
+def test_clear_and_run_refusals(ctx):
+    import torch
+    prof = ctx.turbo_profile(64, 4, 32, 42)
+    st = torch.zeros(2, dtype=torch.int32, device="cuda")
+    with pytest.raises(L.PkvError):
+        ctx.clear_status([(st, 1)] * 9)
+    ctx.clear_status([(st, 1)] * 8)
+    assert (st.cpu() == -1).all()
+    x = torch.ones(64, device="cuda")
+    wire = torch.zeros(prof.blob_len(1), dtype=torch.uint8, device="cuda")
+    from provekv_amd.device import contiguous_segment, segments
+    segs = segments([contiguous_segment(0, 1, 64, 0)])
+    with pytest.raises(ValueError):
+        prof.encode_segments(x, segs, wire, status_cleared=True)
+
+    def run(flags, status, reserved=0):
+        op = L.SegmentsOp(1, 0, L.DT_F32, flags, x.data_ptr(), 64, segs.ctypes.data, wire.data_ptr(), wire.numel(),
+                          0, 1, 1, 0, reserved, status)
+        return L.lib().pkv_run_segments(ctx.ptr, prof.ptr, C.byref(op), None)
+    assert run(2, st.data_ptr()) == run(1, None) == run(0, st.data_ptr(), 1)
+    assert run(2, st.data_ptr()) != 0
+    assert run(0, st.data_ptr()) == 0 and run(1, st.data_ptr()) == 0 and run(0, None) == 0
+    torch.cuda.synchronize()
