@@ -596,6 +596,20 @@ int pkv_blake3_tier_digests(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_byt
                             uint32_t n, uint32_t layers, uint8_t* d_blob_digests, uint8_t* d_layer_digests,
                             void* stream);
 
+/* The digests of a whole build -- up to two tiers, as pkv_blake3_tier_digests
+ * for each -- by one launch sequence over the ranges of both. */
+typedef struct pkv_digest_tier {
+    const uint8_t* d_buf;
+    uint64_t buf_bytes;
+    const pkv_range* ranges;      /* 2 n: key then value per layer entry */
+    uint8_t* d_blob_digests;      /* 64 n bytes */
+    uint8_t* d_layer_digests;     /* 32 n bytes */
+    uint32_t n;
+    uint32_t reserved;            /* 0 */
+} pkv_digest_tier;
+int pkv_blake3_build_digests(pkv_ctx* ctx, const pkv_digest_tier* tiers, uint32_t n_tiers, uint32_t layers,
+                             void* stream);
+
 /* blake3 of host bytes, hashed on the context's device (copy in, the same
  * kernels, copy out, synchronise): blake3::hash over a host slice, as
  * CodecProfileDigest / ArtifactDigest::from_canonical_bytes and from_parts

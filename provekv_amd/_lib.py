@@ -53,7 +53,7 @@ EXPORTS = (
     "pkv_constants_cache_stats", "pkv_constants_cache_clear", "pkv_prepared_len", "pkv_turbo_prepare_queries",
     "pkv_turbo_score_segments", "pkv_score_status", "pkv_turbo_score_batch", "pkv_encode_diagnostics",
     "pkv_radii_log_bound", "pkv_fb2_n_blocks", "pkv_lloyd_refine", "pkv_blake3_ranges", "pkv_blake3_layer_digests",
-    "pkv_blake3_tier_digests", "pkv_blake3",
+    "pkv_blake3_tier_digests", "pkv_blake3_build_digests", "pkv_blake3",
     "pkv_host_angle_bins", "pkv_host_octant_bins", "pkv_host_logf",
     "pkv_host_expf", "pkv_host_expf_fused", "pkv_host_div255", "pkv_host_f32_stable_rel50", "pkv_code_from_json", "pkv_fib_digests", "pkv_host_blake3",
 )
@@ -69,6 +69,13 @@ class SegmentsOp(C.Structure):
 
 
 STATUS_CLEARED = 1
+
+
+class DigestTier(C.Structure):
+    """pkv_digest_tier"""
+    _fields_ = [("d_buf", C.c_void_p), ("buf_bytes", C.c_uint64), ("ranges", C.c_void_p),
+                ("d_blob_digests", C.c_void_p), ("d_layer_digests", C.c_void_p), ("n", C.c_uint32),
+                ("reserved", C.c_uint32)]
 
 
 class Seg(C.Structure):
@@ -190,6 +197,7 @@ def _declare(L):
         "pkv_blake3_ranges": ([P, P, U64, P, U32, P, P], I32),
         "pkv_blake3_layer_digests": ([P, P, U32, U32, P, P], I32),
         "pkv_blake3_tier_digests": ([P, P, U64, P, U32, U32, P, P, P], I32),
+        "pkv_blake3_build_digests": ([P, P, U32, U32, P], I32),
         "pkv_blake3": ([P, P, U64, P], I32),
         "pkv_host_angle_bins": ([P, P, U64, U32, P], None),
         "pkv_host_octant_bins": ([P, P, U64, P, P], None),

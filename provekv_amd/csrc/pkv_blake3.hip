@@ -176,6 +176,14 @@ __device__ __forceinline__ void quad_compress(uint32_t& cv_lo, uint32_t& cv_hi, 
     cv_hi = b ^ d;
 }
 
+// Range r's bytes and its digest's place.
+__device__ __forceinline__ const uint8_t* io_buf(const B3Io& io, uint32_t r) {
+    return r < io.split ? io.buf[0] : io.buf[1];
+}
+__device__ __forceinline__ uint32_t* io_out(const B3Io& io, uint64_t r) {
+    return r < io.split ? io.out[0] + 8ull * r : io.out[1] + 8ull * (r - io.split);
+}
+
 // A quad's block in LDS: 16 words at a pitch of 20, so that the 16 quads of a
 // wave reading the same word fall on 16 different banks.
 constexpr uint32_t QPITCH = 20;
@@ -185,10 +193,9 @@ constexpr uint32_t QPITCH = 20;
 // The first pass with one lane per chunk: one wave per tile of 64 chunks of
 // one range (pass table: B3Pass per range plus a sentinel whose tile_start
 // is the pass's tile count); the wave merges its 64 chaining values.
-__global__ __launch_bounds__(256) void blake3_tree_kernel(const uint8_t* __restrict__ buf,
-                                                          const B3Range* __restrict__ ranges,
+__global__ __launch_bounds__(256) void blake3_tree_kernel(B3Io io, const B3Range* __restrict__ ranges,
                                                           const B3Pass* __restrict__ pass, uint32_t nr,
-                                                          uint32_t* __restrict__ cv_out, uint32_t* __restrict__ out) {
+                                                          uint32_t* __restrict__ cv_out) {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t tile = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
     if (tile >= pass[nr].tile_start) return;
@@ -207,7 +214,7 @@ __global__ __launch_bounds__(256) void blake3_tree_kernel(const uint8_t* __restr
     uint32_t cv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     if (lane < nw) {
         const B3Range rg = ranges[r];
-        chunk_cv(buf + rg.offset, rg.len, first + lane, ps.count == 1u, cv);
+        chunk_cv(io_buf(io, r) + rg.offset, rg.len, first + lane, ps.count == 1u, cv);
     }
     // level s: elements are the lanes that are multiples of s, ceil(nw / s) of
     // them; even element e absorbs element e + 1 when it exists
@@ -220,7 +227,7 @@ __global__ __launch_bounds__(256) void blake3_tree_kernel(const uint8_t* __restr
             b3::parent(cv, o, root_group && c == 2u ? b3::ROOT : 0u);
     }
     if (lane == 0) {   // out is only 4-byte aligned
-        uint32_t* dst = root_group ? out + 8ull * r : cv_out + 8ull * (ps.out_base + g);
+        uint32_t* dst = root_group ? io_out(io, r) : cv_out + 8ull * (ps.out_base + g);
 #pragma unroll
         for (int i = 0; i < 8; ++i) dst[i] = cv[i];
     }
@@ -235,10 +242,9 @@ __global__ __launch_bounds__(256) void blake3_tree_kernel(const uint8_t* __restr
 // are read from LDS before its rounds: 14.4 Ki chunks 30 -> 22.8 us.  What is
 // left is the rounds' dependent chain, about 13 cycles per instruction at a wave
 // per SIMD.
-__global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restrict__ buf,
-                                                          const B3Range* __restrict__ ranges,
+__global__ __launch_bounds__(256) void blake3_quad_kernel(B3Io io, const B3Range* __restrict__ ranges,
                                                           const B3Pass* __restrict__ pass, uint32_t nr,
-                                                          uint32_t* __restrict__ cv_out, uint32_t* __restrict__ out) {
+                                                          uint32_t* __restrict__ cv_out) {
     __shared__ __align__(16) uint32_t blk_s[4][16][QPITCH];   // per wave, per quad: the current 64-byte block
     __shared__ uint32_t cv_s[4][16][8];                       // per wave, per quad: its chaining value
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
@@ -273,7 +279,7 @@ __global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restr
         // through the rest (quads past nq repeat chunk `first`, unused)
         const uint32_t nblk = clen == 0 ? 1u : (clen + 63u) / 64u;
         const uint32_t wblk = nq > 1u ? 16u : __builtin_amdgcn_readfirstlane(nblk);
-        const uint8_t* base = buf + rg.offset + start + 16u * i;   // this lane's 16 bytes of block 0
+        const uint8_t* base = io_buf(io, r) + rg.offset + start + 16u * i;   // this lane's 16 bytes of block 0
         const bool root = ps.count == 1u;
         // whole 16-byte pieces, at any byte alignment; zeros past the chunk
         auto load4 = [&](uint32_t b0, uint4 (&v)[4]) {
@@ -343,7 +349,7 @@ __global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restr
         wave_sync_lds();
     }
     if (quad == 0) {   // out is only 4-byte aligned
-        uint32_t* dst = root_group ? out + 8ull * r : cv_out + 8ull * (ps.out_base + g);
+        uint32_t* dst = root_group ? io_out(io, r) : cv_out + 8ull * (ps.out_base + g);
         dst[i] = cv_s[wave][0][i];
         dst[4u + i] = cv_s[wave][0][4u + i];
     }
@@ -357,9 +363,8 @@ __global__ __launch_bounds__(256) void blake3_quad_kernel(const uint8_t* __restr
 // aligned 16-value group is the first four levels).  A single lane per
 // compression leaves one wave per range chaining whole compressions, which is
 // most of a small wire's digest time.
-__global__ __launch_bounds__(256) void blake3_merge4_kernel(const B3Pass* __restrict__ pass, uint32_t nr,
-                                                            const uint32_t* __restrict__ cv_in,
-                                                            uint32_t* __restrict__ cv_out, uint32_t* __restrict__ out) {
+__global__ __launch_bounds__(256) void blake3_merge4_kernel(B3Io io, const B3Pass* __restrict__ pass, uint32_t nr,
+                                                            const uint32_t* cv_in, uint32_t* cv_out) {
     __shared__ uint32_t cv_s[4][16][8];   // per wave, per quad: a chaining value
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t quad = lane >> 2, i = lane & 3u;
@@ -427,7 +432,7 @@ __global__ __launch_bounds__(256) void blake3_merge4_kernel(const B3Pass* __rest
             merge(0, ng, root_group);
         }
         if (quad == 0) {   // out is only 4-byte aligned
-            uint32_t* dst = root_group ? out + 8ull * r : cv_out + 8ull * (ps.out_base + g);
+            uint32_t* dst = root_group ? io_out(io, r) : cv_out + 8ull * (ps.out_base + g);
             dst[i] = cv_s[0][0][i];
             dst[4u + i] = cv_s[0][0][4u + i];
         }
@@ -438,7 +443,7 @@ __global__ __launch_bounds__(256) void blake3_merge4_kernel(const B3Pass* __rest
 // layer entry, waves 0-3 on its key range and 4-7 on its value range.  A range
 // with values left (count > 0, at most 64 in a last pass) is merged as
 // blake3_merge4_kernel does; one that ended earlier (and every range when
-// `pass` is null) has its payload digest in `digests` already.  Then
+// `pass` is null) has its payload digest in place already.  Then
 // layer_out[i] = blake3 of serde_json's compact text of
 // json!({"layer_index", "key_digests": [k], "value_digests": [v]}) -- a
 // BTreeMap (serde_json without preserve_order), so the keys print sorted:
@@ -456,10 +461,9 @@ struct LayerText {
 };
 __constant__ LayerText c_layer_text = LayerText();
 
-__global__ __launch_bounds__(512) void blake3_layer_kernel(const B3Pass* __restrict__ pass,
-                                                           const uint32_t* __restrict__ cv_in, uint32_t* digests,
-                                                           uint32_t n, uint32_t layers,
-                                                           uint32_t* __restrict__ layer_out) {
+__global__ __launch_bounds__(512) void blake3_layer_kernel(B3Io io, const B3Pass* __restrict__ pass,
+                                                           const uint32_t* __restrict__ cv_in, uint32_t n,
+                                                           uint32_t layers) {
     __shared__ uint32_t cv_s[8][16][8];   // per wave, per quad: a chaining value
     __shared__ uint32_t dig_s[2][8];
     __shared__ uint32_t text_s[64];
@@ -516,7 +520,7 @@ __global__ __launch_bounds__(512) void blake3_layer_kernel(const B3Pass* __restr
                 merge(wave, ng, true);
             }
             if (lane < 8u) {
-                uint32_t* dst = digests + 8ull * r;   // only 4-byte aligned
+                uint32_t* dst = io_out(io, r);   // only 4-byte aligned
                 uint32_t v;
                 if (nw) {
                     v = cv_s[wave][0][lane];
@@ -529,7 +533,9 @@ __global__ __launch_bounds__(512) void blake3_layer_kernel(const B3Pass* __restr
         }
         __syncthreads();
         if (wave == 0) {
-            const uint32_t li = entry % layers;
+            const bool second = entry >= io.split / 2u;   // an entry of the second buffer
+            const uint32_t local = second ? entry - static_cast<uint32_t>(io.split / 2u) : entry;
+            const uint32_t li = local % layers;
             uint32_t nd = 1, top = 1;   // decimal digits of li, 10^(nd - 1)
             for (uint32_t v = li; v >= 10u; v /= 10u) {
                 ++nd;
@@ -571,7 +577,7 @@ __global__ __launch_bounds__(512) void blake3_layer_kernel(const B3Pass* __restr
                               b == nblk - 1 ? len - 64u * b : 64u, flags);
             }
             if (quad == 0) {
-                uint32_t* dst = layer_out + 8ull * entry;
+                uint32_t* dst = (second ? io.layer[1] : io.layer[0]) + 8ull * local;
                 dst[i] = cv_lo;
                 dst[4u + i] = cv_hi;
             }
@@ -580,36 +586,35 @@ __global__ __launch_bounds__(512) void blake3_layer_kernel(const B3Pass* __restr
     }
 }
 
-int launch_blake3_pass(const uint8_t* buf, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
-                       uint32_t* cv_out, uint32_t* out, void* stream) {
+int launch_blake3_pass(const B3Io& io, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
+                       uint32_t* cv_out, void* stream) {
     if (tiles == 0) return hipSuccess;
-    const uint32_t grid = (tiles + 3u) / 4u;
-    hipLaunchKernelGGL(blake3_tree_kernel, dim3(grid), dim3(256), 0, static_cast<hipStream_t>(stream), buf, ranges,
-                       pass, nr, cv_out, out);
+    hipLaunchKernelGGL(blake3_tree_kernel, dim3((tiles + 3u) / 4u), dim3(256), 0, static_cast<hipStream_t>(stream), io,
+                       ranges, pass, nr, cv_out);
     return hipGetLastError();
 }
 
-int launch_blake3_quad(const uint8_t* buf, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
-                       uint32_t* cv_out, uint32_t* out, void* stream) {
+int launch_blake3_quad(const B3Io& io, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
+                       uint32_t* cv_out, void* stream) {
     if (tiles == 0) return hipSuccess;
-    hipLaunchKernelGGL(blake3_quad_kernel, dim3((tiles + 3u) / 4u), dim3(256), 0, static_cast<hipStream_t>(stream), buf,
-                       ranges, pass, nr, cv_out, out);
+    hipLaunchKernelGGL(blake3_quad_kernel, dim3((tiles + 3u) / 4u), dim3(256), 0, static_cast<hipStream_t>(stream), io,
+                       ranges, pass, nr, cv_out);
     return hipGetLastError();
 }
 
-int launch_blake3_merge4(const B3Pass* pass, uint32_t nr, uint32_t tiles, const uint32_t* cv_in, uint32_t* cv_out,
-                         uint32_t* out, void* stream) {
+int launch_blake3_merge4(const B3Io& io, const B3Pass* pass, uint32_t nr, uint32_t tiles, const uint32_t* cv_in,
+                         uint32_t* cv_out, void* stream) {
     if (tiles == 0) return hipSuccess;
-    hipLaunchKernelGGL(blake3_merge4_kernel, dim3(tiles), dim3(256), 0, static_cast<hipStream_t>(stream), pass, nr,
-                       cv_in, cv_out, out);
+    hipLaunchKernelGGL(blake3_merge4_kernel, dim3(tiles), dim3(256), 0, static_cast<hipStream_t>(stream), io, pass, nr,
+                       cv_in, cv_out);
     return hipGetLastError();
 }
 
-int launch_blake3_layers(const B3Pass* pass, const uint32_t* cv_in, uint32_t* digests, uint32_t n, uint32_t layers,
-                         uint32_t* out, void* stream) {
+int launch_blake3_layers(const B3Io& io, const B3Pass* pass, const uint32_t* cv_in, uint32_t n, uint32_t layers,
+                         void* stream) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(blake3_layer_kernel, dim3(n < (1u << 20) ? n : 1u << 20), dim3(512), 0,
-                       static_cast<hipStream_t>(stream), pass, cv_in, digests, n, layers, out);
+                       static_cast<hipStream_t>(stream), io, pass, cv_in, n, layers);
     return hipGetLastError();
 }
 

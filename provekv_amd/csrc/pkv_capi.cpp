@@ -77,7 +77,11 @@ struct Slot {
     hipEvent_t done_ev = nullptr;  // private slot: recorded after the launches of the call that took it
     bool done_recorded = false;
     bool shared = false;         // table only (no status words): reusable by equal tables
-    bool digest = false;         // a pkv_blake3_ranges table (+ its chaining-value scratch)
+    bool digest = false;         // a table of digest ranges (+ its chaining-value scratch), and its plan:
+    std::vector<uint32_t> b3_tiles;   // tiles per pass
+    bool b3_quad = false;             // pass 0 on four lanes per chunk
+    uint64_t b3_end[2] = {0, 0};      // last byte (exclusive) the ranges need of each buffer
+    uint64_t b3_split = 0;
     uint32_t nseg = 0;
     uint64_t hash = 0;
 };
@@ -272,9 +276,8 @@ int validate_segments(const pkv_profile* p, int radii, bool encode, int dtype, c
     if (reinterpret_cast<uintptr_t>(d_f32) % 16 != 0) return PKV_ERR_INVALID_ARG;
     const uint32_t plen = p->kind == PKV_CODEC_TURBO ? turbo_plen(p, radii) : fib_plen(p);
     const uint32_t hdr = hdr_len(p);
-    std::vector<std::pair<uint64_t, uint64_t>> blobs;   // encode only
-    if (encode) blobs.reserve(nseg);
-    uint64_t total = 0;
+    uint64_t total = 0, prev_end = 0;
+    bool in_order = true;   // every blob starts at or after the end of the one before it
     for (uint32_t i = 0; i < nseg; ++i) {
         const pkv_seg& s = segs[i];
         if (s.group == 0) return PKV_ERR_INVALID_ARG;
@@ -288,7 +291,8 @@ int validate_segments(const pkv_profile* p, int radii, bool encode, int dtype, c
         if (!mul_add_ok(s.n_vectors, plen, hdr, &blob_end) ||
             __builtin_add_overflow(blob_end, s.wire_offset, &blob_end) || blob_end > wire_bytes)
             return PKV_ERR_CAPACITY;
-        if (encode) blobs.emplace_back(s.wire_offset, blob_end);
+        in_order &= s.wire_offset >= prev_end;
+        prev_end = blob_end;
         uint64_t tiles = (static_cast<uint64_t>(s.n_vectors) + TILE - 1) / TILE;
         if (tiles == 0) tiles = 1;   // an empty blob still gets its header checked
         tile_start[i] = static_cast<uint32_t>(total);
@@ -296,7 +300,10 @@ int validate_segments(const pkv_profile* p, int radii, bool encode, int dtype, c
         if (total > 0x7fffffffull) return PKV_ERR_INVALID_ARG;
     }
     tile_start[nseg] = static_cast<uint32_t>(total);
-    if (encode) {   // encoded blobs are written by different workgroups: no overlap
+    if (encode && !in_order) {   // encoded blobs are written by different workgroups: no overlap
+        std::vector<std::pair<uint64_t, uint64_t>> blobs(nseg);
+        for (uint32_t i = 0; i < nseg; ++i)
+            blobs[i] = {segs[i].wire_offset, segs[i].wire_offset + hdr + static_cast<uint64_t>(segs[i].n_vectors) * plen};
         std::sort(blobs.begin(), blobs.end());
         for (size_t i = 1; i < blobs.size(); ++i)
             if (blobs[i].first < blobs[i - 1].second) return PKV_ERR_INVALID_ARG;
@@ -304,11 +311,28 @@ int validate_segments(const pkv_profile* p, int radii, bool encode, int dtype, c
     return PKV_OK;
 }
 
-uint64_t fnv1a(const void* p, size_t n) {
+// Hash of a table of 8-byte words (n a multiple of 8), four words a step: the
+// byte-wise hash before it was most of a call's host time at a few hundred
+// segments.  Equal hashes are confirmed by a comparison of the tables.
+uint64_t table_hash(const void* p, size_t n) {
+    constexpr uint64_t kMul = 0x9e3779b97f4a7c15ull;
     const auto* b = static_cast<const uint8_t*>(p);
-    uint64_t h = 1469598103934665603ull;
-    for (size_t i = 0; i < n; ++i) h = (h ^ b[i]) * 1099511628211ull;
-    return h;
+    uint64_t h[4] = {n, 1, 2, 3};
+    size_t i = 0;
+    for (; i + 32 <= n; i += 32)
+        for (int k = 0; k < 4; ++k) {
+            uint64_t w;
+            std::memcpy(&w, b + i + 8 * k, 8);
+            h[k] = (h[k] ^ w) * kMul;
+            h[k] ^= h[k] >> 29;
+        }
+    for (; i + 8 <= n; i += 8) {
+        uint64_t w;
+        std::memcpy(&w, b + i, 8);
+        h[0] = (h[0] ^ w) * kMul;
+        h[0] ^= h[0] >> 29;
+    }
+    return ((h[0] * kMul ^ h[1]) * kMul ^ h[2]) * kMul ^ h[3];
 }
 
 // Takes the next ring slot for `total` bytes (device table + pinned staging),
@@ -369,7 +393,7 @@ int stage_table(pkv_ctx* ctx, const pkv_seg* segs, uint32_t nseg, const std::vec
     const size_t map_bytes = with_map ? sizeof(uint32_t) * ntiles : 0;
     const size_t stat_off = (map_off + map_bytes + 255) & ~static_cast<size_t>(255);
     const size_t total = stat_off + (need_status ? sizeof(uint32_t) * 2 * nseg : 0) + 256;
-    const uint64_t hash = fnv1a(segs, seg_bytes);
+    const uint64_t hash = table_hash(segs, seg_bytes);
     if (!need_status) {
         for (Slot& c : ctx->slots) {
             if (c.shared && c.nseg == nseg && c.hash == hash && std::memcmp(c.host, segs, seg_bytes) == 0) {
@@ -1428,6 +1452,7 @@ struct B3Plan {
     std::vector<uint32_t> tiles;    // per pass
     uint64_t cvs = 0;               // chaining values written by passes that do not finish a range
     bool quad = false;              // pass 0 on four lanes per chunk (16-chunk tiles)
+    uint64_t end[2] = {0, 0};       // last byte (exclusive) the ranges need of each buffer
 };
 
 // Chunks below which pass 0 puts four lanes on a chunk (16 chunks per wave,
@@ -1437,12 +1462,16 @@ struct B3Plan {
 // shells, 48 Ki chunks, 51 / 50 us; 64 Ki chunks 50 / 61 us.
 constexpr uint64_t kB3QuadBelow = 32ull * 1024;
 
-int plan_blake3(const pkv_range* ranges, uint32_t nr, uint64_t buf_bytes, B3Plan* plan) {
+// Ranges r < split lie in the first buffer, the others in the second.
+int plan_blake3(const pkv_range* ranges, uint32_t nr, uint64_t split, const uint64_t (&buf_bytes)[2], B3Plan* plan) {
     std::vector<uint64_t> count(nr), in_base(nr, 0);
     uint64_t total = 0;
     for (uint32_t r = 0; r < nr; ++r) {
         const pkv_range& g = ranges[r];
-        if (g.offset > buf_bytes || g.len > buf_bytes - g.offset) return PKV_ERR_INVALID_ARG;
+        const uint64_t bytes = buf_bytes[r < split ? 0 : 1];
+        if (g.offset > bytes || g.len > bytes - g.offset) return PKV_ERR_INVALID_ARG;
+        uint64_t& end = plan->end[r < split ? 0 : 1];
+        end = std::max(end, g.offset + g.len);
         count[r] = b3::chunks_of(g.len);
         if (count[r] > 0xFFFFFFFFull) return PKV_ERR_INVALID_ARG;
         total += count[r];
@@ -1479,34 +1508,33 @@ int plan_blake3(const pkv_range* ranges, uint32_t nr, uint64_t buf_bytes, B3Plan
     return PKV_OK;
 }
 
-// Caller holds ctx->mu and has made the device current.  With d_layers (nr
-// even: key and value ranges in turn) the last pass also forms the nr / 2
-// layer digests.
-int blake3_ranges_locked(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_bytes, const pkv_range* ranges,
-                         uint32_t nr, uint8_t* d_out, hipStream_t stream, uint8_t* d_layers = nullptr,
-                         uint32_t layers = 0) {
-    B3Plan plan;
-    int rc = plan_blake3(ranges, nr, buf_bytes, &plan);
-    if (rc) return rc;
+// Caller holds ctx->mu and has made the device current.  n_layers != 0 (nr =
+// 2 n_layers, io.split even): the last pass also forms the layer digests.
+int blake3_ranges_locked(pkv_ctx* ctx, const B3Io& io, const uint64_t (&buf_bytes)[2], const pkv_range* ranges,
+                         uint32_t nr, hipStream_t stream, uint32_t n_layers = 0, uint32_t layers = 0) {
     const size_t range_bytes = sizeof(pkv_range) * nr;
     const size_t pass_off = (range_bytes + 255) & ~static_cast<size_t>(255);
-    const size_t pass_bytes = sizeof(B3Pass) * plan.passes.size();
-    const size_t cv_off = (pass_off + pass_bytes + 255) & ~static_cast<size_t>(255);
-    const size_t total = cv_off + 32 * plan.cvs + 256;
-    const uint64_t hash = fnv1a(ranges, range_bytes);
+    const uint64_t hash = table_hash(ranges, range_bytes);
     // The same table again on the same stream (a serving loop's digest of
-    // every step) reuses its slot as is: no upload, and the chaining-value
-    // scratch is rewritten only after the previous call, in stream order.
+    // every step) reuses its slot and plan as they are: no upload, and the
+    // chaining-value scratch is rewritten only after the previous call, in
+    // stream order.
     Slot* sl = nullptr;
     for (Slot& c : ctx->slots)
-        if (c.digest && c.nseg == nr && c.hash == hash && c.users.n == 1 && !c.users.overflow &&
-            c.users.s[0] == stream && std::memcmp(c.host, ranges, range_bytes) == 0) {
+        if (c.digest && c.nseg == nr && c.hash == hash && c.b3_split == io.split && c.users.n == 1 &&
+            !c.users.overflow && c.users.s[0] == stream && c.b3_end[0] <= buf_bytes[0] &&
+            c.b3_end[1] <= buf_bytes[1] && std::memcmp(c.host, ranges, range_bytes) == 0) {
             sl = &c;
             break;
         }
     hipError_t cp = hipSuccess;
     if (!sl) {
-        rc = acquire_slot(ctx, total, &sl);
+        B3Plan plan;
+        int rc = plan_blake3(ranges, nr, io.split, buf_bytes, &plan);
+        if (rc) return rc;
+        const size_t pass_bytes = sizeof(B3Pass) * plan.passes.size();
+        const size_t cv_off = (pass_off + pass_bytes + 255) & ~static_cast<size_t>(255);
+        rc = acquire_slot(ctx, cv_off + 32 * plan.cvs + 256, &sl);
         if (rc) return rc;
         auto* h = static_cast<uint8_t*>(sl->host);
         std::memcpy(h, ranges, range_bytes);
@@ -1516,28 +1544,41 @@ int blake3_ranges_locked(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_bytes,
         sl->digest = cp == hipSuccess;
         sl->nseg = nr;
         sl->hash = hash;
+        sl->b3_tiles = std::move(plan.tiles);
+        sl->b3_quad = plan.quad;
+        sl->b3_end[0] = plan.end[0];
+        sl->b3_end[1] = plan.end[1];
+        sl->b3_split = io.split;
     }
+    const size_t np = sl->b3_tiles.size();
+    const size_t cv_off = (pass_off + sizeof(B3Pass) * np * (nr + 1) + 255) & ~static_cast<size_t>(255);
     auto* d = static_cast<uint8_t*>(sl->dev);
     auto* d_ranges = reinterpret_cast<const B3Range*>(d);
     auto* d_cv = reinterpret_cast<uint32_t*>(d + cv_off);
-    auto* out = reinterpret_cast<uint32_t*>(d_out);
+    auto d_pass = [&](size_t p) { return reinterpret_cast<const B3Pass*>(d + pass_off) + p * (nr + 1); };
     int e = cp;
-    for (size_t p = 0; p < plan.tiles.size() && !e; ++p) {
-        const auto* d_pass = reinterpret_cast<const B3Pass*>(d + pass_off) + p * (nr + 1);
+    for (size_t p = 0; p < np && !e; ++p) {
+        const uint32_t tiles = sl->b3_tiles[p];
         if (p == 0)
-            e = plan.quad ? launch_blake3_quad(d_buf, d_ranges, d_pass, nr, plan.tiles[p], d_cv, out, stream)
-                          : launch_blake3_pass(d_buf, d_ranges, d_pass, nr, plan.tiles[p], d_cv, out, stream);
-        else if (!d_layers || p + 1 < plan.tiles.size())
-            e = launch_blake3_merge4(d_pass, nr, plan.tiles[p], d_cv, d_cv, out, stream);
+            e = sl->b3_quad ? launch_blake3_quad(io, d_ranges, d_pass(0), nr, tiles, d_cv, stream)
+                            : launch_blake3_pass(io, d_ranges, d_pass(0), nr, tiles, d_cv, stream);
+        else if (!n_layers || p + 1 < np)
+            e = launch_blake3_merge4(io, d_pass(p), nr, tiles, d_cv, d_cv, stream);
     }
-    if (d_layers && !e) {
-        const size_t last = plan.tiles.size() - 1;   // a single pass ended every range itself
-        const auto* d_pass = last ? reinterpret_cast<const B3Pass*>(d + pass_off) + last * (nr + 1) : nullptr;
-        e = launch_blake3_layers(d_pass, d_cv, out, nr / 2, layers, reinterpret_cast<uint32_t*>(d_layers), stream);
-    }
+    if (n_layers && !e)   // a single pass ended every range itself
+        e = launch_blake3_layers(io, np > 1 ? d_pass(np - 1) : nullptr, d_cv, n_layers, layers, stream);
     const int rc2 = finish_slot(sl, stream);
     if (e) return hip_status(static_cast<hipError_t>(e));
     return rc2;
+}
+
+// One buffer of nr ranges, its digests at d_out.
+B3Io one_buffer(const uint8_t* d_buf, uint64_t nr, uint8_t* d_out) {
+    B3Io io{};
+    io.buf[0] = d_buf;
+    io.out[0] = reinterpret_cast<uint32_t*>(d_out);
+    io.split = nr;
+    return io;
 }
 
 }  // namespace
@@ -1550,7 +1591,8 @@ int pkv_blake3_ranges(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_bytes, co
         return PKV_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
-    return blake3_ranges_locked(ctx, d_buf, buf_bytes, ranges, n, d_out, static_cast<hipStream_t>(stream));
+    return blake3_ranges_locked(ctx, one_buffer(d_buf, n, d_out), {buf_bytes, 0}, ranges, n,
+                                static_cast<hipStream_t>(stream));
 }
 
 int pkv_blake3_layer_digests(pkv_ctx* ctx, const uint8_t* d_kv_digests, uint32_t n, uint32_t layers, uint8_t* d_out,
@@ -1562,9 +1604,10 @@ int pkv_blake3_layer_digests(pkv_ctx* ctx, const uint8_t* d_kv_digests, uint32_t
         return PKV_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lock(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
-    const int e = launch_blake3_layers(nullptr, nullptr,
-                                       reinterpret_cast<uint32_t*>(const_cast<uint8_t*>(d_kv_digests)), n, layers,
-                                       reinterpret_cast<uint32_t*>(d_out), stream);   // reads the digests only
+    // no range is left to hash: the payload digests are only read
+    B3Io io = one_buffer(nullptr, 2ull * n, const_cast<uint8_t*>(d_kv_digests));
+    io.layer[0] = reinterpret_cast<uint32_t*>(d_out);
+    const int e = launch_blake3_layers(io, nullptr, nullptr, n, layers, stream);
     return e ? hip_status(static_cast<hipError_t>(e)) : PKV_OK;
 }
 
@@ -1573,13 +1616,45 @@ int pkv_blake3_tier_digests(pkv_ctx* ctx, const uint8_t* d_buf, uint64_t buf_byt
                             void* stream) {
     if (!ctx || layers == 0) return PKV_ERR_INVALID_ARG;
     if (n == 0) return PKV_OK;
-    if (n > 0x7FFFFFFFu || !ranges || !d_blob_digests || !d_layer_digests || (!d_buf && buf_bytes) ||
-        reinterpret_cast<uintptr_t>(d_blob_digests) % 4 || reinterpret_cast<uintptr_t>(d_layer_digests) % 4)
-        return PKV_ERR_INVALID_ARG;
+    const pkv_digest_tier tier{d_buf, buf_bytes, ranges, d_blob_digests, d_layer_digests, n, 0};
+    return pkv_blake3_build_digests(ctx, &tier, 1, layers, stream);
+}
+
+int pkv_blake3_build_digests(pkv_ctx* ctx, const pkv_digest_tier* tiers, uint32_t n_tiers, uint32_t layers,
+                             void* stream) {
+    if (!ctx || layers == 0 || n_tiers > 2 || (n_tiers && !tiers)) return PKV_ERR_INVALID_ARG;
+    B3Io io{};
+    uint64_t bytes[2] = {0, 0}, total = 0;
+    const pkv_range* ranges = nullptr;
+    uint32_t used = 0;
+    for (uint32_t k = 0; k < n_tiers; ++k) {
+        const pkv_digest_tier& t = tiers[k];
+        if (t.n == 0) continue;
+        if (t.n > 0x7FFFFFFFu || !t.ranges || !t.d_blob_digests || !t.d_layer_digests || (!t.d_buf && t.buf_bytes) ||
+            reinterpret_cast<uintptr_t>(t.d_blob_digests) % 4 || reinterpret_cast<uintptr_t>(t.d_layer_digests) % 4)
+            return PKV_ERR_INVALID_ARG;
+        io.buf[used] = t.d_buf;
+        io.out[used] = reinterpret_cast<uint32_t*>(t.d_blob_digests);
+        io.layer[used] = reinterpret_cast<uint32_t*>(t.d_layer_digests);
+        bytes[used] = t.buf_bytes;
+        if (used == 0) io.split = 2ull * t.n;
+        ranges = t.ranges;
+        total += t.n;
+        ++used;
+    }
+    if (used == 0) return PKV_OK;
+    if (total > 0x7FFFFFFFu) return PKV_ERR_INVALID_ARG;
+    std::vector<pkv_range> both;
+    if (used == 2) {   // the second tier's ranges after the first's
+        both.reserve(2 * total);
+        both.insert(both.end(), tiers[0].ranges, tiers[0].ranges + 2ull * tiers[0].n);
+        both.insert(both.end(), tiers[1].ranges, tiers[1].ranges + 2ull * tiers[1].n);
+        ranges = both.data();
+    }
     std::lock_guard<std::mutex> lock(ctx->mu);
     HIP_TRY(hipSetDevice(ctx->device));
-    return blake3_ranges_locked(ctx, d_buf, buf_bytes, ranges, 2 * n, d_blob_digests, static_cast<hipStream_t>(stream),
-                                d_layer_digests, layers);
+    return blake3_ranges_locked(ctx, io, bytes, ranges, static_cast<uint32_t>(2 * total),
+                                static_cast<hipStream_t>(stream), static_cast<uint32_t>(total), layers);
 }
 
 int pkv_blake3(pkv_ctx* ctx, const void* data, uint64_t len, uint8_t out[32]) {
@@ -1594,7 +1669,7 @@ int pkv_blake3(pkv_ctx* ctx, const void* data, uint64_t len, uint8_t out[32]) {
     hipStream_t st = ctx->own_stream;
     if (len) HIP_TRY(hipMemcpyAsync(d_in, data, len, hipMemcpyHostToDevice, st));
     const pkv_range rg{0, len};
-    rc = blake3_ranges_locked(ctx, d_in, len, &rg, 1, d_hash, st);
+    rc = blake3_ranges_locked(ctx, one_buffer(d_in, 1, d_hash), {len, 0}, &rg, 1, st);
     if (rc) { (void)hipStreamSynchronize(st); return rc; }
     HIP_TRY(hipMemcpyAsync(out, d_hash, 32, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));

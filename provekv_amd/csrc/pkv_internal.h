@@ -232,19 +232,30 @@ static_assert(sizeof(B3Range) == sizeof(pkv_range), "range layout");
 struct B3Pass {
     uint32_t tile_start, count, in_base, out_base;
 };
+// What a digest call reads and writes: ranges r < split are ranges of buf[0]
+// with digests at out[0] + 8r, the others of buf[1] at out[1] + 8(r - split)
+// (one buffer: split = the number of ranges).  With layer digests split is even,
+// entry e is ranges 2e, 2e + 1, and entries from split / 2 on count from
+// layer[1].
+struct B3Io {
+    const uint8_t* buf[2];
+    uint32_t* out[2];
+    uint32_t* layer[2];
+    uint64_t split;
+};
 // Pass 0 with one lane per chunk (tiles of 64 chunks).
-int launch_blake3_pass(const uint8_t* buf, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
-                       uint32_t* cv_out, uint32_t* out, void* stream);
+int launch_blake3_pass(const B3Io& io, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
+                       uint32_t* cv_out, void* stream);
 // Pass 0 with four lanes per chunk (tiles of 16 chunks; pass records as for
 // launch_blake3_pass).
-int launch_blake3_quad(const uint8_t* buf, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
-                       uint32_t* cv_out, uint32_t* out, void* stream);
+int launch_blake3_quad(const B3Io& io, const B3Range* ranges, const B3Pass* pass, uint32_t nr, uint32_t tiles,
+                       uint32_t* cv_out, void* stream);
 // A merge pass (tiles of 64 chaining values) with four lanes per
 // compression, one workgroup per tile.
-int launch_blake3_merge4(const B3Pass* pass, uint32_t nr, uint32_t tiles, const uint32_t* cv_in, uint32_t* cv_out,
-                         uint32_t* out, void* stream);
-// A tier's last pass (null: every range of it has ended) and its n layer digests.
-int launch_blake3_layers(const B3Pass* pass, const uint32_t* cv_in, uint32_t* digests, uint32_t n, uint32_t layers,
-                         uint32_t* out, void* stream);
+int launch_blake3_merge4(const B3Io& io, const B3Pass* pass, uint32_t nr, uint32_t tiles, const uint32_t* cv_in,
+                         uint32_t* cv_out, void* stream);
+// The last pass (null: every range has ended) and the n layer digests.
+int launch_blake3_layers(const B3Io& io, const B3Pass* pass, const uint32_t* cv_in, uint32_t n, uint32_t layers,
+                         void* stream);
 
 }  // namespace pkv

@@ -3774,6 +3774,7 @@ constexpr size_t stage_bytes() {
 // Dynamic LDS above 64 KiB must be allowed per kernel before launch.
 template <typename K>
 hipError_t allow_lds(K kernel, size_t bytes) {
+    if (bytes <= 64 * 1024) return hipSuccess;
     return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                static_cast<int>(bytes));
 }

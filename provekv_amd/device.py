@@ -40,8 +40,11 @@ def _torch():
 
 
 def _stream_ptr(stream):
-    torch = _torch()
     if stream is None:
+        torch = _torch()
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:   # the handle alone: building a Stream object costs as much as a kernel launch
+            return C.c_void_p(raw(torch.cuda.current_device()))
         stream = torch.cuda.current_stream()
     return C.c_void_p(stream.cuda_stream)
 
@@ -134,17 +137,28 @@ class Context:
         of its 2 n blobs (rows of `ranges`, key then value per entry) into
         `blob_out` [n, 2, 32] and the layer digests into `layer_out` [n, 32],
         one call for what blake3_ranges and layer_digests do in two."""
+        self.build_digests([(buf, ranges, blob_out, layer_out)], layers, stream)
+
+    def build_digests(self, tiers, layers: int, stream=None) -> None:
+        """The digests of up to two tiers in one launch sequence
+        (pkv_blake3_build_digests): rows of (buf, ranges, blob_out, layer_out)
+        as tier_digests takes them."""
         torch = _torch()
-        rg = np.ascontiguousarray(np.asarray(ranges, dtype=np.uint64).reshape(-1, 2))
-        if len(rg) % 2:
-            raise ValueError("ranges come in key / value pairs")
-        n = len(rg) // 2
-        for t, need in ((buf, 0), (blob_out, 64 * n), (layer_out, 32 * n)):
-            if t.dtype != torch.uint8 or not t.is_contiguous() or t.numel() < need:
-                raise ValueError("buf, blob_out and layer_out must be contiguous uint8 tensors of the needed size")
-        rc = L.lib().pkv_blake3_tier_digests(self.ptr, buf.data_ptr(), buf.numel(), rg.ctypes.data, n, layers,
-                                             blob_out.data_ptr(), layer_out.data_ptr(), _stream_ptr(stream))
-        L.check(rc, "pkv_blake3_tier_digests")
+        ops = (L.DigestTier * len(tiers))()
+        keep = []   # the range arrays live until the call returns
+        for op, (buf, ranges, blob_out, layer_out) in zip(ops, tiers):
+            rg = np.ascontiguousarray(np.asarray(ranges, dtype=np.uint64).reshape(-1, 2))
+            if len(rg) % 2:
+                raise ValueError("ranges come in key / value pairs")
+            n = len(rg) // 2
+            for t, need in ((buf, 0), (blob_out, 64 * n), (layer_out, 32 * n)):
+                if t.dtype != torch.uint8 or not t.is_contiguous() or t.numel() < need:
+                    raise ValueError("buf, blob_out and layer_out must be contiguous uint8 tensors of the needed size")
+            keep.append(rg)
+            op.d_buf, op.buf_bytes, op.ranges, op.n = buf.data_ptr(), buf.numel(), rg.ctypes.data, n
+            op.d_blob_digests, op.d_layer_digests = blob_out.data_ptr(), layer_out.data_ptr()
+        L.check(L.lib().pkv_blake3_build_digests(self.ptr, ops, len(tiers), layers, _stream_ptr(stream)),
+                "pkv_blake3_build_digests")
 
     def blake3(self, data: bytes) -> bytes:
         """blake3::hash of host bytes, computed on this device."""

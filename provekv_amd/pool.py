@@ -322,21 +322,22 @@ class TwoTierPlan:
         proveKV/src/codec.rs:85-95; key then value), and
         bufs["pool_layer_digests"] / bufs["shell_layer_digests"]
         [owners * layers, 32] every layer's block_digest (PoolLayer /
-        ShellLayer::compute_digest, pool.rs:83-103, shell.rs:48-66).  Four
-        launches per tier at most (payload passes, then the layer digests), one
-        library call per tier.
-        With a `side` stream the shell tier runs there, concurrently with the
-        pool tier (each tier alone leaves most of the GPU idle); the calling
-        stream waits for both."""
+        ShellLayer::compute_digest, pool.rs:83-103, shell.rs:48-66).  One
+        library call and one launch sequence for both tiers (payload passes,
+        the last of them with the layer digests), on the calling stream: tiers
+        apart on two streams spent longer on the two cross-stream waits than
+        they saved.  Work queued on a `side` stream before the call comes
+        before the digests."""
         import torch
         main = stream if stream is not None else torch.cuda.current_stream()
-        if side is not None:   # two events kept for every call (creating them is most of a wait's cost)
-            evs = getattr(self, "_digest_events", None)
-            if evs is None:
-                evs = self._digest_events = (torch.cuda.Event(), torch.cuda.Event())
-            evs[0].record(main)
-            side.wait_event(evs[0])
-        for tier, name, st in ((self.pool, "pool", main), (self.shells, "shell", side or main)):
+        if side is not None:
+            if torch.cuda.is_current_stream_capturing():   # side may join a capture only by a fork from it
+                side.wait_stream(main)
+                main.wait_stream(side)
+            elif not side.query():
+                main.wait_stream(side)
+        tiers = []
+        for tier, name in ((self.pool, "pool"), (self.shells, "shell")):
             n = len(tier.blob_offsets) // 2
             if f"{name}_digests" not in bufs:
                 dev = bufs[f"{name}_wire"].device
@@ -345,11 +346,8 @@ class TwoTierPlan:
             ranges = getattr(tier, "ranges", None)
             if ranges is None:
                 ranges = tier.ranges = np.array([(off, ln) for _, _, _, off, ln in tier.blob_offsets], np.uint64)
-            self.ctx.tier_digests(bufs[f"{name}_wire"], ranges, self.layers, bufs[f"{name}_digests"],
-                                  bufs[f"{name}_layer_digests"], stream=st)
-        if side is not None:
-            evs[1].record(side)
-            main.wait_event(evs[1])
+            tiers.append((bufs[f"{name}_wire"], ranges, bufs[f"{name}_digests"], bufs[f"{name}_layer_digests"]))
+        self.ctx.build_digests(tiers, self.layers, main)
 
     def digest_report(self, bufs) -> dict:
         """The digests of the last digests() call as the reference prints them

@@ -60,3 +60,66 @@ def test_tier_layer_digests(ctx, layers, big):
     got = ctx.layer_digests(kv.view(1234, 2, 32), 100000).cpu().numpy()
     for i in (0, 9, 10, 99, 100, 999, 1000, 1233):
         assert bytes(got[i]) == O.layer_digest(i, ref[0].tobytes(), ref[1].tobytes())
+
+
+@pytest.mark.parametrize("na,nb", [(4, 0), (0, 3), (5, 7), (1, 200)])
+@pytest.mark.parametrize("side", [False, True])
+def test_build_digests_two_buffers(ctx, na, nb, side):
+    """Both tiers of a build by one launch sequence, from two buffers of their own,
+    repeated on other bytes and after work queued on a side stream."""
+    import torch
+    rng = np.random.RandomState(na + nb)
+    bufs, tiers, refs = [], [], []
+    for n, size in ((na, 70000), (nb, 20000)):
+        rg = np.array([(k * size + k % 3, int(rng.randint(0, size - 3))) for k in range(2 * n)],
+                      np.uint64).reshape(-1, 2)
+        bufs.append(torch.zeros(2 * n * size + 8, dtype=torch.uint8, device="cuda"))
+        tiers.append((bufs[-1], rg, torch.zeros((n, 2, 32), dtype=torch.uint8, device="cuda"),
+                      torch.zeros((n, 32), dtype=torch.uint8, device="cuda")))
+    other = torch.cuda.Stream()
+    for rep in range(3):
+        new = [torch.from_numpy(rng.randint(0, 256, b.numel()).astype(np.uint8)).cuda() for b in bufs]
+        torch.cuda.synchronize()
+        if side:
+            with torch.cuda.stream(other):
+                torch.cuda._sleep(2_000_000)
+                for b, x in zip(bufs, new):
+                    b.copy_(x)
+            torch.cuda.current_stream().wait_stream(other)
+        else:
+            for b, x in zip(bufs, new):
+                b.copy_(x)
+        ctx.build_digests(tiers, 3)
+        for x, (_, rg, blob, lay) in zip(new, tiers):
+            ref = O.blake3_ranges(x.cpu().numpy(), rg) if len(rg) else np.zeros((0, 32), np.uint8)
+            assert np.array_equal(blob.cpu().numpy().reshape(-1, 32), ref), rep
+            want = [O.layer_digest(i % 3, ref[2 * i].tobytes(), ref[2 * i + 1].tobytes()) for i in range(len(rg) // 2)]
+            assert [bytes(r) for r in lay.cpu().numpy()] == want, rep
+
+
+def test_plan_digests_follow_the_side_stream(ctx):
+    """TwoTierPlan.digests(side=...) hashes what the side stream had queued."""
+    import torch
+    from provekv_amd import synth
+    from provekv_amd.pool import TwoTierPlan
+    plan = TwoTierPlan(ctx, 2, 3, 64, 20, [3, 2])
+    bufs = plan.alloc()
+    side = torch.cuda.Stream()
+    x = [torch.from_numpy(synth.corpus_tokens(s, 2, 3, plan.tokens, 64).reshape(-1)).cuda() for s in (1, 2)]
+    torch.cuda.synchronize()
+
+    def host():
+        torch.cuda.synchronize()
+        return plan.digest_report(bufs)
+    want = []
+    for v in x:
+        plan.encode(v, bufs)
+        plan.digests(bufs)
+        want.append(host())
+    assert want[0] != want[1]
+    for k in (0, 1, 0):
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(2_000_000)
+        plan.encode(x[k], bufs, stream=side)
+        plan.digests(bufs, side=side)
+        assert host() == want[k]

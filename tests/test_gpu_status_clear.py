@@ -70,3 +70,27 @@ def test_clear_and_run_refusals(ctx):
     assert run(2, st.data_ptr()) != 0
     assert run(0, st.data_ptr()) == 0 and run(1, st.data_ptr()) == 0 and run(0, None) == 0
     torch.cuda.synchronize()
+
+
+def test_blob_order_and_overlap(ctx):
+    """Blobs may lie in any order in the wire; overlapping ones are refused, in
+    table order or out of it."""
+    import torch
+    from oracle import oracle as O
+    from provekv_amd.device import segments
+    prof = ctx.turbo_profile(64, 4, 32, 42)
+    n, blob = 3, prof.blob_len(3)
+    x = torch.from_numpy(np.random.RandomState(3).randn(4 * n, 64).astype(np.float32)).cuda()
+    wire = torch.zeros(5 * blob, dtype=torch.uint8, device="cuda")
+
+    def encode(offsets):
+        segs = segments([(k * n * 64, 0, 64, o, n, n) for k, o in enumerate(offsets)])
+        prof.encode_segments(x.view(-1), segs, wire)
+    for offsets in ([0, blob, 2 * blob, 3 * blob], [3 * blob + 1, 0, 2 * blob + 1, blob], [7, 3 * blob, blob + 9, 4 * blob]):
+        encode(offsets)
+        w = wire.cpu().numpy()
+        for k, o in enumerate(offsets):
+            assert w[o:o + blob].tobytes() == O.turbo_encode_batch(x[k * n:(k + 1) * n].cpu().numpy(), 42)
+    for offsets in ([0, blob - 1, 2 * blob, 3 * blob], [3 * blob, 0, 2 * blob, 2 * blob + 1], [0, blob, 0, 2 * blob]):
+        with pytest.raises(L.PkvError):
+            encode(offsets)
