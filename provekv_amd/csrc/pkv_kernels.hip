@@ -94,24 +94,24 @@ __device__ __forceinline__ uint32_t lds_byte(const uint32_t* lds, uint32_t off) 
     return (lds[off >> 2] >> (8 * (off & 3))) & 0xffu;
 }
 
-// Move nbytes from LDS (LDS byte 0 == dst byte 0) to global memory at any
-// byte alignment.  Needs one readable padding dword after the staged bytes.
-__device__ void lds_to_global(uint8_t* __restrict__ dst, const uint32_t* lds, uint32_t nbytes, int lane) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(dst);
-    uint32_t head = static_cast<uint32_t>((4u - (a & 3u)) & 3u);
-    if (head > nbytes) head = nbytes;
-    if (static_cast<uint32_t>(lane) < head) dst[lane] = static_cast<uint8_t>(lds_byte(lds, lane));
-    const uint32_t body = (nbytes - head) >> 2;
-    uint32_t* d32 = reinterpret_cast<uint32_t*>(dst + head);
-    const uint32_t sh = head;   // 0..3
-    for (uint32_t k = lane; k < body; k += WAVE) {
-        const uint32_t q = (head >> 2) + k;    // head < 4, so q == k
-        uint32_t w0 = lds[q], w1 = lds[q + 1];
-        d32[k] = sh ? __builtin_amdgcn_alignbyte(w1, w0, sh) : w0;
+// Move nbytes (a multiple of 4) from LDS (LDS byte 0 == dst byte 0) to global
+// memory at any byte alignment, 16 bytes per lane and store; the last store of a
+// range of at least 16 bytes starts early enough to end with it (bytes stored
+// twice get the same value).  Dword stores shifted into place by v_alignbyte
+// cost the encodes 2 to 5 %: config-2 shells, f32 radii,
+// 52.2 -> 49.5 us; 4.2 M head_dim-128 vectors 905 -> 884 us.
+typedef uint32_t v4u_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void lds_to_global(uint8_t* __restrict__ dst, const uint32_t* lds, uint32_t nbytes,
+                                              int lane) {
+    if (nbytes < 16u) {   // one fib payload
+        if (static_cast<uint32_t>(lane) < nbytes) dst[lane] = static_cast<uint8_t>(lds_byte(lds, lane));
+        return;
     }
-    const uint32_t t0 = head + (body << 2);
-    const uint32_t tail = nbytes - t0;
-    if (static_cast<uint32_t>(lane) < tail) dst[t0 + lane] = static_cast<uint8_t>(lds_byte(lds, t0 + lane));
+    for (uint32_t o = 16u * static_cast<uint32_t>(lane); o < nbytes; o += 16u * WAVE) {
+        const uint32_t at = min(o, nbytes - 16u);
+        const v4u_a4 v = *reinterpret_cast<const v4u_a4*>(lds + (at >> 2));
+        __builtin_memcpy(dst + at, &v, 16);
+    }
 }
 
 // Move nbytes from global memory at any byte alignment into LDS (LDS byte 0 ==
@@ -151,7 +151,6 @@ __device__ void global_to_lds(uint32_t* lds, const uint8_t* __restrict__ src, ui
 // and an extra instruction per 4 bytes.)  SKIP: loads wholly past the range
 // are left out (for callers whose usual range is well below MAXK loads;
 // otherwise the test costs more than the rare repeat).
-typedef uint32_t v4u_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <uint32_t MAXK, bool SKIP>
 __device__ __forceinline__ void global_to_lds16(uint32_t* lds, const uint8_t* __restrict__ src, uint32_t nbytes,
                                                 int lane) {
@@ -227,11 +226,15 @@ __device__ void stage_rows_in(float* stage, const void* __restrict__ in, bool bf
     }
 }
 
-// f32 -> bfloat16 bits, round to nearest even (torch's / c10's conversion).
-__device__ __forceinline__ uint32_t bf16_rne(float x) {
-    const uint32_t u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;   // NaN stays a (quiet) NaN
-    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+// Two f32 -> bfloat16 bits, round to nearest even (torch's / c10's conversion;
+// a NaN keeps its upper bits and turns quiet): one v_cvt_pk_bf16_f32, equal to
+// the integer rounding it replaces on every float, where that took six
+// operations a value (config-3 step into one bf16 cache 404 -> 364 us, with the
+// other changes to its decodes; the shells' decode into one 36 -> 32 us).
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2bf));
 }
 
 // f32 -> binary16 bits, round to nearest even (v_cvt_f16_f32 in the default mode).
@@ -240,7 +243,7 @@ __device__ __forceinline__ uint32_t f16_rne(float x) {
 }
 
 __device__ __forceinline__ uint32_t pack_out2(float a, float b, uint32_t dt) {
-    return dt == PKV_BF16 ? bf16_rne(a) | (bf16_rne(b) << 16) : f16_rne(a) | (f16_rne(b) << 16);
+    return dt == PKV_BF16 ? bf16_pair(a, b) : f16_rne(a) | (f16_rne(b) << 16);
 }
 
 // Store four consecutive values of one output vector at element offset `off`
@@ -269,7 +272,7 @@ __device__ __forceinline__ void store_out1(void* __restrict__ out, const LaunchC
     if (lc.out_dtype == PKV_F32) {
         for (uint32_t k = 0; k < lc.fanout; ++k, off += lc.fanout_stride) static_cast<float*>(out)[off] = v;
     } else {
-        const uint16_t w = static_cast<uint16_t>(lc.out_dtype == PKV_BF16 ? bf16_rne(v) : f16_rne(v));
+        const uint16_t w = static_cast<uint16_t>(lc.out_dtype == PKV_BF16 ? bf16_pair(v, v) & 0xffffu : f16_rne(v));
         for (uint32_t k = 0; k < lc.fanout; ++k, off += lc.fanout_stride) static_cast<uint16_t*>(out)[off] = w;
     }
 }
@@ -1872,8 +1875,11 @@ __host__ __device__ constexpr uint32_t turbo_split_wave_words(uint32_t pwd) { re
 // head) those are 16 heads at two consecutive tokens, so each store
 // instruction writes two runs of two adjacent 256 B rows (tokens t, t + 1 of
 // one head).  Any other layout is only another order of the same stores.
-template <int PB>
-__global__ __launch_bounds__(TILE) void turbo_decode_split_kernel(
+// One kernel per radii codec: with both in one, the f32 path's schedule suffered
+// from the other's code (4.2 M vectors to f32, f32 radii: 387 us together, 362 us
+// apart).
+template <int PB, bool LOSSY>
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void turbo_decode_split_kernel(
     LaunchCommon lc, const uint8_t* __restrict__ wire, void* __restrict__ out,
     const float* __restrict__ signs, const float* __restrict__ cs_tab, uint64_t seed, uint32_t pbits_rt,
     uint32_t proj, uint32_t mode) {
@@ -1887,7 +1893,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split_kernel(
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
-    if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
+    if (LOSSY && threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
     __syncthreads();
 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -1976,11 +1982,10 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split_kernel(
         // this lane's output row offset, computed once (one division by the
         // segment's group) and handed to the storing lanes by a shuffle
         const uint64_t my_off = vec_elem_offset(seg, vi);
-        const bool f32r = lc.radii == PKV_RADII_F32;
-        const uint32_t rwords = f32r ? 32u : 32u / 4 + 2;
+        constexpr uint32_t rwords = LOSSY ? 32u / 4 + 2 : 32u;
         bool ok = true;
         float r[HP];
-        if (f32r) {
+        if constexpr (!LOSSY) {
 #pragma unroll
             for (int i = 0; i < HP; ++i) {
                 r[i] = u2f(pword(16 * h + i));
@@ -2061,7 +2066,7 @@ __host__ __device__ constexpr uint32_t turbo_split128_wave_words(uint32_t pwd) {
     return (16 * pwd + 4 > 16 * (128 + 4) + 4) ? 16 * pwd + 4 : 16 * (128 + 4) + 4;
 }
 
-template <int PB>
+template <int PB, bool LOSSY>
 __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     LaunchCommon lc, const uint8_t* __restrict__ wire, void* __restrict__ out,
     const float* __restrict__ signs, const float* __restrict__ cs_tab, uint64_t seed, uint32_t pbits_rt,
@@ -2076,7 +2081,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
-    if (threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
+    if (LOSSY && threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -2107,11 +2112,10 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     const uint32_t mine = min(static_cast<uint32_t>(n), nv - 1);
     const uint32_t* pw = sw + mine * pwd;
     const uint64_t my_off = vec_elem_offset(seg, t0 + mine);
-    const bool f32r = lc.radii == PKV_RADII_F32;
-    const uint32_t rwords = f32r ? 64u : 64u / 4 + 2;
+    constexpr uint32_t rwords = LOSSY ? 64u / 4 + 2 : 64u;
     bool ok = true;
     float r[HP];
-    if (f32r) {
+    if constexpr (!LOSSY) {
 #pragma unroll
         for (int i = 0; i < HP; ++i) {
             r[i] = u2f(pw[(i < 8 ? 8 * q : 24 + 8 * q) + i]);
@@ -3884,18 +3888,22 @@ int launch_turbo_decode(const LaunchCommon& lc, const TurboDev& td, const uint8_
         if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 workgroups per tile
         // a resident grid (four workgroups per CU) walking contiguous shares
         const uint32_t grid = std::min(2 * nblocks, lc.grid_cap ? lc.grid_cap : 1024u);
-        return td.pbits == 3 ? launch_big_lds(turbo_decode_split_kernel<3>, grid, lds, st, lc, wire, out,
-                                              td.signs, td.cs, td.seed, td.pbits, td.proj, td.mode)
-                             : launch_big_lds(turbo_decode_split_kernel<0>, grid, lds, st, lc, wire, out,
-                                              td.signs, td.cs, td.seed, td.pbits, td.proj, td.mode);
+#define PKV_SPLIT64(PB, LO)                                                                                  \
+    launch_big_lds(turbo_decode_split_kernel<PB, LO>, grid, lds, st, lc, wire, out, td.signs, td.cs, td.seed, \
+                   td.pbits, td.proj, td.mode)
+        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT64(3, false) : PKV_SPLIT64(0, false);
+        return td.pbits == 3 ? PKV_SPLIT64(3, true) : PKV_SPLIT64(0, true);
+#undef PKV_SPLIT64
     }
     if (td.dim == 128 && td.pbits <= 4) {
         if (nblocks > (1u << 29)) return hipErrorInvalidValue;   // 4 workgroups per tile
         const size_t lds = static_cast<size_t>(WAVES) * turbo_split128_wave_words(lc.plen >> 2) * sizeof(uint32_t);
-        return td.pbits == 3 ? launch_big_lds(turbo_decode_split128_kernel<3>, 4 * nblocks, lds, st, lc, wire, out,
-                                              td.signs, td.cs, td.seed, td.pbits, td.proj)
-                             : launch_big_lds(turbo_decode_split128_kernel<0>, 4 * nblocks, lds, st, lc, wire, out,
-                                              td.signs, td.cs, td.seed, td.pbits, td.proj);
+#define PKV_SPLIT128(PB, LO)                                                                            \
+    launch_big_lds(turbo_decode_split128_kernel<PB, LO>, 4 * nblocks, lds, st, lc, wire, out, td.signs, \
+                   td.cs, td.seed, td.pbits, td.proj)
+        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT128(3, false) : PKV_SPLIT128(0, false);
+        return td.pbits == 3 ? PKV_SPLIT128(3, true) : PKV_SPLIT128(0, true);
+#undef PKV_SPLIT128
     }
     if (td.dim == 64)
         return td.pbits == 3
