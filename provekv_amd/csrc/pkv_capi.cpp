@@ -486,18 +486,15 @@ FibDev fib_dev(const pkv_profile* p) {
     return f;
 }
 
-// Clears the status words (unless the caller has) and launches the encode or decode kernel of the
+// Clears the status words (unless the caller has, or each workgroup stores its
+// segment's) and launches the encode or decode kernel of the
 // profile over a device-resident segment table (dsegs, dtiles: nseg + 1 tile
-// prefix, nblocks tiles in all).  Returns a hipError_t as int.
+// prefix, nblocks tiles in all; segs: the host's copy).  Returns a hipError_t as int.
 int launch_segments(const pkv_profile* prof, int radii, bool encode, int dtype, const void* d_f32,
-                    const uint8_t* d_wire, const SegDev* dsegs, const uint32_t* dtiles, uint32_t nseg,
+                    const uint8_t* d_wire, const pkv_seg* segs, const SegDev* dsegs, const uint32_t* dtiles, uint32_t nseg,
                     uint32_t nblocks, uint32_t* status, bool per_vector, uint32_t fanout, uint64_t fanout_stride,
                     uint32_t grid_cap, hipStream_t stream, float* diag = nullptr, const uint32_t* dmap = nullptr,
                     bool cleared = false) {
-    if (!cleared) {
-        const int e = launch_fill_u32(status, STATUS_NONE, 2ull * nseg, stream);
-        if (e) return e;
-    }
     LaunchCommon lc;
     lc.segs = dsegs;
     lc.tile_start = dtiles;
@@ -513,6 +510,16 @@ int launch_segments(const pkv_profile* prof, int radii, bool encode, int dtype, 
     lc.fanout_stride = fanout_stride;
     lc.grid_cap = grid_cap;
     lc.diag = diag;
+    if (!cleared && prof->kind == PKV_CODEC_TURBO && nblocks == nseg) {   // as many tiles as segments
+        const uint32_t most = turbo_own_vectors(lc, turbo_dev(prof), encode, nblocks);
+        uint32_t i = 0;
+        while (i < nseg && segs[i].n_vectors - 1u < most) ++i;   // 1 .. most vectors
+        lc.own_status = i == nseg ? 1u : 0u;
+    }
+    if (!cleared && !lc.own_status) {
+        const int e = launch_fill_u32(status, STATUS_NONE, 2ull * nseg, stream);
+        if (e) return e;
+    }
     if (prof->kind == PKV_CODEC_TURBO)
         return encode ? launch_turbo_encode(lc, turbo_dev(prof), d_f32, const_cast<uint8_t*>(d_wire), nblocks, stream)
                       : launch_turbo_decode(lc, turbo_dev(prof), d_wire, const_cast<void*>(d_f32), nblocks, stream);
@@ -556,7 +563,7 @@ int run_segments_locked(pkv_ctx* ctx, const pkv_profile* prof, int radii, bool e
     rc = stage_table(ctx, segs, nseg, tiles, d_status == nullptr, stream, &sl, &dsegs, &dtiles, &dstat, &dmap);
     if (rc) return rc;
     uint32_t* status = d_status ? d_status : dstat;
-    const int e = launch_segments(prof, radii, encode, dtype, d_f32, d_wire, dsegs, dtiles, nseg, tiles[nseg], status,
+    const int e = launch_segments(prof, radii, encode, dtype, d_f32, d_wire, segs, dsegs, dtiles, nseg, tiles[nseg], status,
                                   per_vector, fanout, fanout_stride, grid_cap, stream, diag, dmap, cleared);
     int rc2 = finish_slot(sl, stream);
     if (e) return hip_status(static_cast<hipError_t>(e));
@@ -1397,7 +1404,7 @@ int pkv_decode_segments_noalloc(pkv_ctx* ctx, const pkv_profile* prof, int radii
     // pageable host sources: the runtime stages them before returning
     HIP_TRY(hipMemcpyAsync(base, segs, sizeof(pkv_seg) * nseg, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(base + kNaTileOff, tiles, sizeof(uint32_t) * (nseg + 1), hipMemcpyHostToDevice, st));
-    const int e = launch_segments(prof, radii, false, out_dtype, d_out, d_wire, reinterpret_cast<const SegDev*>(base),
+    const int e = launch_segments(prof, radii, false, out_dtype, d_out, d_wire, segs, reinterpret_cast<const SegDev*>(base),
                                   reinterpret_cast<const uint32_t*>(base + kNaTileOff), nseg, tiles[nseg], d_status,
                                   false, fanout, fanout_stride, 0, st);
     const hipError_t re = hipEventRecord(sc.ev, st);

@@ -106,6 +106,8 @@ struct LaunchCommon {
     uint64_t fanout_stride;       // ... this many elements apart
     uint32_t grid_cap = 0;        // at most this many workgroups, each walking tiles (0: one per tile);
                                   // d64 turbo decode and the fib MFMA decode
+    uint32_t own_status = 0;      // turbo: every segment's vectors fall to one workgroup, which stores its
+                                  // two status words itself (they need no clear)
     float* diag = nullptr;        // encode diagnostics (pkv_encode_diagnostics): the matrix-core values
                                   // the kernel decided from, per vector of the (single) segment;
                                   // non-null selects the kernels' diagnostic instantiations
@@ -163,6 +165,8 @@ void constants_cache_stats(uint64_t* hits, uint64_t* misses, uint64_t* entries);
 void constants_cache_clear();
 
 // Kernel launchers (pkv_kernels.hip).  Return a hipError_t as int.
+// Most vectors a segment may have (and at least one) for LaunchCommon::own_status, 0: never.
+uint32_t turbo_own_vectors(const LaunchCommon& lc, const TurboDev& td, bool encode, uint32_t nblocks);
 int launch_turbo_encode(const LaunchCommon& lc, const TurboDev& td, const void* in, uint8_t* wire,
                         uint32_t nblocks, void* stream);
 int launch_turbo_decode(const LaunchCommon& lc, const TurboDev& td, const uint8_t* wire, void* out,

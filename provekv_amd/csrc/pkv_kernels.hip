@@ -339,6 +339,35 @@ __device__ __forceinline__ void status_fail(uint32_t* status, uint32_t seg, int 
     atomicMin(status + 2 * seg + word, (index << 4) | kind);
 }
 
+// The two status words of a segment.  OWN: its vectors all fall to one
+// workgroup, which gathers the words in LDS and stores them at the kernel's
+// end, so the launch needs no clear of the status words before it: a call that
+// small is bound by its launches (48 segments of 32 vectors encoded in 8.5 us,
+// 10.1 with the clear as a launch of its own; 128 of 20 decoded in 8.4,
+// 11.3).  Otherwise failures are marked in the cleared words as they occur.
+// A template argument: as a run-time flag it cost the large calls 1 to 3 %.
+// Four LDS words for two: the dynamic LDS begins where the static arrays end,
+// and 16-byte accesses at 8 past a multiple of 16 cost the decodes 25 %.
+template <bool OWN>
+struct SegStatus {
+    uint32_t* lds;
+    __device__ __forceinline__ void init() const {   // before the workgroup's first barrier
+        if (OWN && threadIdx.x < 2) lds[threadIdx.x] = 0xFFFFFFFFu;
+    }
+    __device__ __forceinline__ void fail(uint32_t* status, uint32_t seg, int word, uint32_t index,
+                                         uint32_t kind) const {
+        if constexpr (OWN) atomicMin(lds + word, (index << 4) | kind);
+        else status_fail(status, seg, word, index, kind);
+    }
+    // Every thread of the workgroup, last; `first`: the workgroup holds the segment's vectors.
+    __device__ __forceinline__ void store(uint32_t* status, uint32_t seg, bool first) const {
+        if constexpr (OWN) {
+            __syncthreads();
+            if (first && threadIdx.x < 2) status[2 * seg + threadIdx.x] = lds[threadIdx.x];
+        }
+    }
+};
+
 // TQB1 header byte i (turbo-quant/src/wire.rs:267-346).
 __device__ __forceinline__ uint32_t tqb1_byte(uint32_t i, uint32_t dim, uint32_t pbits, uint32_t radii,
                                               uint32_t proj, uint64_t seed, uint32_t n, uint32_t plen) {
@@ -936,7 +965,7 @@ __device__ __forceinline__ void qjl_split8(const float (&v)[32], int c0, float s
 
 // DIAG: also write every projection's matrix-core dot and acceptance bound
 // (divided by the residual's scale) to lc.diag[((vector * proj) + j) * 2 + {0, 1}].
-template <int PB, bool DIAG>
+template <int PB, bool DIAG, bool OWN>
 __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
     LaunchCommon lc, const void* __restrict__ in, uint8_t* __restrict__ wire, const float* __restrict__ signs,
     const float* __restrict__ qjl, const float* __restrict__ cs_tab, const uint32_t* __restrict__ qa,
@@ -946,6 +975,8 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
     extern __shared__ uint32_t smem_u[];   // per wave: 32 payloads (+ f32 radii for BlockLogU8)
     __shared__ float cs_lds[512];
     __shared__ LogfEntry logf_lds[16];
+    __shared__ uint32_t own_lds[OWN ? 4 : 1];
+    const SegStatus<OWN> own{own_lds};
     // the signs (+-1.0), then -sign * scale: the scale is 2^-3, so both are exact
     __shared__ __align__(16) float sg_lds[2 * DIM];
 
@@ -953,6 +984,7 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (threadIdx.x < 16) logf_lds[threadIdx.x] = c_logf_tab[threadIdx.x];
+    own.init();
     for (uint32_t t = threadIdx.x; t < DIM; t += blockDim.x) {
         const float sv = signs[t];
         sg_lds[t] = sv;
@@ -1239,9 +1271,9 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
         bad |= partner(bad, h);
         if (active && h == 0) {
             const uint32_t vi = t0 + n;
-            if (bad & 1u) status_fail(lc.status, sidx, 1, vi, KIND_NONFINITE_INPUT);
-            else if (bad & 2u) status_fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RADIUS);
-            else if (bad & 4u) status_fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RESIDUAL);
+            if (bad & 1u) own.fail(lc.status, sidx, 1, vi, KIND_NONFINITE_INPUT);
+            else if (bad & 2u) own.fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RADIUS);
+            else if (bad & 4u) own.fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RESIDUAL);
             pv[rwords + bwords] = sbits[0];
             if (proj > 32) pv[rwords + bwords + 1] = sbits[1];
         }
@@ -1268,6 +1300,7 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
         blob[threadIdx.x] = static_cast<uint8_t>(
             tqb1_byte(threadIdx.x, DIM, pbits, lc.radii, proj, seed, seg.n_vectors, plen));
     }
+    own.store(lc.status, sidx, (blockIdx.x & 1u) == 0);
 }
 
 // Head_dim 128: four lanes per vector, lane (q, n) = (lane / 16, lane % 16)
@@ -1402,7 +1435,7 @@ __device__ __forceinline__ uint32_t or_quarters(uint32_t x, int q) {
     return x | partner(x, q >> 1);
 }
 
-template <int PB, bool DIAG>
+template <int PB, bool DIAG, bool OWN>
 __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
     LaunchCommon lc, const void* __restrict__ in, uint8_t* __restrict__ wire, const float* __restrict__ signs,
     const float* __restrict__ qjl, const float* __restrict__ cs_tab, const uint32_t* __restrict__ qa,
@@ -1413,11 +1446,14 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
     extern __shared__ uint32_t smem_u[];   // per wave: 16 payloads
     __shared__ float cs_lds[512];
     __shared__ LogfEntry logf_lds[16];
+    __shared__ uint32_t own_lds[OWN ? 4 : 1];
+    const SegStatus<OWN> own{own_lds};
 
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (threadIdx.x < 16) logf_lds[threadIdx.x] = c_logf_tab[threadIdx.x];
+    own.init();
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1688,9 +1724,9 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
         const uint32_t bad = or_quarters((finite ? 0u : 1u) | (rfinite ? 0u : 2u) | (resfinite ? 0u : 4u), q);
         if (active && q == 0) {
             const uint32_t vi = t0 + n;
-            if (bad & 1u) status_fail(lc.status, sidx, 1, vi, KIND_NONFINITE_INPUT);
-            else if (bad & 2u) status_fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RADIUS);
-            else if (bad & 4u) status_fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RESIDUAL);
+            if (bad & 1u) own.fail(lc.status, sidx, 1, vi, KIND_NONFINITE_INPUT);
+            else if (bad & 2u) own.fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RADIUS);
+            else if (bad & 4u) own.fail(lc.status, sidx, 1, vi, KIND_NONFINITE_RESIDUAL);
             pv[rwords + bwords] = sbits[0];
             if (proj > 32) pv[rwords + bwords + 1] = sbits[1];
         }
@@ -1701,6 +1737,7 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
         blob[threadIdx.x] = static_cast<uint8_t>(
             tqb1_byte(threadIdx.x, DIM, pbits, lc.radii, proj, seed, seg.n_vectors, plen));
     }
+    own.store(lc.status, sidx, (blockIdx.x & 3u) == 0);
 }
 
 // ------------------------------------------------------------ turbo decode
@@ -1878,7 +1915,7 @@ __host__ __device__ constexpr uint32_t turbo_split_wave_words(uint32_t pwd) { re
 // One kernel per radii codec: with both in one, the f32 path's schedule suffered
 // from the other's code (4.2 M vectors to f32, f32 radii: 387 us together, 362 us
 // apart).
-template <int PB, bool LOSSY>
+template <int PB, bool LOSSY, bool OWN>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void turbo_decode_split_kernel(
     LaunchCommon lc, const uint8_t* __restrict__ wire, void* __restrict__ out,
     const float* __restrict__ signs, const float* __restrict__ cs_tab, uint64_t seed, uint32_t pbits_rt,
@@ -1889,11 +1926,14 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
     extern __shared__ uint32_t smem_u[];   // per wave: two buffers of turbo_split_buf_words
     __shared__ float cs_lds[32];           // levels <= 16
     __shared__ uint64_t exp_lds[32];
+    __shared__ uint32_t own_lds[OWN ? 4 : 1];
+    const SegStatus<OWN> own{own_lds};
 
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (LOSSY && threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
+    own.init();
     __syncthreads();
 
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -1966,7 +2006,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
         const bool hbad = lane < 38 && tqb1_checked(lane) &&
                           it.hb != tqb1_byte(lane, DIM, pbits, lc.radii, proj, seed, seg.n_vectors, plen);
         if (__ballot(hbad) != 0ull) {
-            if (lane == 0) status_fail(lc.status, it.sidx, 0, 0u, KIND_HEADER);
+            if (lane == 0) own.fail(lc.status, it.sidx, 0, 0u, KIND_HEADER);
             continue;
         }
         if (!it.n0) continue;
@@ -2018,7 +2058,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
         fwht_split(y, h);
         const float scale = fwht_scale<DIM>();
         const bool vok = ok && partner(ok ? 1u : 0u, h);
-        if (active && h == 0 && !vok) status_fail(lc.status, it.sidx, 1, vi, KIND_CORRUPT);
+        if (active && h == 0 && !vok) own.fail(lc.status, it.sidx, 1, vi, KIND_CORRUPT);
         // rows to write: the active, good vectors (lane n's vector: run n / 16, j)
         const uint32_t wmask = static_cast<uint32_t>(__ballot(active && h == 0 && vok));
         // Rows leave through LDS (staged over the consumed payload buffer), 16
@@ -2055,6 +2095,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(4))) void 
             }
         }
     }
+    own.store(lc.status, sidx, (vb0 & 1u) == 0);   // such a launch has one half-tile per workgroup
 }
 
 // Turbo decode at head_dim 128: four lanes per vector as in
@@ -2066,7 +2107,7 @@ __host__ __device__ constexpr uint32_t turbo_split128_wave_words(uint32_t pwd) {
     return (16 * pwd + 4 > 16 * (128 + 4) + 4) ? 16 * pwd + 4 : 16 * (128 + 4) + 4;
 }
 
-template <int PB, bool LOSSY>
+template <int PB, bool LOSSY, bool OWN>
 __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     LaunchCommon lc, const uint8_t* __restrict__ wire, void* __restrict__ out,
     const float* __restrict__ signs, const float* __restrict__ cs_tab, uint64_t seed, uint32_t pbits_rt,
@@ -2077,11 +2118,14 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     extern __shared__ uint32_t smem_u[];   // per wave: 16 payloads, then 16 decoded rows
     __shared__ float cs_lds[512];
     __shared__ uint64_t exp_lds[32];
+    __shared__ uint32_t own_lds[OWN ? 4 : 1];
+    const SegStatus<OWN> own{own_lds};
 
     const uint32_t pbits = PB ? static_cast<uint32_t>(PB) : pbits_rt;
     const uint32_t levels = 1u << pbits;
     for (uint32_t t = threadIdx.x; t < 2 * levels; t += blockDim.x) cs_lds[t] = cs_tab[t];
     if (LOSSY && threadIdx.x < 32) exp_lds[threadIdx.x] = c_exp2f_tab[threadIdx.x];
+    own.init();
     __syncthreads();
 
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -2093,86 +2137,89 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
     const uint32_t plen = lc.plen, pwd = plen >> 2;
     const uint8_t* blob = wire + seg.wire_offset;
 
-    // header check (every wave; 38 bytes)
-    const uint32_t hb = lane < 38 ? blob[lane] : 0u;
-    const bool hbad = lane < 38 && tqb1_checked(lane) &&
-                      hb != tqb1_byte(lane, DIM, pbits, lc.radii, proj, seed, seg.n_vectors, plen);
-    if (__ballot(hbad) != 0ull) {
-        if (lane == 0) status_fail(lc.status, sidx, 0, 0u, KIND_HEADER);
-        return;
-    }
-    const uint32_t t0 = tile * TILE + (blockIdx.x & 3u) * (TILE / 4) + GV * static_cast<uint32_t>(wave);
-    if (t0 >= seg.n_vectors) return;
-    const uint32_t nv = min(static_cast<uint32_t>(GV), seg.n_vectors - t0);
-    uint32_t* sw = smem_u + wave * turbo_split128_wave_words(pwd);
-    global_to_lds16<5, true>(sw, blob + 38 + static_cast<uint64_t>(t0) * plen, nv * plen, lane);   // <= 16 * 296 B
-    wave_sync();
+    do {
+        // header check (every wave; 38 bytes)
+        const uint32_t hb = lane < 38 ? blob[lane] : 0u;
+        const bool hbad = lane < 38 && tqb1_checked(lane) &&
+                          hb != tqb1_byte(lane, DIM, pbits, lc.radii, proj, seed, seg.n_vectors, plen);
+        if (__ballot(hbad) != 0ull) {
+            if (lane == 0) own.fail(lc.status, sidx, 0, 0u, KIND_HEADER);
+            break;
+        }
+        const uint32_t t0 = tile * TILE + (blockIdx.x & 3u) * (TILE / 4) + GV * static_cast<uint32_t>(wave);
+        if (t0 >= seg.n_vectors) break;
+        const uint32_t nv = min(static_cast<uint32_t>(GV), seg.n_vectors - t0);
+        uint32_t* sw = smem_u + wave * turbo_split128_wave_words(pwd);
+        global_to_lds16<5, true>(sw, blob + 38 + static_cast<uint64_t>(t0) * plen, nv * plen, lane);   // <= 16 * 296 B
+        wave_sync();
 
-    const bool active = static_cast<uint32_t>(n) < nv;
-    const uint32_t mine = min(static_cast<uint32_t>(n), nv - 1);
-    const uint32_t* pw = sw + mine * pwd;
-    const uint64_t my_off = vec_elem_offset(seg, t0 + mine);
-    constexpr uint32_t rwords = LOSSY ? 64u / 4 + 2 : 64u;
-    bool ok = true;
-    float r[HP];
-    if constexpr (!LOSSY) {
-#pragma unroll
+        const bool active = static_cast<uint32_t>(n) < nv;
+        const uint32_t mine = min(static_cast<uint32_t>(n), nv - 1);
+        const uint32_t* pw = sw + mine * pwd;
+        const uint64_t my_off = vec_elem_offset(seg, t0 + mine);
+        constexpr uint32_t rwords = LOSSY ? 64u / 4 + 2 : 64u;
+        bool ok = true;
+        float r[HP];
+        if constexpr (!LOSSY) {
+    #pragma unroll
+            for (int i = 0; i < HP; ++i) {
+                r[i] = u2f(pw[(i < 8 ? 8 * q : 24 + 8 * q) + i]);
+                ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);   // radius.rs:88-104
+            }
+        } else {
+            uint32_t w[4];
+    #pragma unroll
+            for (int k = 0; k < 4; ++k) w[k] = pw[(k < 2 ? 2 * q : 6 + 2 * q) + k];
+            radii_u8<HP>(w, u2f(pw[16]), u2f(pw[17]), exp_lds, r, ok);
+        }
+        // this lane's two runs of 8 angle indices, 8 pbits (<= 32) bits each, at
+        // bits 8 pbits q and 8 pbits (4 + q)
+        uint64_t pk;
+        {
+            const uint32_t nb = 8u * pbits;
+            uint64_t run[2];
+    #pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const uint32_t bit0 = nb * (static_cast<uint32_t>(q) + 4u * half);
+                const uint32_t* aw = pw + rwords + (bit0 >> 5);
+                const uint64_t v = static_cast<uint64_t>(aw[0]) | static_cast<uint64_t>(aw[1]) << 32;
+                run[half] = (v >> (bit0 & 31u)) & ((1ull << nb) - 1u);
+            }
+            pk = run[0] | run[1] << nb;
+        }
+        // the angle field is 64 * pbits bits, a whole number of words: no padding
+        // bits to check (bitpack.rs:88-109); nor in the 32/64-bit QJL field
+
+        float y[32];
+    #pragma unroll
         for (int i = 0; i < HP; ++i) {
-            r[i] = u2f(pw[(i < 8 ? 8 * q : 24 + 8 * q) + i]);
-            ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);   // radius.rs:88-104
+            const uint32_t bin = static_cast<uint32_t>(pk >> (static_cast<uint32_t>(i) * pbits)) & (levels - 1u);
+            y[2 * i] = r[i] * cs_lds[2 * bin];
+            y[2 * i + 1] = r[i] * cs_lds[2 * bin + 1];
         }
-    } else {
-        uint32_t w[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = pw[(k < 2 ? 2 * q : 6 + 2 * q) + k];
-        radii_u8<HP>(w, u2f(pw[16]), u2f(pw[17]), exp_lds, r, ok);
-    }
-    // this lane's two runs of 8 angle indices, 8 pbits (<= 32) bits each, at
-    // bits 8 pbits q and 8 pbits (4 + q)
-    uint64_t pk;
-    {
-        const uint32_t nb = 8u * pbits;
-        uint64_t run[2];
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const uint32_t bit0 = nb * (static_cast<uint32_t>(q) + 4u * half);
-            const uint32_t* aw = pw + rwords + (bit0 >> 5);
-            const uint64_t v = static_cast<uint64_t>(aw[0]) | static_cast<uint64_t>(aw[1]) << 32;
-            run[half] = (v >> (bit0 & 31u)) & ((1ull << nb) - 1u);
+        fwht128_inv(y);   // layout F -> layout G
+        const float scale = fwht_scale<DIM>();
+        const bool vok = or_quarters(ok ? 0u : 1u, q) == 0u;
+        if (active && q == 0 && !vok) own.fail(lc.status, sidx, 1, t0 + n, KIND_CORRUPT);
+        // rows through LDS (over the consumed payloads) so they leave coalesced
+        wave_sync();
+        float* stage = reinterpret_cast<float*>(sw);
+        {
+            const uint32_t g0 = 16u * static_cast<uint32_t>(((q & 1) << 1) | (q >> 1)), g1 = 64u + g0;
+    #pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const uint32_t e = (k < 4 ? g0 : g1) + 4u * (k & 3);
+                const float4 sg = *reinterpret_cast<const float4*>(signs + e);
+                *reinterpret_cast<float4*>(stage + n * (DIM + 4) + e) =
+                    make_float4((y[4 * k] * scale) * sg.x, (y[4 * k + 1] * scale) * sg.y, (y[4 * k + 2] * scale) * sg.z,
+                                (y[4 * k + 3] * scale) * sg.w);
+            }
         }
-        pk = run[0] | run[1] << nb;
-    }
-    // the angle field is 64 * pbits bits, a whole number of words: no padding
-    // bits to check (bitpack.rs:88-109); nor in the 32/64-bit QJL field
-
-    float y[32];
-#pragma unroll
-    for (int i = 0; i < HP; ++i) {
-        const uint32_t bin = static_cast<uint32_t>(pk >> (static_cast<uint32_t>(i) * pbits)) & (levels - 1u);
-        y[2 * i] = r[i] * cs_lds[2 * bin];
-        y[2 * i + 1] = r[i] * cs_lds[2 * bin + 1];
-    }
-    fwht128_inv(y);   // layout F -> layout G
-    const float scale = fwht_scale<DIM>();
-    const bool vok = or_quarters(ok ? 0u : 1u, q) == 0u;
-    if (active && q == 0 && !vok) status_fail(lc.status, sidx, 1, t0 + n, KIND_CORRUPT);
-    // rows through LDS (over the consumed payloads) so they leave coalesced
-    wave_sync();
-    float* stage = reinterpret_cast<float*>(sw);
-    {
-        const uint32_t g0 = 16u * static_cast<uint32_t>(((q & 1) << 1) | (q >> 1)), g1 = 64u + g0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t e = (k < 4 ? g0 : g1) + 4u * (k & 3);
-            const float4 sg = *reinterpret_cast<const float4*>(signs + e);
-            *reinterpret_cast<float4*>(stage + n * (DIM + 4) + e) =
-                make_float4((y[4 * k] * scale) * sg.x, (y[4 * k + 1] * scale) * sg.y, (y[4 * k + 2] * scale) * sg.z,
-                            (y[4 * k + 3] * scale) * sg.w);
-        }
-    }
-    const uint32_t wmask = static_cast<uint32_t>(__ballot(active && q == 0 && vok));
-    wave_sync();
-    stage_rows_out_at<DIM>(out, lc, stage, my_off, nv, wmask, lane);
+        const uint32_t wmask = static_cast<uint32_t>(__ballot(active && q == 0 && vok));
+        wave_sync();
+        stage_rows_out_at<DIM>(out, lc, stage, my_off, nv, wmask, lane);
+    } while (false);
+    own.store(lc.status, sidx, (blockIdx.x & 3u) == 0);
 }
 
 // ------------------------------------------------------------ scoring on codes
@@ -3842,6 +3889,26 @@ hipError_t launch_big_lds(K kernel, uint32_t nblocks, size_t lds, hipStream_t st
     return hipGetLastError();
 }
 
+namespace {
+constexpr uint32_t kSplit64Grid = 1024;   // a resident grid, four workgroups per CU
+}
+
+// The matrix-core encodes and the split decodes give a workgroup half a tile
+// (head_dim 64) or a quarter (128) of a segment.  Up to one resident grid
+// (four workgroups per CU): 384 segments of 128 head_dim-64 vectors encode in
+// 16.5 us (18.0 with the clear) and decode to f32 in 9.8 (12.2).  Past that the
+// 1 % that the owning kernels are slower reaches what the clear costs, and a
+// decode's workgroups walk several half-tiles.  The general kernels (no
+// projections, more than 4 bits) are left with the clear: their waves end by
+// returns of their own.
+uint32_t turbo_own_vectors(const LaunchCommon& lc, const TurboDev& td, bool encode, uint32_t nblocks) {
+    if (lc.diag || td.pbits > 4 || (encode && !(td.mode && td.qa))) return 0;
+    if (td.dim != 64 && td.dim != 128) return 0;
+    const uint32_t parts = td.dim == 64 ? 2u : 4u;   // workgroups per tile
+    const uint32_t cap = !encode && td.dim == 64 && lc.grid_cap ? std::min(lc.grid_cap, kSplit64Grid) : kSplit64Grid;
+    return static_cast<uint64_t>(parts) * nblocks <= cap ? TILE / parts : 0u;
+}
+
 int launch_turbo_encode(const LaunchCommon& lc, const TurboDev& td, const void* in, uint8_t* wire,
                         uint32_t nblocks, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -3849,21 +3916,23 @@ int launch_turbo_encode(const LaunchCommon& lc, const TurboDev& td, const void* 
         if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 workgroups per tile
         const size_t vec_words = (lc.plen >> 2) + (lc.radii == PKV_RADII_F32 ? 0u : 32u);
         const size_t lds = static_cast<size_t>(WAVES) * (32 * vec_words + 4) * sizeof(uint32_t);
-#define PKV_QJL64(PB, DG)                                                                                      \
-    launch_big_lds(turbo_encode_qjl_kernel<PB, DG>, 2 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl, td.cs, \
+#define PKV_QJL64(PB, DG, OW)                                                                                      \
+    launch_big_lds(turbo_encode_qjl_kernel<PB, DG, OW>, 2 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl, td.cs, \
                    td.qa, td.qb, td.seed, td.pbits, td.proj)
-        if (lc.diag) return td.pbits == 3 ? PKV_QJL64(3, true) : PKV_QJL64(0, true);
-        return td.pbits == 3 ? PKV_QJL64(3, false) : PKV_QJL64(0, false);
+        if (lc.diag) return td.pbits == 3 ? PKV_QJL64(3, true, false) : PKV_QJL64(0, true, false);
+        if (lc.own_status) return td.pbits == 3 ? PKV_QJL64(3, false, true) : PKV_QJL64(0, false, true);
+        return td.pbits == 3 ? PKV_QJL64(3, false, false) : PKV_QJL64(0, false, false);
 #undef PKV_QJL64
     }
     if (td.dim == 128 && td.mode && td.qa && td.pbits <= 4) {
         if (nblocks > (1u << 29)) return hipErrorInvalidValue;   // 4 workgroups per tile
         const size_t lds = static_cast<size_t>(WAVES) * (16 * (lc.plen >> 2) + 4) * sizeof(uint32_t);
-#define PKV_QJL128(PB, DG)                                                                                      \
-    launch_big_lds(turbo_encode_qjl128_kernel<PB, DG>, 4 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl,   \
+#define PKV_QJL128(PB, DG, OW)                                                                                      \
+    launch_big_lds(turbo_encode_qjl128_kernel<PB, DG, OW>, 4 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl,   \
                    td.cs, td.qa, td.qb, td.seed, td.pbits, td.proj)
-        if (lc.diag) return td.pbits == 3 ? PKV_QJL128(3, true) : PKV_QJL128(0, true);
-        return td.pbits == 3 ? PKV_QJL128(3, false) : PKV_QJL128(0, false);
+        if (lc.diag) return td.pbits == 3 ? PKV_QJL128(3, true, false) : PKV_QJL128(0, true, false);
+        if (lc.own_status) return td.pbits == 3 ? PKV_QJL128(3, false, true) : PKV_QJL128(0, false, true);
+        return td.pbits == 3 ? PKV_QJL128(3, false, false) : PKV_QJL128(0, false, false);
 #undef PKV_QJL128
     }
     if (lc.diag) return hipErrorInvalidValue;   // diagnostics exist for the matrix-core paths only
@@ -3886,23 +3955,31 @@ int launch_turbo_decode(const LaunchCommon& lc, const TurboDev& td, const uint8_
     if (td.dim == 64 && td.pbits <= 4) {
         const size_t lds = static_cast<size_t>(WAVES) * turbo_split_wave_words(lc.plen >> 2) * sizeof(uint32_t);
         if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 workgroups per tile
-        // a resident grid (four workgroups per CU) walking contiguous shares
-        const uint32_t grid = std::min(2 * nblocks, lc.grid_cap ? lc.grid_cap : 1024u);
-#define PKV_SPLIT64(PB, LO)                                                                                  \
-    launch_big_lds(turbo_decode_split_kernel<PB, LO>, grid, lds, st, lc, wire, out, td.signs, td.cs, td.seed, \
+        // a resident grid walking contiguous shares
+        const uint32_t grid = std::min(2 * nblocks, lc.grid_cap ? lc.grid_cap : kSplit64Grid);
+#define PKV_SPLIT64(PB, LO, OW)                                                                                  \
+    launch_big_lds(turbo_decode_split_kernel<PB, LO, OW>, grid, lds, st, lc, wire, out, td.signs, td.cs, td.seed, \
                    td.pbits, td.proj, td.mode)
-        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT64(3, false) : PKV_SPLIT64(0, false);
-        return td.pbits == 3 ? PKV_SPLIT64(3, true) : PKV_SPLIT64(0, true);
+        if (lc.own_status) {
+            if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT64(3, false, true) : PKV_SPLIT64(0, false, true);
+            return td.pbits == 3 ? PKV_SPLIT64(3, true, true) : PKV_SPLIT64(0, true, true);
+        }
+        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT64(3, false, false) : PKV_SPLIT64(0, false, false);
+        return td.pbits == 3 ? PKV_SPLIT64(3, true, false) : PKV_SPLIT64(0, true, false);
 #undef PKV_SPLIT64
     }
     if (td.dim == 128 && td.pbits <= 4) {
         if (nblocks > (1u << 29)) return hipErrorInvalidValue;   // 4 workgroups per tile
         const size_t lds = static_cast<size_t>(WAVES) * turbo_split128_wave_words(lc.plen >> 2) * sizeof(uint32_t);
-#define PKV_SPLIT128(PB, LO)                                                                            \
-    launch_big_lds(turbo_decode_split128_kernel<PB, LO>, 4 * nblocks, lds, st, lc, wire, out, td.signs, \
+#define PKV_SPLIT128(PB, LO, OW)                                                                            \
+    launch_big_lds(turbo_decode_split128_kernel<PB, LO, OW>, 4 * nblocks, lds, st, lc, wire, out, td.signs, \
                    td.cs, td.seed, td.pbits, td.proj)
-        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT128(3, false) : PKV_SPLIT128(0, false);
-        return td.pbits == 3 ? PKV_SPLIT128(3, true) : PKV_SPLIT128(0, true);
+        if (lc.own_status) {
+            if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT128(3, false, true) : PKV_SPLIT128(0, false, true);
+            return td.pbits == 3 ? PKV_SPLIT128(3, true, true) : PKV_SPLIT128(0, true, true);
+        }
+        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT128(3, false, false) : PKV_SPLIT128(0, false, false);
+        return td.pbits == 3 ? PKV_SPLIT128(3, true, false) : PKV_SPLIT128(0, true, false);
 #undef PKV_SPLIT128
     }
     if (td.dim == 64)

@@ -94,3 +94,61 @@ def test_blob_order_and_overlap(ctx):
     for offsets in ([0, blob - 1, 2 * blob, 3 * blob], [3 * blob, 0, 2 * blob, 2 * blob + 1], [0, blob, 0, 2 * blob]):
         with pytest.raises(L.PkvError):
             encode(offsets)
+
+
+@pytest.mark.parametrize("dim,bits", [(64, 4), (64, 2), (128, 4), (128, 8)])
+@pytest.mark.parametrize("radii", [0, 1])
+@pytest.mark.parametrize("sizes,cap", [([1, 64, 3], 0), ([64, 2, 65], 0), ([128, 5, 1], 0), ([129, 2, 3], 0),
+                                       ([2, 70, 1], 0), ([3, 128, 2, 64], 3)])
+def test_words_stored_by_the_owning_workgroup(ctx, dim, bits, radii, sizes, cap):
+    """Calls whose segments each fall to one workgroup store the words themselves,
+    over stale ones; a call after an explicit clear marks them in memory.  Both report
+    the same failures, at the first and last vectors and in the header."""
+    import torch
+    from provekv_amd.device import segments
+    prof = ctx.turbo_profile(dim, bits, 32, 42)
+    rows, off, elem = [], 0, 0
+    for n in sizes:
+        rows.append((elem, 0, dim, off, n, max(n, 1)))
+        off += prof.blob_len(n, radii) + 3
+        elem += n * dim
+    segs = segments(rows)
+    nseg = len(sizes)
+    x = np.random.RandomState(dim).randn(elem).astype(np.float32)
+    bad = x.copy()
+    bad[rows[0][0] + (sizes[0] - 1) * dim + dim - 1] = np.nan          # last vector of the first segment
+    bad[rows[-1][0]] = np.inf                                          # first of the last segment
+    wire = torch.zeros(off, dtype=torch.uint8, device="cuda")
+    out = torch.zeros(elem, device="cuda")
+
+    def both(call):
+        own = torch.zeros(2 * nseg, dtype=torch.int32, device="cuda")  # stale: a failure at vector 0
+        ref = torch.zeros_like(own)
+        call(own, False)
+        ctx.clear_status([(ref, nseg)])
+        call(ref, True)
+        own, ref = (s.cpu().numpy().view(np.uint32).reshape(-1, 2) for s in (own, ref))
+        assert np.array_equal(own, ref)
+        return own
+
+    def encode(v):
+        t = torch.from_numpy(v).cuda()
+        return both(lambda st, cl: prof.encode_segments(t, segs, wire, radii=radii, status=st, status_cleared=cl))
+
+    def decode(w):
+        return both(lambda st, cl: prof.decode_segments(w, segs, out, radii=radii, status=st, status_cleared=cl,
+                                                        max_workgroups=cap))
+    st = encode(bad)
+    assert (st[0, 1] >> 4, st[-1, 1] >> 4) == (sizes[0] - 1, 0)
+    assert (st[1:-1] == 0xFFFFFFFF).all() and (st[:, 0] == 0xFFFFFFFF).all()
+    assert (encode(x) == 0xFFFFFFFF).all()
+    assert (decode(wire) == 0xFFFFFFFF).all()
+    w = wire.clone()
+    w[rows[-1][3]] ^= 1                                                # header of the last segment
+    plen = (prof.blob_len(2, radii) - prof.blob_len(1, radii))
+    rw = dim // 2 if radii else 0                                      # the first radius, or the radii's minimum
+    at = rows[0][3] + 38 + (sizes[0] - 1) * plen + rw
+    w[at:at + 4] = torch.tensor([0, 0, 0xC0, 0x7F], dtype=torch.uint8, device="cuda")   # NaN
+    st = decode(w)
+    assert st[-1, 0] >> 4 == 0 and st[-1, 0] != 0xFFFFFFFF
+    assert st[0, 1] >> 4 == sizes[0] - 1 and st[0, 0] == 0xFFFFFFFF
