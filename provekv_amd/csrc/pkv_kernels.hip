@@ -699,20 +699,18 @@ __device__ __forceinline__ void signs_stage1(float (&v)[32], const float (&sg)[3
 // The hardware log2 times ln 2 rounded to f32: within g_logb of logf.
 __device__ __forceinline__ float cheap_logf(float v) { return __builtin_amdgcn_logf(v) * 0x1.62e430p-1f; }
 
-// Correctly rounded sqrt of x >= 2^-96, +0, +inf or NaN: the hardware root s
-// (v_sqrt_f32, within 1 ulp) moved to a neighbour s -+ 1 ulp when the exact
-// remainder fma(-s', s, x) shows the root lies past the midpoint -- the
-// fix-up of the compiler's own f32 sqrt expansion, without the rescaling it
-// applies below 2^-96 or the +-0 / +inf select, which this fix-up already
-// gets right (+0: the neighbours' remainders are NaN and -0; +inf: NaN).
-// Below 2^-96 (callers route such inputs to __builtin_sqrtf) the remainder
-// may underflow.
+// Correctly rounded sqrt of a finite x >= 2^-96: g = x y from the hardware
+// 1 / sqrt (v_rsq_f32), then one Newton step g + (x - g^2) (y / 2) with the
+// remainder and the sum in single fmas.  sqrt_check_kernel compares it with
+// __builtin_sqrtf on every float of the domain before a context is created.
+// Five instructions per radius; the two-neighbour fix-up of v_sqrt_f32 took
+// nine: with radii_bins' single fma per octant test and the hardware root in
+// qjl_norm_bound, 4.2 M head_dim-128 bf16 vectors encode in 876 us (888), 2.1 M
+// head_dim-64 in 416 (422).  +0 and +inf give NaN: callers replace those.
 __device__ __forceinline__ float sqrt_normal(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sd = u2f(f2u(s) - 1u), su = u2f(f2u(s) + 1u);
-    float r = __builtin_fmaf(-sd, s, x) <= 0.0f ? sd : s;
-    r = __builtin_fmaf(-su, s, x) > 0.0f ? su : r;
-    return r;
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
 }
 
 // CompressedRadiiV1 BlockLogU8 (turbo-quant/src/radius.rs:58-77) of one
@@ -815,19 +813,24 @@ __device__ __forceinline__ void block_log_u8(const float (&r)[16], int part, con
 
 // Radii and angle bins (polar.rs:246-266, 413-421) of a lane's 16 pairs
 // (y[2i], y[2i + 1]): r[i] = sqrt(fl(a^2) + fl(b^2)), the bins pbits apart
-// in pk, rsum the lane's radius sum (its finiteness stands for every radius
-// and input element).  At pbits = 3 a pair octant_bin_f passes takes the
-// octant's bin and sqrt_normal's radius (its fl(a^2) + fl(b^2) >= 2^-94);
+// in pk, zsum the lane's sum of fl(a^2) + fl(b^2) (finite only when every
+// radius and input element is).  PRE8: y is the rotated vector before its
+// scale of 2^-3; every fast-path operation commutes with it, so only the
+// radius is scaled, one multiply instead of two.  At pbits = 3 a pair
+// octant_bin_f passes takes the octant's bin and sqrt_normal's radius (its fl(a^2) + fl(b^2) >= 2^-94);
 // the other pairs -- near an octant line or outside the covered range, every
-// pair of a lane whose radius sum is not finite, every pair at other widths
+// pair of a lane whose zsum is not finite, every pair at other widths
 // -- take angle_bin_exact and __builtin_sqrtf.  Every lane of the wave must
 // call it.
-template <int PB>
+template <int PB, bool PRE8>
 __device__ __forceinline__ void radii_bins(const float (&y)[32], uint32_t pbits, float (&r)[16], uint64_t& pk,
-                                           float& rsum) {
+                                           float& zsum) {
     constexpr int HP = 16;
-    uint64_t any_unsafe = 0;   // the wave's lanes with a pair that needs the exact formulas
-    rsum = 0.0f;
+    constexpr float pre = PRE8 ? 0.125f : 1.0f;
+    // the least of octant_bin_f's test differences (NaN only beside a zsum
+    // that is not finite); a pair needs the exact formulas when it is not positive
+    float least = u2f(0x7f800000u);
+    zsum = 0.0f;
     pk = 0;
     // octant_bin_f's bins, bit by bit: each pair shifts the sign bits of g,
     // a ^ b and b into a shift register (v_alignbit), ascending bit order,
@@ -840,23 +843,25 @@ __device__ __forceinline__ void radii_bins(const float (&y)[32], uint32_t pbits,
     for (int i = 0; i < HP; ++i) {
         const float a = y[2 * i], b = y[2 * i + 1];
         const float aa = a * a, bb = b * b;
-        r[i] = sqrt_normal(aa + bb);
-        rsum = rsum + r[i];
-        bool uns = true;
+        const float z = aa + bb;
+        zsum = zsum + z;
         if constexpr (PB == 3) {
+            r[i] = PRE8 ? sqrt_normal(z) * pre : sqrt_normal(z);
             const float fa = __builtin_fabsf(a), fb = __builtin_fabsf(b);
             const float g = fa - fb;
-            const float mx = __builtin_fmaxf(__builtin_fmaxf(fa, fb), 0x1p-31f);
+            const float mx = __builtin_fmaxf(__builtin_fmaxf(fa, fb), 0x1p-31f / pre);
             const float m3 = __builtin_fminf(__builtin_fminf(fa, fb), __builtin_fabsf(g));
-            uns = !(mx < m3 * 65536.0f);   // octant_bin_f's test
+            // octant_bin_f's test mx < m3 * 2^16 (one fma has its sign)
+            least = __builtin_fminf(least, __builtin_fmaf(m3, 65536.0f, -mx));
             const uint32_t src[3] = {f2u(g), f2u(a) ^ f2u(b), f2u(b)};
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 if (3 * i + k < 32) w0 = __builtin_amdgcn_alignbit(w0, src[k], 31);
                 else w1 = __builtin_amdgcn_alignbit(w1, src[k], 31);
             }
+        } else {
+            r[i] = 0.0f;   // replaced below
         }
-        any_unsafe |= __ballot(uns);
     }
     if constexpr (PB == 3) {
         w0 = __builtin_bitreverse32(w0);
@@ -865,16 +870,15 @@ __device__ __forceinline__ void radii_bins(const float (&y)[32], uint32_t pbits,
         w1 ^= ((w1 >> 1) & 0x2492u) ^ 0x9249u;           // the same fields, one bit up (pair 10 straddles)
         pk = (static_cast<uint64_t>(w1) << 32) | w0;
     }
-    const bool force = !isfinite_f(rsum);
-    any_unsafe |= __ballot(force);
-    if (any_unsafe) {
-        // this lane's pairs again (the fast loop keeps only the wave's OR)
+    const bool force = PB != 3 || !isfinite_f(zsum);
+    if (__ballot(force || !(least > 0.0f))) {
+        // this lane's pairs again (the fast loop keeps only the least difference)
         const uint32_t levels = 1u << pbits;
         uint32_t slow = force ? 0xffffu : 0u;
 #pragma unroll
         for (int i = 0; i < HP; ++i) {
             bool uns = true;
-            if constexpr (PB == 3) (void)octant_bin_f(y[2 * i], y[2 * i + 1], uns);
+            if constexpr (PB == 3) (void)octant_bin_f(y[2 * i] * pre, y[2 * i + 1] * pre, uns);
             slow |= (uns ? 1u : 0u) << i;
         }
         for (uint32_t m = slow; m; m &= m - 1u) {
@@ -886,6 +890,8 @@ __device__ __forceinline__ void radii_bins(const float (&y)[32], uint32_t pbits,
                 a = static_cast<uint32_t>(j) == i ? y[2 * j] : a;
                 b = static_cast<uint32_t>(j) == i ? y[2 * j + 1] : b;
             }
+            a *= pre;
+            b *= pre;
             const uint64_t bin = angle_bin_exact(a, b, pbits);
             pk = (pk & ~(static_cast<uint64_t>(levels - 1u) << (i * pbits))) | (bin << (i * pbits));
             const float aa = a * a, bb = b * b;
@@ -922,12 +928,14 @@ __device__ __forceinline__ v4f mfma16x32(const v4u& a, const v4u& b, const v4f& 
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
 }
 
-// |res| rounded up: rn2 is the f32 sum of the squares (one fma each, then
+// |res| rounded up, from the hardware root (sqrt_check_kernel: within 2^-20 of
+// the exact one on every normal float).  rn2 is the f32 sum of the squares (one fma each, then
 // the lanes' partial sums added), within (1 + 35u) rn2 + 2^-144 of the exact
 // one (relative roundings while normal, at most 2^-150 each while subnormal),
-// so |res| <= sqrt(rn2) (1 + 19u) + 2^-72, which 1.0001 and 2^-70 cover.
+// so |res| <= sqrt(rn2) (1 + 19u) + 2^-72 <= s (1 + 2^-20)(1 + 19u) + 2^-72 for
+// the root s of max(rn2, 2^-126), which 1.0001 and 2^-70 cover.
 __device__ __forceinline__ float qjl_norm_bound(float rn2) {
-    return __builtin_fmaf(__builtin_sqrtf(rn2), 1.0001f, 0x1p-70f);
+    return __builtin_fmaf(__builtin_amdgcn_sqrtf(rn2 < 0x1p-126f ? 0x1p-126f : rn2), 1.0001f, 0x1p-70f);
 }
 
 // 2^(14 - e) for the exponent e of rn >= |res| (clamped to [-60, 127]): every
@@ -1058,9 +1066,7 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
             lds_half(sg_lds, sg);
             signs_stage1(y, sg);
         }
-        fwht_split<2>(y, h);
-#pragma unroll
-        for (int c = 0; c < 32; ++c) y[c] *= scale;
+        fwht_split<2>(y, h);   // the scale of 2^-3 is left to radii_bins
 
         // zero this vector's angle index words: both halves OR into them
         if (h == 0 && active)
@@ -1069,15 +1075,15 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
 
         // radii and angle bins (polar.rs:246-266, 413-421) of pairs 16h + i
         float r[HP];
-        float rsum;
+        float zsum;
         uint64_t pk;
-        radii_bins<PB>(y, pbits, r, pk, rsum);
+        radii_bins<PB, true>(y, pbits, r, pk, zsum);
         // A non-finite input makes every FWHT output, so every radius,
-        // non-finite; a finite sum of the (non-negative) radii therefore
+        // non-finite; a finite sum of the (non-negative) squares therefore
         // clears both checks.  Otherwise (or on an overflowing sum) they run
         // element by element.
         bool finite = true, rfinite = true;
-        if (!isfinite_f(rsum)) {
+        if (!isfinite_f(zsum)) {
             float x[32];
             load_half(x);
 #pragma unroll
@@ -1534,15 +1540,15 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl128_kernel(
         // radii and angle bins (polar.rs:246-266, 413-421) of pairs 8q + i
         // (i < 8) and 32 + 8q + i - 8 (layout F)
         float r[HP];
-        float rsum;
+        float zsum;
         uint64_t pk;
-        radii_bins<PB>(y, pbits, r, pk, rsum);
+        radii_bins<PB, false>(y, pbits, r, pk, zsum);
         // A non-finite input makes every FWHT output, so every radius,
-        // non-finite; a finite sum of the (non-negative) radii therefore
+        // non-finite; a finite sum of the (non-negative) squares therefore
         // clears both checks.  Otherwise (or on an overflowing sum) they run
         // element by element.
         bool finite = true, rfinite = true;
-        if (!isfinite_f(rsum)) {
+        if (!isfinite_f(zsum)) {
             float x[32];
             load_x(x, q0, q0 + 16);
 #pragma unroll
@@ -3795,20 +3801,21 @@ __global__ void f16_subnormal_probe_kernel(float* out) {
     }
 }
 
-// sqrt_normal against __builtin_sqrtf on every float it is used on (2^-96 ..
-// +inf) and on +0 and NaN; *bad counts the disagreements.
-constexpr uint32_t kSqrtLo = 0x0f800000u, kSqrtHi = 0x7f800001u;
+// sqrt_normal against __builtin_sqrtf on every float it is used on (finite,
+// from 2^-96), and the hardware root qjl_norm_bound takes, within 2^-20 of it
+// on every normal float; *bad counts the disagreements.
+constexpr uint32_t kRootLo = 0x00800000u, kSqrtLo = 0x0f800000u, kSqrtHi = 0x7f800000u;
 
 __global__ __launch_bounds__(256) void sqrt_check_kernel(uint32_t per, uint32_t* bad) {
     const uint64_t t = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-    const uint64_t b0 = kSqrtLo + t * per;
+    const uint64_t b0 = kRootLo + t * per;
     const uint32_t u0 = static_cast<uint32_t>(b0 < kSqrtHi ? b0 : kSqrtHi);
     const uint32_t u1 = static_cast<uint32_t>(b0 + per < kSqrtHi ? b0 + per : kSqrtHi);
     uint32_t n = 0;
-    for (uint32_t u = u0; u < u1; ++u) n += f2u(sqrt_normal(u2f(u))) != f2u(__builtin_sqrtf(u2f(u))) ? 1u : 0u;
-    if (t == 0) {
-        n += f2u(sqrt_normal(0.0f)) != 0u ? 1u : 0u;
-        n += isfinite_f(sqrt_normal(u2f(0x7fc00000u))) || (f2u(sqrt_normal(u2f(0x7fc00000u))) & 0x7fffffu) == 0u ? 1u : 0u;
+    for (uint32_t u = u0; u < u1; ++u) {
+        const float x = u2f(u), s = __builtin_sqrtf(x);
+        n += u >= kSqrtLo && f2u(sqrt_normal(x)) != f2u(s) ? 1u : 0u;
+        n += !(__builtin_fabsf(__builtin_amdgcn_sqrtf(x) - s) < s * 0x1p-20f) ? 1u : 0u;
     }
     if (n) atomicAdd(bad, n);
 }
@@ -3851,7 +3858,7 @@ int launch_f16_subnormal_probe(float* out, void* stream) {
 int launch_sqrt_check(uint32_t* bad, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     constexpr uint64_t threads = static_cast<uint64_t>(kLogbBlocks) * 256;
-    const uint32_t per = static_cast<uint32_t>((static_cast<uint64_t>(kSqrtHi - kSqrtLo) + threads - 1) / threads);
+    const uint32_t per = static_cast<uint32_t>((static_cast<uint64_t>(kSqrtHi - kRootLo) + threads - 1) / threads);
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, bad, 0u, static_cast<uint64_t>(1));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
