@@ -367,7 +367,7 @@ def bench_config0(args):
         args, name="config0", prof=prof, radii=L.RADII_F32, inp=inp, segs=segs, wire=wire, out=out,
         metric="KV codec encode+decode GB/s (f32 in) and % HBM peak, config 0 (single-layer turbo b=4 round trip)",
         f32_bytes=x.nbytes, enc_alg=x.nbytes + 2 * blob, dec_alg=2 * blob + x.nbytes,
-        kernels=("turbo_encode_qjl_kernel<3, false>", "turbo_decode_split_kernel<3>"),
+        kernels=("turbo_encode_qjl_kernel<3, false, false>", "turbo_decode_split_kernel<3, false, false>"),
         summary="codec_kernels_config0.md",
         parity=lambda: _blob_parity(prof, wire, out, segs, lambda b: xs[b], [0, 1],
                                     lambda v: O.turbo_encode_batch(v, SEED, signs=signs, G=G),
@@ -418,7 +418,7 @@ def bench_config1(args):
         args, name="config1", prof=Prof, radii=L.RADII_F32, inp=inp, segs=tier.dec, wire=wire, out=out,
         metric="KV codec encode+decode GB/s (f32 in) and % HBM peak, config 1 (fib_k4_n32 cold pool)",
         f32_bytes=f32, enc_alg=f32 + tier.wire_bytes, dec_alg=tier.wire_bytes + f32,
-        kernels=("fib_encode_kernel<64, false>", "fib_decode_mfma_kernel<64, false>"),
+        kernels=("fib_encode_kernel<64, false>", "fib_decode_mfma_kernel<64, false, true>"),
         summary="codec_kernels_config1.md",
         parity=lambda: _blob_parity(prof, wire, out, tier.dec, blob_in, [0, 1, 23, 46, 47],
                                     lambda v: O.fib_encode_batch(v, cb, rot),
@@ -475,7 +475,8 @@ def bench_config2(args):
             segs=tier.dec, wire=wire, out=out,
             metric="KV codec encode+decode GB/s (f32 in) and % HBM peak, config 2 (N=8 turbo b=4 shells)",
             f32_bytes=f32, enc_alg=f32 + tier.wire_bytes, dec_alg=tier.wire_bytes + f32,
-            kernels=("turbo_encode_qjl_kernel<3, false>", "turbo_decode_split_kernel<3>"),
+            kernels=("turbo_encode_qjl_kernel<3, false, false>",
+                     f"turbo_decode_split_kernel<3, {'true' if lossy else 'false'}, false>"),
             summary="codec_kernels_config2.md", tag=" [lossy]" if lossy else " [lossless]",
             parity=lambda prof=prof, wire=wire, out=out, tier=tier, blob_in=blob_in, rc=rc: _blob_parity(
                 prof, wire, out, tier.dec, blob_in, [0, 1, 191, 383],
@@ -541,7 +542,7 @@ def bench_config4(args):
         args, name="config4", prof=prof, radii=rc, inp=flat, segs=segs, wire=wire, out=out,
         metric="KV codec encode+decode GB/s (f32-equivalent KV) and % HBM peak, config 4 (Llama-3-8B shape)",
         f32_bytes=f32, enc_alg=nb * n * dim * 2 + wire.numel(), dec_alg=wire.numel() + f32,
-        kernels=("turbo_encode_qjl128_kernel<3, false>", "turbo_decode_split128_kernel<3>"),
+        kernels=("turbo_encode_qjl128_kernel<3, false, false>", "turbo_decode_split128_kernel<3, true, false>"),
         summary="codec_kernels_config4.md", parity=parity,
         cpu=lambda: cpu_baseline(jobs, jb, f32, "config 4, the first 8192 vectors of each of the 64 blobs "
                                  "(f32 upcast of the bf16 input)", budget_s=10.0),
@@ -586,10 +587,12 @@ def bench_config3(args):
     from provekv_amd.device import default_context
     from provekv_amd.pool import DeviceKVCache, TwoTierPlan
     need_gpu()
-    kernel = {"fib_encode": "fib_encode_kernel<64, false>", "turbo_encode": "turbo_encode_qjl_kernel<3, false>",
-              "fib_decode": "fib_decode_mfma_kernel<64, true>" if args.copies > 1 else
-                            "fib_decode_mfma_kernel<64, false>",
-              "turbo_decode": "turbo_decode_split_kernel<3>"}
+    kernel = {"fib_encode": "fib_encode_kernel<64, false>", "turbo_encode": "turbo_encode_qjl_kernel<3, false, false>",
+              "fib_decode": "fib_decode_mfma_kernel<64, false, true>" if args.copies == 1 else
+                            "fib_decode_mfma_kernel<64, true, true>"
+                            if args.copies <= (3 if args.cache_dtype == "f32" else 6) else
+                            "fib_decode_mfma_kernel<64, true, false>",
+              "turbo_decode": f"turbo_decode_split_kernel<3, {'true' if args.lossy else 'false'}, false>"}
     layers, heads, dim, prefix, agents = 24, 32, 64, 800, [28] * 8
     log(f"[bench] generating synthetic corpus ({prefix + sum(agents)} tokens x {layers}L x {heads}H x 2 x {dim})")
     corpus = synth.corpus_tokens(3, layers, heads, prefix + sum(agents), dim)
@@ -1066,7 +1069,7 @@ def bench_digest(args):
            "workload": "digest", "unit": "GB/s", "steps": args.steps, "warmup": args.warmup,
            "parity_all_digests": bool(parity),
            "config3": {"ranges": len(plan.pool.blob_offsets) + len(plan.shells.blob_offsets),
-                       "tiers": "one stream" if side is None else "pool and shell tiers on two streams",
+                       "tiers": "one stream" if side is None else "both tiers in one call",
                        "bytes": int(wire_bytes), "ms_per_call": round(ms, 4),
                        "gbs": round(wire_bytes / (ms * 1e-3) / 1e9, 1), "roofline": valu(wire_bytes, ms)},
            "bulk_512x1MiB": {"bytes": bulk_bytes, "ms_per_call": round(bms, 4),

@@ -1327,46 +1327,6 @@ __global__ __launch_bounds__(TILE) void turbo_encode_qjl_kernel(
 // The undecided dots are recomputed in the reference's order, block by block,
 // each block's holder continuing the previous block's sum.
 
-// Value of lane l ^ 16 (the other quarter of the same half).
-// fwht_normalized stages (turbo-quant/src/rotation.rs:379-398) on a 128-wide
-// vector split over four lanes, 32 elements per lane.
-template <int FIRST = 1>
-__device__ __forceinline__ void fwht_quarter(float (&v)[32], int q) {
-#pragma unroll
-    for (int step = FIRST; step < 32; step *= 2) {
-#pragma unroll
-        for (int start = 0; start < 32; start += 2 * step) {
-#pragma unroll
-            for (int off = 0; off < step; ++off) {
-                const float a = v[start + off], b = v[start + off + step];
-                v[start + off] = a + b;
-                v[start + off + step] = a - b;
-            }
-        }
-    }
-    // step 32: element c of quarter 2k with c of quarter 2k + 1: (a + b, a - b);
-    // step 64: quarters 0, 1 with 2, 3.  On element pairs (c, c + 16): a
-    // v_permlane16_swap of v[c], v[c + 16] leaves step 32's (a, b) of element
-    // c in the even rows and of element c + 16 in the odd rows, and every lane
-    // forms a + b, a - b; a v_permlane32_swap of those two then holds step 64's
-    // (a, b) -- quarters 0 / 2 in rows 0, 1, quarters 1 / 3 in rows 2, 3 -- for
-    // the same a + b, a - b; the two swaps in reverse order return every
-    // result to its quarter and element.
-    (void)q;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-        auto p = __builtin_amdgcn_permlane16_swap(f2u(v[c]), f2u(v[c + 16]), false, false);
-        float a = u2f(p[0]), b = u2f(p[1]);
-        p = __builtin_amdgcn_permlane32_swap(f2u(a + b), f2u(a - b), false, false);
-        a = u2f(p[0]);
-        b = u2f(p[1]);
-        p = __builtin_amdgcn_permlane32_swap(f2u(a + b), f2u(a - b), false, false);
-        p = __builtin_amdgcn_permlane16_swap(p[0], p[1], false, false);
-        v[c] = u2f(p[0]);
-        v[c + 16] = u2f(p[1]);
-    }
-}
-
 // Stages 2..64 of fwht_normalized on the standard layout (element 32q + c in
 // v[c]; stage 1 already applied), ending in layout F.  Per c: a
 // v_permlane16_swap of v[c], v[c + 16] gives each row the stage-32 pair
