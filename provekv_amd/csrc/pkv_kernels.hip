@@ -98,7 +98,7 @@ __device__ __forceinline__ uint32_t lds_byte(const uint32_t* lds, uint32_t off) 
 // memory at any byte alignment, 16 bytes per lane and store; the last store of a
 // range of at least 16 bytes starts early enough to end with it (bytes stored
 // twice get the same value).  Dword stores shifted into place by v_alignbyte
-// cost the encodes 2 to 5 %: config-2 shells, f32 radii,
+// cost the encodes 2 to 5 %: 344 k head_dim-64 vectors, f32 radii,
 // 52.2 -> 49.5 us; 4.2 M head_dim-128 vectors 905 -> 884 us.
 typedef uint32_t v4u_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ void lds_to_global(uint8_t* __restrict__ dst, const uint32_t* lds, uint32_t nbytes,
@@ -229,8 +229,9 @@ __device__ void stage_rows_in(float* stage, const void* __restrict__ in, bool bf
 // Two f32 -> bfloat16 bits, round to nearest even (torch's / c10's conversion;
 // a NaN keeps its upper bits and turns quiet): one v_cvt_pk_bf16_f32, equal to
 // the integer rounding it replaces on every float, where that took six
-// operations a value (config-3 step into one bf16 cache 404 -> 364 us, with the
-// other changes to its decodes; the shells' decode into one 36 -> 32 us).
+// operations a value (a step of 1.2 M pool and 0.34 M shell vectors
+// into one bf16 cache 404 -> 364 us, with the other changes to its decodes; the
+// shells' decode into one 36 -> 32 us).
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
@@ -4076,9 +4077,9 @@ int launch_fib_decode(const LaunchCommon& lc, const FibDev& fd, const uint8_t* w
     if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 half-tiles per tile
     // The table of partial sums pays while the arithmetic is the bound; past
     // 12 output bytes per value the decode is bound by its writes and the
-    // table's reads slow them down (config-3 step, table against none: 2 f32
-    // copies 425 / 439 us, 3 474 / 476, 4 527 / 520, 8 798 / 778; 4 bf16 copies
-    // 441 / 460, 8 544 / 527).
+    // table's reads slow them down (a step of 1.2 M pool and 0.34 M shell
+    // vectors, table against none: 2 f32 copies 425 / 439 us, 3 474 / 476, 4
+    // 527 / 520, 8 798 / 778; 4 bf16 copies 441 / 460, 8 544 / 527).
     const bool table = lc.fanout <= (lc.out_dtype == PKV_F32 ? 3u : 6u);
     auto kern = lc.fanout == 1 ? fib_decode_mfma_kernel<64, false, true>
                 : table        ? fib_decode_mfma_kernel<64, true, true>
