@@ -326,8 +326,10 @@ class TwoTierPlan:
         library call and one launch sequence for both tiers (payload passes,
         the last of them with the layer digests), on the calling stream: tiers
         apart on two streams spent longer on the two cross-stream waits than
-        they saved.  Work queued on a `side` stream before the call comes
-        before the digests."""
+        they saved.  With a `side` stream the call is ordered on both sides
+        with it: work queued on `side` before the call comes before the
+        digests, work queued there afterwards (the next shell encode into the
+        same wire, a read of the digests) after them."""
         import torch
         main = stream if stream is not None else torch.cuda.current_stream()
         if side is not None:
@@ -348,6 +350,8 @@ class TwoTierPlan:
                 ranges = tier.ranges = np.array([(off, ln) for _, _, _, off, ln in tier.blob_offsets], np.uint64)
             tiers.append((bufs[f"{name}_wire"], ranges, bufs[f"{name}_digests"], bufs[f"{name}_layer_digests"]))
         self.ctx.build_digests(tiers, self.layers, main)
+        if side is not None:   # an event of its own per call: threads may share the plan
+            side.wait_stream(main)
 
     def digest_report(self, bufs) -> dict:
         """The digests of the last digests() call as the reference prints them

@@ -1,0 +1,103 @@
+"""The order TwoTierPlan's calls leave between the calling stream and a `side`
+stream, on the CPU: streams and events that only record what each queued
+operation comes after."""
+import contextlib
+
+import pytest
+import torch
+
+from provekv_amd.pool import TwoTierPlan
+
+
+class Event:
+    after = frozenset()
+
+    def record(self, stream):
+        self.after = stream.after
+
+
+class Stream:
+    """A queue whose operations come after everything in `after`."""
+
+    def __init__(self, capturing=False, idle=False):
+        self.after, self.capturing, self.idle = frozenset(), capturing, idle
+
+    def run(self, name):
+        before, self.after = self.after, self.after | {name}
+        return before
+
+    def record_event(self):
+        ev = Event()
+        ev.record(self)
+        return ev
+
+    def wait_event(self, event):
+        self.after = self.after | event.after
+
+    def wait_stream(self, other):
+        self.wait_event(other.record_event())
+
+    def query(self):
+        assert not self.capturing, "a query invalidates a capture"
+        return self.idle
+
+
+class Profile:
+    def __init__(self, ctx, name):
+        self.ctx, self.name = ctx, name
+
+    def payload_len(self, radii=0):
+        return 12
+
+    def encode_segments(self, *a, stream=None, **kw):
+        self.ctx.log[f"{self.name} encode"] = stream.run(f"{self.name} encode")
+
+    def decode_segments(self, *a, stream=None, **kw):
+        self.ctx.log[f"{self.name} decode"] = stream.run(f"{self.name} decode")
+
+
+class Context:
+    def __init__(self):
+        self.log = {}
+
+    def fib_profile(self, *a):
+        return Profile(self, "pool")
+
+    def turbo_profile(self, *a):
+        return Profile(self, "shells")
+
+    def build_digests(self, tiers, layers, stream):
+        self.log["digests"] = stream.run("digests")
+
+
+@pytest.fixture
+def plan(monkeypatch):
+    current = [Stream()]
+
+    @contextlib.contextmanager
+    def use(stream):
+        current.append(stream)
+        yield
+        current.pop()
+
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "stream", use)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: current[-1])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[-1].capturing)
+    return TwoTierPlan(Context(), 2, 3, 64, 20, [3, 2])
+
+
+@pytest.mark.parametrize("idle", [False, True])
+@pytest.mark.parametrize("capturing", [False, True])
+def test_digests_come_between_the_side_streams_work(plan, idle, capturing):
+    """What was queued on `side` before the call comes before the digests, what
+    is queued there afterwards (the next encode into the hashed wire) after."""
+    bufs = plan.alloc("cpu")
+    main, side = torch.cuda.current_stream(), Stream(idle=idle)
+    main.capturing = capturing
+    if not idle:
+        side.run("encode before")
+    plan.digests(bufs, side=side)
+    assert idle or "encode before" in plan.ctx.log["digests"]
+    assert "digests" in side.run("encode after")
+    assert "digests" in main.run("next call")
