@@ -333,7 +333,12 @@ class TwoTierPlan:
         import torch
         main = stream if stream is not None else torch.cuda.current_stream()
         if side is not None:
-            if torch.cuda.is_current_stream_capturing():   # side may join a capture only by a fork from it
+            if stream is None:
+                capturing = torch.cuda.is_current_stream_capturing()
+            else:
+                with torch.cuda.stream(main):
+                    capturing = torch.cuda.is_current_stream_capturing()
+            if capturing:   # side may join a capture only by a fork from it
                 side.wait_stream(main)
                 main.wait_stream(side)
             elif not side.query():

@@ -101,3 +101,17 @@ def test_digests_come_between_the_side_streams_work(plan, idle, capturing):
     assert idle or "encode before" in plan.ctx.log["digests"]
     assert "digests" in side.run("encode after")
     assert "digests" in main.run("next call")
+
+
+@pytest.mark.parametrize("joined", [False, True])
+def test_digests_on_an_explicit_capturing_stream(plan, joined):
+    """The calling stream, not the current one, decides whether the call is part
+    of a capture: `side` is then forked from it and never queried."""
+    bufs = plan.alloc("cpu")
+    main, side = Stream(capturing=True), Stream(capturing=joined)
+    main.run("capture begins")
+    waited = []
+    side.wait_stream = lambda other: (waited.append(other), Stream.wait_stream(side, other))
+    plan.digests(bufs, stream=main, side=side)
+    assert waited == [main, main]   # the fork, then the order after the digests
+    assert "capture begins" in side.after and "digests" in side.after
