@@ -243,7 +243,10 @@ class TwoTierPlan:
         import torch
         main = stream if stream is not None else torch.cuda.current_stream()
         self._cache_tables(bufs, cache)
-        self._clear(bufs, ("pool_status", "shell_status", "pool_cstatus", "shell_cstatus"), main)
+        # with `side`, the shell rehydrate clears its own words there: a read of
+        # them that side still has queued comes first
+        on_main = ("pool_status", "shell_status", "pool_cstatus", "shell_cstatus")
+        self._clear(bufs, on_main if side is None else on_main[:3], main)
         if side is None:
             self._encode_pool(corpus, bufs, main)
             self._encode_shells(corpus, bufs, main)
@@ -254,7 +257,7 @@ class TwoTierPlan:
         self._encode_shells(corpus, bufs, main)
         shells_encoded.record(main)
         side.wait_event(shells_encoded)
-        self._rehydrate_tier("shells", bufs, cache, side, max_workgroups=side_workgroups)
+        self._rehydrate_tier("shells", bufs, cache, side, max_workgroups=side_workgroups, cleared=False)
         self._encode_pool(corpus, bufs, main, max_workgroups=pool_workgroups)
         self._rehydrate_tier("pool", bufs, cache, main)
         join.record(side)
@@ -281,18 +284,20 @@ class TwoTierPlan:
             if name not in bufs:
                 bufs[name] = torch.empty(2 * n, dtype=torch.int32, device=cache.buf.device)
 
-    def _rehydrate_tier(self, tier: str, bufs, cache: DeviceKVCache, stream, max_workgroups: int = 0):
-        """One tier into `cache` (its status words cleared before)."""
+    def _rehydrate_tier(self, tier: str, bufs, cache: DeviceKVCache, stream, max_workgroups: int = 0,
+                        cleared: bool = True):
+        """One tier into `cache` (cleared: its status words were, earlier in
+        stream order)."""
         pseg, sseg = self._cache_segs
         out = cache.buf.view(-1)
         if tier == "pool":
             self.fib.decode_segments(bufs["pool_wire"], pseg, out, status=bufs["pool_cstatus"], stream=stream,
-                                     fanout=cache.copies, fanout_stride=cache.copy_stride, status_cleared=True)
+                                     fanout=cache.copies, fanout_stride=cache.copy_stride, status_cleared=cleared)
         else:
             self.turbo.decode_segments(bufs["shell_wire"], sseg, out, radii=self.radii,
                                        status=bufs["shell_cstatus"], stream=stream, fanout=cache.copies,
                                        fanout_stride=cache.copy_stride, max_workgroups=max_workgroups,
-                                       status_cleared=True)
+                                       status_cleared=cleared)
             cache.mark_filled(self.tokens)
 
     def check_rehydrate(self, bufs):

@@ -6,7 +6,7 @@ import contextlib
 import pytest
 import torch
 
-from provekv_amd.pool import TwoTierPlan
+from provekv_amd.pool import DeviceKVCache, TwoTierPlan
 
 
 class Event:
@@ -49,16 +49,30 @@ class Profile:
     def payload_len(self, radii=0):
         return 12
 
-    def encode_segments(self, *a, stream=None, **kw):
-        self.ctx.log[f"{self.name} encode"] = stream.run(f"{self.name} encode")
+    def _run(self, op, stream, status, status_cleared):
+        before = self.ctx.log[f"{self.name} {op}"] = stream.run(f"{self.name} {op}")
+        if status_cleared:
+            assert self.ctx.cleared[status.data_ptr()] in before
+        else:
+            self.ctx.log["clear", status.data_ptr()] = before
 
-    def decode_segments(self, *a, stream=None, **kw):
-        self.ctx.log[f"{self.name} decode"] = stream.run(f"{self.name} decode")
+    def encode_segments(self, *a, stream=None, status=None, status_cleared=False, **kw):
+        self._run("encode", stream, status, status_cleared)
+
+    def decode_segments(self, *a, stream=None, status=None, status_cleared=False, **kw):
+        self._run("decode", stream, status, status_cleared)
 
 
 class Context:
     def __init__(self):
-        self.log = {}
+        self.log, self.cleared = {}, {}
+
+    def clear_status(self, buffers, stream=None):
+        name = f"clear {len(self.log)}"
+        before = stream.run(name)
+        for status, _ in buffers:
+            self.cleared[status.data_ptr()] = name
+            self.log["clear", status.data_ptr()] = before
 
     def fib_profile(self, *a):
         return Profile(self, "pool")
@@ -115,3 +129,18 @@ def test_digests_on_an_explicit_capturing_stream(plan, joined):
     plan.digests(bufs, stream=main, side=side)
     assert waited == [main, main]   # the fork, then the order after the digests
     assert "capture begins" in side.after and "digests" in side.after
+
+
+@pytest.mark.parametrize("two_streams", [False, True])
+def test_step_clears_status_words_after_their_readers(plan, two_streams):
+    """The words of a tier are cleared on the stream its rehydrate runs on: what
+    that stream had queued (a read of the last step's words) comes before."""
+    bufs, cache = plan.alloc("cpu"), DeviceKVCache(2, 3, plan.tokens, 64, device="cpu")
+    main, side = torch.cuda.current_stream(), Stream() if two_streams else None
+    readers = {"pool_cstatus": main, "shell_cstatus": side or main, "pool_status": main, "shell_status": main}
+    for step in range(2):
+        plan.build_and_rehydrate(None, bufs, cache, side=side)
+        for name, stream in readers.items():
+            if step:
+                assert f"read {name}" in plan.ctx.log["clear", bufs[name].data_ptr()]
+            stream.run(f"read {name}")
