@@ -194,27 +194,31 @@ class TwoTierPlan:
 
     def _encode_pool(self, corpus, bufs, stream, max_workgroups: int = 0):
         self.fib.encode_segments(corpus, self.pool.enc, bufs["pool_wire"], status=bufs["pool_status"], stream=stream,
-                                 max_workgroups=max_workgroups, status_cleared=True)
+                                 max_workgroups=max_workgroups, status_cleared=bufs["pool_status"] is not None)
 
     def _encode_shells(self, corpus, bufs, stream):
         self.turbo.encode_segments(corpus, self.shells.enc, bufs["shell_wire"], radii=self.radii,
-                                   status=bufs["shell_status"], stream=stream, status_cleared=True)
+                                   status=bufs["shell_status"], stream=stream,
+                                   status_cleared=bufs["shell_status"] is not None)
 
     def _clear(self, bufs, names, stream):
         """The named status words in one launch: each call of a step would
         otherwise clear its own in a launch before its kernel (1.4 us and a
-        launch gap each; three of a step's four are saved)."""
+        launch gap each; three of a step's four are saved).  An entry that is
+        None leaves its call to check itself and raise."""
         n = {"pool": len(self.pool.enc), "shell": len(self.shells.enc)}
-        self.ctx.clear_status([(bufs[k], n[k.split("_")[0]]) for k in names], stream)
+        self.ctx.clear_status([(bufs[k], n[k.split("_")[0]]) for k in names if bufs[k] is not None], stream)
 
     def decode(self, bufs, stream=None):
         """Rehydrate the pool once and every shell: two launches, after one
         that clears both tiers' status words."""
         self._clear(bufs, ("pool_dstatus", "shell_dstatus"), stream)
         self.fib.decode_segments(bufs["pool_wire"], self.pool.dec, bufs["pool_out"],
-                                 status=bufs["pool_dstatus"], stream=stream, status_cleared=True)
+                                 status=bufs["pool_dstatus"], stream=stream,
+                                 status_cleared=bufs["pool_dstatus"] is not None)
         self.turbo.decode_segments(bufs["shell_wire"], self.shells.dec, bufs["shell_out"], radii=self.radii,
-                                   status=bufs["shell_dstatus"], stream=stream, status_cleared=True)
+                                   status=bufs["shell_dstatus"], stream=stream,
+                                   status_cleared=bufs["shell_dstatus"] is not None)
 
     def rehydrate(self, bufs, cache: DeviceKVCache, stream=None):
         """Decode the pool and every shell straight into `cache` -- prefix at
@@ -290,12 +294,14 @@ class TwoTierPlan:
         stream order)."""
         pseg, sseg = self._cache_segs
         out = cache.buf.view(-1)
+        status = bufs["pool_cstatus" if tier == "pool" else "shell_cstatus"]
+        cleared = cleared and status is not None
         if tier == "pool":
-            self.fib.decode_segments(bufs["pool_wire"], pseg, out, status=bufs["pool_cstatus"], stream=stream,
+            self.fib.decode_segments(bufs["pool_wire"], pseg, out, status=status, stream=stream,
                                      fanout=cache.copies, fanout_stride=cache.copy_stride, status_cleared=cleared)
         else:
             self.turbo.decode_segments(bufs["shell_wire"], sseg, out, radii=self.radii,
-                                       status=bufs["shell_cstatus"], stream=stream, fanout=cache.copies,
+                                       status=status, stream=stream, fanout=cache.copies,
                                        fanout_stride=cache.copy_stride, max_workgroups=max_workgroups,
                                        status_cleared=cleared)
             cache.mark_filled(self.tokens)

@@ -47,6 +47,28 @@ def test_step_reports_after_one_clear(ctx, two_streams):
         assert (v == 0xFFFFFFFF).all(), k
 
 
+@pytest.mark.parametrize("two_streams", [False, True])
+def test_step_without_status_words_raises(ctx, two_streams):
+    """Status entries that are None: each call reports its own failure."""
+    import torch
+    plan = TwoTierPlan(ctx, 2, 3, 64, 9, [4, 1])
+    bufs, cache = plan.alloc(), DeviceKVCache(2, 3, plan.tokens, 64)
+    bufs.update({f"{tier}_{s}": None for tier in ("pool", "shell") for s in ("status", "dstatus", "cstatus")})
+    side = torch.cuda.Stream() if two_streams else None
+    good = torch.from_numpy(synth.corpus_tokens(7, 2, 3, plan.tokens, 64)).cuda()
+    plan.build_and_rehydrate(good.view(-1), bufs, cache, side=side)
+    plan.encode(good.view(-1), bufs)
+    plan.decode(bufs)
+    for token in (3, 9):   # the pool's, then a shell's
+        bad = good.clone()
+        bad[token, 1, 2, 0, 5] = float("nan")
+        torch.cuda.synchronize()
+        with pytest.raises(L.PkvError):
+            plan.build_and_rehydrate(bad.view(-1), bufs, cache, side=side)
+        with pytest.raises(L.PkvError):
+            plan.encode(bad.view(-1), bufs)
+
+
 def test_clear_and_run_refusals(ctx):
     import torch
     prof = ctx.turbo_profile(64, 4, 32, 42)

@@ -51,7 +51,9 @@ class Profile:
 
     def _run(self, op, stream, status, status_cleared):
         before = self.ctx.log[f"{self.name} {op}"] = stream.run(f"{self.name} {op}")
-        if status_cleared:
+        if status is None:
+            assert not status_cleared
+        elif status_cleared:
             assert self.ctx.cleared[status.data_ptr()] in before
         else:
             self.ctx.log["clear", status.data_ptr()] = before
@@ -144,3 +146,19 @@ def test_step_clears_status_words_after_their_readers(plan, two_streams):
             if step:
                 assert f"read {name}" in plan.ctx.log["clear", bufs[name].data_ptr()]
             stream.run(f"read {name}")
+
+
+@pytest.mark.parametrize("two_streams", [False, True])
+def test_calls_without_status_words(plan, two_streams):
+    """Buffers whose status entries are None: every call checks itself (it raises
+    the first failure), and nothing is cleared for it."""
+    bufs, cache = plan.alloc("cpu"), DeviceKVCache(2, 3, plan.tokens, 64, device="cpu")
+    bufs.update({f"{tier}_{s}": None for tier in ("pool", "shell") for s in ("status", "dstatus", "cstatus")})
+    side = Stream() if two_streams else None
+    main = torch.cuda.current_stream()
+    plan.encode(None, bufs, stream=main)
+    plan.decode(bufs, stream=main)
+    plan.rehydrate(bufs, cache, stream=main)
+    plan.build_and_rehydrate(None, bufs, cache, side=side)
+    assert {"pool encode", "shells encode", "pool decode", "shells decode"} <= set(plan.ctx.log)
+    assert not plan.ctx.cleared
