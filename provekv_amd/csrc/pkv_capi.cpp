@@ -1043,10 +1043,16 @@ static int fib_verify_mfma_products(pkv_ctx* ctx, pkv_profile* p) {
 }
 
 // The matrix-core decode's table of partial sums (ready when this returns).
+// Without memory for it the profile decodes by the kernel that forms every sum.
 static int fib_build_prefix(pkv_ctx* ctx, pkv_profile* p) {
     if (!p->mfma_decode) return PKV_OK;
-    HIP_TRY(hipMalloc(reinterpret_cast<void**>(&p->d_prefix),
-                      (sizeof(float) * p->dim) << (5 * FIB_PREFIX_BLOCKS)));
+    const hipError_t me =
+        hipMalloc(reinterpret_cast<void**>(&p->d_prefix), (sizeof(float) * p->dim) << (5 * FIB_PREFIX_BLOCKS));
+    if (me != hipSuccess) {
+        p->d_prefix = nullptr;
+        (void)hipGetLastError();   // the next launch check must not see it
+        return me == hipErrorOutOfMemory ? PKV_OK : hip_status(me);
+    }
     const hipError_t e = static_cast<hipError_t>(launch_fib_prefix(p->d_rot32, p->d_cb, p->d_prefix, ctx->own_stream));
     const hipError_t se = hipStreamSynchronize(ctx->own_stream);
     return hip_status(e == hipSuccess ? se : e);

@@ -84,7 +84,7 @@ struct FibDev {
     const double* rot64;    // dim * dim, row-major (the encode's exact redo)
     const float* rot32t;    // dim * dim, f32(rot) transposed: [col][row] (VALU decode)
     const float* rot32;     // dim * dim, f32(rot) row-major (MFMA decode)
-    const float* prefix;    // 32^FIB_PREFIX_BLOCKS * dim partial sums (MFMA decode)
+    const float* prefix;    // 32^FIB_PREFIX_BLOCKS * dim partial sums (MFMA decode), or null
     int mfma_decode;        // matrix-core products verified bit-exact for this profile
     const uint32_t* mf;     // MF_WORDS (encode MFMA operands)
     float thr;              // argmin acceptance margin for the approximate keys

@@ -4079,11 +4079,12 @@ int launch_fib_decode(const LaunchCommon& lc, const FibDev& fd, const uint8_t* w
     // 12 output bytes per value the decode is bound by its writes and the
     // table's reads slow them down (a step of 1.2 M pool and 0.34 M shell
     // vectors, table against none: 2 f32 copies 425 / 439 us, 3 474 / 476, 4
-    // 527 / 520, 8 798 / 778; 4 bf16 copies 441 / 460, 8 544 / 527).
-    const bool table = lc.fanout <= (lc.out_dtype == PKV_F32 ? 3u : 6u);
-    auto kern = lc.fanout == 1 ? fib_decode_mfma_kernel<64, false, true>
-                : table        ? fib_decode_mfma_kernel<64, true, true>
-                               : fib_decode_mfma_kernel<64, true, false>;
+    // 527 / 520, 8 798 / 778; 4 bf16 copies 441 / 460, 8 544 / 527).  A profile
+    // created without memory for the table has none at any fan-out.
+    const bool table = fd.prefix && lc.fanout <= (lc.out_dtype == PKV_F32 ? 3u : 6u);
+    auto kern = !table           ? fib_decode_mfma_kernel<64, true, false>
+                : lc.fanout == 1 ? fib_decode_mfma_kernel<64, false, true>
+                                 : fib_decode_mfma_kernel<64, true, true>;
     // one half-tile per workgroup (a resident grid walking them was slower: one
     // copy 172 against 164 us, 8 copies 830 against 778 us for the step) unless
     // the caller bounds its share of the GPU
