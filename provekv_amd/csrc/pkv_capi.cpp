@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -88,6 +89,20 @@ struct Slot {
 
 struct NoallocScratch;   // pkv_decode_segments_noalloc's per-device scratch (below)
 
+// A fib decode's table of partial sums, shared by the profiles of a device with
+// the same constants; the last of them frees it.
+struct FibPrefix {
+    int device = 0;
+    std::vector<float> key;   // what the sums are formed from: rows of f32(Pi), then the codebook
+    float* d = nullptr;
+    FibPrefix() = default;
+    FibPrefix(const FibPrefix&) = delete;
+    FibPrefix& operator=(const FibPrefix&) = delete;
+    ~FibPrefix() {
+        if (d) (void)hipFree(d);
+    }
+};
+
 }  // namespace
 
 struct pkv_ctx {
@@ -131,7 +146,7 @@ struct pkv_profile {
     double* d_rot64 = nullptr;   // row-major f64 rotation (encode's exact redo)
     float* d_rot32t = nullptr;
     float* d_rot32 = nullptr;
-    float* d_prefix = nullptr;   // decode partial sums (matrix-core decode only)
+    std::shared_ptr<FibPrefix> prefix;   // decode partial sums (matrix-core decode only), or none
     int mfma_decode = 0;
     uint32_t* d_mf = nullptr;
     float thr = 0.0f;
@@ -475,7 +490,7 @@ FibDev fib_dev(const pkv_profile* p) {
     f.rot64 = p->d_rot64;
     f.rot32t = p->d_rot32t;
     f.rot32 = p->d_rot32;
-    f.prefix = p->d_prefix;
+    f.prefix = p->prefix ? p->prefix->d : nullptr;
     f.mfma_decode = p->mfma_decode;
     f.mf = p->d_mf;
     f.thr = p->thr;
@@ -1042,20 +1057,44 @@ static int fib_verify_mfma_products(pkv_ctx* ctx, pkv_profile* p) {
     return PKV_OK;
 }
 
-// The matrix-core decode's table of partial sums (ready when this returns).
-// Without memory for it the profile decodes by the kernel that forms every sum.
+// The tables in use (a table leaves with its last profile).
+static std::mutex g_prefix_mu;
+static std::vector<std::weak_ptr<FibPrefix>> g_prefix;
+
+// The matrix-core decode's table of partial sums: that of a profile with the same
+// constants, or a new one, complete when this returns.  Without memory for it the
+// profile decodes by the kernel that forms every sum.
 static int fib_build_prefix(pkv_ctx* ctx, pkv_profile* p) {
     if (!p->mfma_decode) return PKV_OK;
+    std::vector<float> key(p->rot32.begin(), p->rot32.begin() + FIB_PREFIX_BLOCKS * p->k * p->dim);
+    key.insert(key.end(), p->codebook.begin(), p->codebook.end());
+    std::lock_guard<std::mutex> lock(g_prefix_mu);
+    g_prefix.erase(std::remove_if(g_prefix.begin(), g_prefix.end(), [](auto& w) { return w.expired(); }),
+                   g_prefix.end());
+    for (const auto& w : g_prefix) {
+        std::shared_ptr<FibPrefix> t = w.lock();
+        if (t && t->device == ctx->device && t->key.size() == key.size() &&
+            std::memcmp(t->key.data(), key.data(), sizeof(float) * key.size()) == 0) {
+            p->prefix = std::move(t);
+            return PKV_OK;
+        }
+    }
+    auto t = std::make_shared<FibPrefix>();
+    t->device = ctx->device;
+    t->key = std::move(key);
     const hipError_t me =
-        hipMalloc(reinterpret_cast<void**>(&p->d_prefix), (sizeof(float) * p->dim) << (5 * FIB_PREFIX_BLOCKS));
+        hipMalloc(reinterpret_cast<void**>(&t->d), (sizeof(float) * p->dim) << (5 * FIB_PREFIX_BLOCKS));
     if (me != hipSuccess) {
-        p->d_prefix = nullptr;
+        t->d = nullptr;
         (void)hipGetLastError();   // the next launch check must not see it
         return me == hipErrorOutOfMemory ? PKV_OK : hip_status(me);
     }
-    const hipError_t e = static_cast<hipError_t>(launch_fib_prefix(p->d_rot32, p->d_cb, p->d_prefix, ctx->own_stream));
+    const hipError_t e = static_cast<hipError_t>(launch_fib_prefix(p->d_rot32, p->d_cb, t->d, ctx->own_stream));
     const hipError_t se = hipStreamSynchronize(ctx->own_stream);
-    return hip_status(e == hipSuccess ? se : e);
+    if (e != hipSuccess || se != hipSuccess) return hip_status(e == hipSuccess ? se : e);
+    g_prefix.push_back(t);
+    p->prefix = std::move(t);
+    return PKV_OK;
 }
 
 static int fib_profile_common(pkv_ctx* ctx, uint32_t dim, uint32_t k, uint32_t n, std::vector<float> cb,
@@ -1240,10 +1279,9 @@ void pkv_profile_destroy(pkv_profile* p) {
                     static_cast<void*>(p->d_qa), static_cast<void*>(p->d_qb),
                     static_cast<void*>(p->d_cb), static_cast<void*>(p->d_rot_t), static_cast<void*>(p->d_rot64),
                     static_cast<void*>(p->d_rot32t),
-                    static_cast<void*>(p->d_mf), static_cast<void*>(p->d_rot32), static_cast<void*>(p->d_cb64),
-                    static_cast<void*>(p->d_prefix)})
+                    static_cast<void*>(p->d_mf), static_cast<void*>(p->d_rot32), static_cast<void*>(p->d_cb64)})
         if (d) (void)hipFree(d);
-    delete p;
+    delete p;   // with the table of partial sums when no other profile holds it
 }
 
 int pkv_fib_decode_path(const pkv_profile* p) {

@@ -1,6 +1,7 @@
 """The fib decode's table of partial sums as the host half keeps it, on the CPU
 with the HIP runtime replaced by tests/host_hip.cpp: a profile whose table cannot
-be allocated is created all the same and decodes by the kernel without one."""
+be allocated is created all the same and decodes by the kernel without one, and
+profiles with equal constants share a table."""
 import ctypes as C
 import os
 import subprocess
@@ -28,7 +29,7 @@ def _child(stub, name):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-@pytest.mark.parametrize("name", ["no_memory", "with_memory"])
+@pytest.mark.parametrize("name", ["no_memory", "with_memory", "equal_constants"])
 def test_profile_creation(stub, name):
     _child(stub, name)
 
@@ -58,7 +59,7 @@ class Host:
     def decode(self, prof, fanout):
         """The kernel a decode of 5 vectors into `fanout` f32 copies launches."""
         from provekv_amd.device import SEG_DTYPE
-        segs = np.array([(0, 64, 0, 0, 5, 5)], dtype=SEG_DTYPE)
+        segs = np.array([(0, 0, 64, 0, 5, 5)], dtype=SEG_DTYPE)
         wire, status = np.zeros(19 + 5 * 12 + 16, np.uint8), np.zeros(4, np.uint32)
         out = np.zeros(fanout * 5 * 64 + 4, np.float32)
         ptr = out.ctypes.data + -out.ctypes.data % 16
@@ -87,6 +88,21 @@ def child_with_memory(h):
     assert "fib_decode_mfma_kernelILi64ELb1ELb1E" in h.decode(prof, 2)
     assert STAGED_NO_TABLE in h.decode(prof, 4)
     h.L.pkv_profile_destroy(prof)
+    assert h.tables() == 0
+
+
+def child_equal_constants(h):
+    a, b, other = h.profile(), h.profile(), h.profile(seed=1)
+    assert h.tables() == 2
+    h.L.pkv_profile_destroy(a)
+    assert h.tables() == 2   # b's
+    assert "fib_decode_mfma_kernelILi64ELb0ELb1E" in h.decode(b, 1)
+    h.L.pkv_profile_destroy(b)
+    assert h.tables() == 1
+    b = h.profile()          # built again
+    assert h.tables() == 2
+    h.L.pkv_profile_destroy(b)
+    h.L.pkv_profile_destroy(other)
     assert h.tables() == 0
 
 

@@ -79,6 +79,22 @@ def test_fib_decode_rules(ctx, dtype, fanout, heads, cap):
         assert torch.equal(got[c].view(bits), want.view(bits)), c
 
 
+def test_handles_of_equal_constants(ctx):
+    """They share the table of partial sums, and the one that is left keeps it."""
+    import torch
+    cb, rot = _constants()
+    blob = _blob(np.random.RandomState(3), 100)
+    wire = torch.from_numpy(np.frombuffer(blob, np.uint8).copy()).cuda()
+    segs = np.array([(0, 0, 64, 0, 100, 100)], dtype=SEG_DTYPE)
+    want = O.fib_decode_batch(blob, cb, rot).view(np.uint32)
+    profs = [ctx.fib_profile_with_constants(cb, rot) for _ in range(3)]
+    for p in profs:
+        out = torch.zeros(100 * 64, device="cuda")
+        p.decode_segments(wire, segs, out)
+        assert np.array_equal(out.cpu().numpy().view(np.uint32).reshape(100, 64), want)
+        p.close()
+
+
 def _rows(blob, idx):
     """The blob of the vectors `idx` of `blob`."""
     hdr = bytearray(blob[:19])
