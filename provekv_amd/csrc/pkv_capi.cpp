@@ -1506,12 +1506,19 @@ struct B3Plan {
     uint64_t end[2] = {0, 0};       // last byte (exclusive) the ranges need of each buffer
 };
 
-// Chunks below which pass 0 puts four lanes on a chunk (16 chunks per wave,
-// ~1.4x the instructions, a quarter of the latency): one lane per chunk would
-// leave the GPU with fewer than half a wave per SIMD.  Measured (both passes of
-// a call, one lane / four): config 3's pool, 14.4 Ki chunks, 47 / 30 us; its
-// shells, 48 Ki chunks, 51 / 50 us; 64 Ki chunks 50 / 61 us.
-constexpr uint64_t kB3QuadBelow = 32ull * 1024;
+// Chunks of a call (both tiers of a build together) below which pass 0 puts four
+// lanes on a chunk: 16 chunks per wave, ~1.4x the instructions, a quarter of the
+// latency; one lane per chunk leaves the GPU with at most a wave per SIMD there.
+// Measured, one lane / four, us a call, over 48 ranges | 48 and 384 ranges of two
+// tiers | 600 ranges of equal size:
+//   16 Ki  58 / 40 | 54 / 34 | 57 / 44      52 Ki  55 / 63 | 52 / 58 | 92 / 66
+//   32 Ki  56 / 50 | 52 / 49 | 59 / 55      64 Ki  90 / 70 | 82 / 66 | 93 / 74
+//   44 Ki  55 / 51 | 50 / 49 | 90 / 58      80 Ki  89 / 77 | 82 / 73 | 87 / 83
+//   48 Ki  54 / 51 | 52 / 57 | 95 / 65      96 Ki  85 / 80 | 78 / 82 | 87 / 91
+// Four lanes are ahead in every shape up to 44 Ki; past 48 Ki the count alone does
+// not decide (one lane steps up with its second wave per SIMD, 1,024 tiles of 64
+// chunks of a range).
+constexpr uint64_t kB3QuadBelow = 48ull * 1024;
 
 // Ranges r < split lie in the first buffer, the others in the second.
 int plan_blake3(const pkv_range* ranges, uint32_t nr, uint64_t split, const uint64_t (&buf_bytes)[2], B3Plan* plan) {

@@ -97,6 +97,27 @@ def test_build_digests_two_buffers(ctx, na, nb, side):
             assert [bytes(r) for r in lay.cpu().numpy()] == want, rep
 
 
+@pytest.mark.parametrize("chunks", [48 * 1024 - 1, 48 * 1024], ids=["four_lanes", "one_lane"])
+def test_build_digests_at_the_first_pass_line(ctx, chunks):
+    """The chunks of both tiers together decide the form of the first pass."""
+    import torch
+    rng = np.random.RandomState(5)
+    data = rng.randint(0, 256, (28 << 20) + 8).astype(np.uint8)
+    tiers, refs = [], []
+    for k, n, total in ((0, 7, 28 * 1024), (1, 30, chunks - 28 * 1024)):
+        cuts = np.linspace(0, total, 2 * n + 1).astype(np.int64)   # whole chunks, less 5 bytes at each end
+        rg = np.stack([1024 * cuts[:-1] + k, 1024 * np.diff(cuts) - 5], 1).astype(np.uint64)
+        refs.append(O.blake3_ranges(data, rg))
+        tiers.append((torch.from_numpy(data).cuda(), rg, torch.zeros((n, 2, 32), dtype=torch.uint8, device="cuda"),
+                      torch.zeros((n, 32), dtype=torch.uint8, device="cuda")))
+    assert sum(-(-int(ln) // 1024) for _, rg, _, _ in tiers for _, ln in rg) == chunks
+    ctx.build_digests(tiers, 3)
+    for (_, rg, blob, lay), ref in zip(tiers, refs):
+        assert np.array_equal(blob.cpu().numpy().reshape(-1, 32), ref)
+        want = [O.layer_digest(i % 3, ref[2 * i].tobytes(), ref[2 * i + 1].tobytes()) for i in range(len(rg) // 2)]
+        assert [bytes(r) for r in lay.cpu().numpy()] == want
+
+
 def test_plan_digests_follow_the_side_stream(ctx):
     """TwoTierPlan.digests(side=...) hashes what the side stream had queued."""
     import torch

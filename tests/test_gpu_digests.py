@@ -60,7 +60,7 @@ def _chunks(ranges):
 
 @pytest.mark.parametrize("mode", ["quad", "lane"])
 def test_ranges_match_oracle(ctx, mode):
-    """Both first-pass forms: a call of fewer than 32 Ki chunks runs four
+    """Both first-pass forms: a call of fewer than 48 Ki chunks runs four
     lanes per chunk, a larger one one lane per chunk."""
     import torch
     rng = np.random.default_rng(11)
@@ -71,13 +71,13 @@ def test_ranges_match_oracle(ctx, mode):
     if mode == "quad":
         keep, total = [], 0
         for r in ranges:
-            if total + _chunks([r]) < 32 * 1024:
+            if total + _chunks([r]) < 48 * 1024:
                 keep.append(r)
                 total += _chunks([r])
         ranges = keep
-        assert _chunks(ranges) < 32 * 1024 and any(ln > 4096 * 1024 for _, ln in ranges)
+        assert _chunks(ranges) < 48 * 1024 and any(ln > 4096 * 1024 for _, ln in ranges)
     else:
-        assert _chunks(ranges) >= 32 * 1024
+        assert _chunks(ranges) >= 48 * 1024
     print(f"{len(ranges)} ranges over {n} bytes", flush=True)
     got = ctx.blake3_ranges(buf, ranges)
     torch.cuda.synchronize()
@@ -87,7 +87,7 @@ def test_ranges_match_oracle(ctx, mode):
 
 
 def test_ranges_lane_mode_match_oracle(ctx):
-    """32 Ki chunks or more in one call (here: 40 overlapping ranges of
+    """48 Ki chunks or more in one call (here: 40 overlapping ranges of
     ~4.1 MB) take the one-lane-per-chunk first pass; fewer take four lanes
     per chunk (the other range tests here)."""
     import torch
@@ -96,7 +96,7 @@ def test_ranges_lane_mode_match_oracle(ctx):
     host = rng.integers(0, 256, n, dtype=np.uint8)
     buf = torch.from_numpy(host).cuda()
     ranges = [(int(a), 4100 * 1024 + int(b)) for a, b in zip(rng.integers(0, 900_000, 40), rng.integers(0, 2048, 40))]
-    assert sum((ln + 1023) // 1024 for _, ln in ranges) >= 32 * 1024
+    assert sum((ln + 1023) // 1024 for _, ln in ranges) >= 48 * 1024
     got = ctx.blake3_ranges(buf, ranges).cpu().numpy()
     assert np.array_equal(got, O.blake3_ranges(host, ranges))
 
