@@ -1687,6 +1687,7 @@ int pkv_blake3_build_digests(pkv_ctx* ctx, const pkv_digest_tier* tiers, uint32_
     uint32_t used = 0;
     for (uint32_t k = 0; k < n_tiers; ++k) {
         const pkv_digest_tier& t = tiers[k];
+        if (t.reserved) return PKV_ERR_INVALID_ARG;
         if (t.n == 0) continue;
         if (t.n > 0x7FFFFFFFu || !t.ranges || !t.d_blob_digests || !t.d_layer_digests || (!t.d_buf && t.buf_bytes) ||
             reinterpret_cast<uintptr_t>(t.d_blob_digests) % 4 || reinterpret_cast<uintptr_t>(t.d_layer_digests) % 4)

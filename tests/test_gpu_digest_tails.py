@@ -97,6 +97,20 @@ def test_build_digests_two_buffers(ctx, na, nb, side):
             assert [bytes(r) for r in lay.cpu().numpy()] == want, rep
 
 
+def test_build_digests_refuses_a_reserved_field(ctx):
+    import ctypes as C
+    import torch
+    from provekv_amd import _lib as L
+    buf, rg = torch.zeros(64, dtype=torch.uint8, device="cuda"), np.array([(0, 8), (8, 8)], np.uint64)
+    blob, lay = (torch.zeros(n, dtype=torch.uint8, device="cuda") for n in (64, 32))
+    for n in (0, 1):
+        for reserved, ok in ((0, True), (1, False)):
+            t = L.DigestTier(buf.data_ptr(), 64, rg.ctypes.data, blob.data_ptr(), lay.data_ptr(), n, reserved)
+            rc = L.lib().pkv_blake3_build_digests(ctx.ptr, C.byref(t), 1, 3, None)
+            assert (rc == 0) == ok
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("chunks", [48 * 1024 - 1, 48 * 1024], ids=["four_lanes", "one_lane"])
 def test_build_digests_at_the_first_pass_line(ctx, chunks):
     """The chunks of both tiers together decide the form of the first pass."""
