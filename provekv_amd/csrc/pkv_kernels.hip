@@ -227,8 +227,8 @@ __device__ void stage_rows_in(float* stage, const void* __restrict__ in, bool bf
 }
 
 // Two f32 -> bfloat16 bits, round to nearest even (torch's / c10's conversion;
-// a NaN keeps its upper bits and turns quiet): one v_cvt_pk_bf16_f32, equal to
-// the integer rounding it replaces on every float, where that took six
+// a NaN keeps its upper bits and turns quiet): one v_cvt_pk_bf16_f32, compared with
+// the integer rounding on all 2^32 inputs (no difference), which took six
 // operations a value (a step of 1.2 M pool and 0.34 M shell vectors
 // into one bf16 cache 404 -> 364 us, with the other changes to its decodes; the
 // shells' decode into one 36 -> 32 us).
