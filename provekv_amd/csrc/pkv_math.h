@@ -346,9 +346,9 @@ PKV_HD float og_expf(float x, const uint64_t* tab) {
 }
 
 // og_expf for |x| <= 32.5 with the multiply-adds fused (7 f64 operations
-// instead of 13, no range checks): the same f32 for every such x -- the two
-// finite floats on which the forms differ are 0x1.04845ep+5 and
-// -0x1.f8cbb2p+5 (every float below 88 in magnitude was compared).
+// instead of 13, no range checks): the same f32 for every such x.  Below 88 in
+// magnitude the forms differ on two floats only, 0x1.04845ep+5 and
+// -0x1.f8cbb2p+5 (all were compared).
 PKV_HD float og_expf_fused(float x, const uint64_t* tab) {
     const double N = 32.0;
     const double InvLn2N = 0x1.71547652b82fep+0 * 32.0;

@@ -319,3 +319,21 @@ def test_lossy_decode_short_forms():
     q = np.zeros_like(u)
     L.lib().pkv_host_div255(u.ctypes.data, u.size, q.ctypes.data)
     assert np.array_equal(q, u / np.float32(255.0))
+
+
+def test_fused_expf_on_every_float_it_takes():
+    """The fused expf has the restated expf's bits on all 2,214,854,658 floats of
+    |x| <= 32.5."""
+    from concurrent.futures import ThreadPoolExecutor
+    lib, step = L.lib(), 1 << 22
+    edge = int(np.float32(32.5).view(np.uint32)) + 1
+
+    def same(first, last):   # the library calls and numpy's loops release the interpreter
+        x = np.arange(first, last, dtype=np.uint32).view(np.float32)
+        got, want = np.empty_like(x), np.empty_like(x)
+        lib.pkv_host_expf_fused(x.ctypes.data, x.size, got.ctypes.data)
+        lib.pkv_host_expf(x.ctypes.data, x.size, want.ctypes.data)
+        return last - first if np.array_equal(got.view(np.uint32), want.view(np.uint32)) else 0
+    runs = [(s + i, s + min(i + step, edge)) for s in (0, 1 << 31) for i in range(0, edge, step)]
+    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        assert sum(pool.map(same, *zip(*runs))) == 2 * edge == 2_214_854_658
