@@ -344,7 +344,7 @@ class TwoTierPlan:
         import torch
         main = stream if stream is not None else torch.cuda.current_stream()
         if side is not None:
-            if stream is None:
+            if stream is None or stream == torch.cuda.current_stream():
                 capturing = torch.cuda.is_current_stream_capturing()
             else:
                 with torch.cuda.stream(main):
