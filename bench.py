@@ -1069,7 +1069,7 @@ def bench_digest(args):
            "workload": "digest", "unit": "GB/s", "steps": args.steps, "warmup": args.warmup,
            "parity_all_digests": bool(parity),
            "config3": {"ranges": len(plan.pool.blob_offsets) + len(plan.shells.blob_offsets),
-                       "tiers": "one stream" if side is None else "both tiers in one call",
+                       "tiers": "both in one call" + ("" if side is None else ", ordered with a side stream"),
                        "bytes": int(wire_bytes), "ms_per_call": round(ms, 4),
                        "gbs": round(wire_bytes / (ms * 1e-3) / 1e9, 1), "roofline": valu(wire_bytes, ms)},
            "bulk_512x1MiB": {"bytes": bulk_bytes, "ms_per_call": round(bms, 4),

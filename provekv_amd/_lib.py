@@ -46,16 +46,16 @@ EXPORTS = (
     "pkv_fib_profile_create_with_constants", "pkv_profile_destroy", "pkv_fib_decode_path", "pkv_turbo_constants",
     "pkv_fib_constants", "pkv_profile_constants", "pkv_payload_len", "pkv_header_len", "pkv_blob_len",
     "pkv_write_header",
-    "pkv_segments_status", "pkv_encode_segments", "pkv_encode_segments_bounded", "pkv_decode_segments", "pkv_decode_segments_ex",
-    "pkv_decode_segments_bounded", "pkv_decode_segments_noalloc", "pkv_status_clear", "pkv_run_segments",
-    "pkv_encode_batch_compact",
-    "pkv_decode_batch_compact", "pkv_parse_header", "pkv_record_len", "pkv_encode_vectors", "pkv_decode_vectors",
-    "pkv_constants_cache_stats", "pkv_constants_cache_clear", "pkv_prepared_len", "pkv_turbo_prepare_queries",
+    "pkv_segments_status", "pkv_encode_segments", "pkv_encode_segments_bounded", "pkv_decode_segments",
+    "pkv_decode_segments_ex", "pkv_decode_segments_bounded", "pkv_decode_segments_noalloc", "pkv_status_clear",
+    "pkv_run_segments", "pkv_encode_batch_compact", "pkv_decode_batch_compact", "pkv_parse_header",
+    "pkv_record_len", "pkv_encode_vectors", "pkv_decode_vectors", "pkv_constants_cache_stats",
+    "pkv_constants_cache_clear", "pkv_prepared_len", "pkv_turbo_prepare_queries",
     "pkv_turbo_score_segments", "pkv_score_status", "pkv_turbo_score_batch", "pkv_encode_diagnostics",
     "pkv_radii_log_bound", "pkv_fb2_n_blocks", "pkv_lloyd_refine", "pkv_blake3_ranges", "pkv_blake3_layer_digests",
     "pkv_blake3_tier_digests", "pkv_blake3_build_digests", "pkv_blake3",
-    "pkv_host_angle_bins", "pkv_host_octant_bins", "pkv_host_logf",
-    "pkv_host_expf", "pkv_host_expf_fused", "pkv_host_div255", "pkv_host_f32_stable_rel50", "pkv_code_from_json", "pkv_fib_digests", "pkv_host_blake3",
+    "pkv_host_angle_bins", "pkv_host_octant_bins", "pkv_host_logf", "pkv_host_expf", "pkv_host_expf_fused",
+    "pkv_host_div255", "pkv_host_f32_stable_rel50", "pkv_code_from_json", "pkv_fib_digests", "pkv_host_blake3",
 )
 
 

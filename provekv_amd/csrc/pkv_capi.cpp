@@ -318,7 +318,8 @@ int validate_segments(const pkv_profile* p, int radii, bool encode, int dtype, c
     if (encode && !in_order) {   // encoded blobs are written by different workgroups: no overlap
         std::vector<std::pair<uint64_t, uint64_t>> blobs(nseg);
         for (uint32_t i = 0; i < nseg; ++i)
-            blobs[i] = {segs[i].wire_offset, segs[i].wire_offset + hdr + static_cast<uint64_t>(segs[i].n_vectors) * plen};
+            blobs[i] = {segs[i].wire_offset,
+                        segs[i].wire_offset + hdr + static_cast<uint64_t>(segs[i].n_vectors) * plen};
         std::sort(blobs.begin(), blobs.end());
         for (size_t i = 1; i < blobs.size(); ++i)
             if (blobs[i].first < blobs[i - 1].second) return PKV_ERR_INVALID_ARG;
@@ -506,10 +507,10 @@ FibDev fib_dev(const pkv_profile* p) {
 // profile over a device-resident segment table (dsegs, dtiles: nseg + 1 tile
 // prefix, nblocks tiles in all; segs: the host's copy).  Returns a hipError_t as int.
 int launch_segments(const pkv_profile* prof, int radii, bool encode, int dtype, const void* d_f32,
-                    const uint8_t* d_wire, const pkv_seg* segs, const SegDev* dsegs, const uint32_t* dtiles, uint32_t nseg,
-                    uint32_t nblocks, uint32_t* status, bool per_vector, uint32_t fanout, uint64_t fanout_stride,
-                    uint32_t grid_cap, hipStream_t stream, float* diag = nullptr, const uint32_t* dmap = nullptr,
-                    bool cleared = false) {
+                    const uint8_t* d_wire, const pkv_seg* segs, const SegDev* dsegs, const uint32_t* dtiles,
+                    uint32_t nseg, uint32_t nblocks, uint32_t* status, bool per_vector, uint32_t fanout,
+                    uint64_t fanout_stride, uint32_t grid_cap, hipStream_t stream, float* diag = nullptr,
+                    const uint32_t* dmap = nullptr, bool cleared = false) {
     LaunchCommon lc;
     lc.segs = dsegs;
     lc.tile_start = dtiles;
@@ -560,8 +561,8 @@ int run_segments_locked(pkv_ctx* ctx, const pkv_profile* prof, int radii, bool e
     if (dtype != PKV_F32 && dtype != PKV_BF16 && (encode || dtype != PKV_F16)) return PKV_ERR_INVALID_ARG;
     if (encode && fanout != 1) return PKV_ERR_INVALID_ARG;
     std::vector<uint32_t> tiles(static_cast<size_t>(nseg) + 1);
-    int rc = validate_segments(prof, radii, encode, dtype, d_f32, f32_elems, segs, nseg, d_wire, wire_bytes, tiles.data(),
-                               fanout, fanout_stride);
+    int rc = validate_segments(prof, radii, encode, dtype, d_f32, f32_elems, segs, nseg, d_wire, wire_bytes,
+                               tiles.data(), fanout, fanout_stride);
     if (rc) return rc;
     HIP_TRY(hipSetDevice(ctx->device));
     if (!d_status) {
@@ -578,8 +579,8 @@ int run_segments_locked(pkv_ctx* ctx, const pkv_profile* prof, int radii, bool e
     rc = stage_table(ctx, segs, nseg, tiles, d_status == nullptr, stream, &sl, &dsegs, &dtiles, &dstat, &dmap);
     if (rc) return rc;
     uint32_t* status = d_status ? d_status : dstat;
-    const int e = launch_segments(prof, radii, encode, dtype, d_f32, d_wire, segs, dsegs, dtiles, nseg, tiles[nseg], status,
-                                  per_vector, fanout, fanout_stride, grid_cap, stream, diag, dmap, cleared);
+    const int e = launch_segments(prof, radii, encode, dtype, d_f32, d_wire, segs, dsegs, dtiles, nseg, tiles[nseg],
+                                  status, per_vector, fanout, fanout_stride, grid_cap, stream, diag, dmap, cleared);
     int rc2 = finish_slot(sl, stream);
     if (e) return hip_status(static_cast<hipError_t>(e));
     if (rc2 || d_status) return rc2;
@@ -1448,7 +1449,8 @@ int pkv_decode_segments_noalloc(pkv_ctx* ctx, const pkv_profile* prof, int radii
     // pageable host sources: the runtime stages them before returning
     HIP_TRY(hipMemcpyAsync(base, segs, sizeof(pkv_seg) * nseg, hipMemcpyHostToDevice, st));
     HIP_TRY(hipMemcpyAsync(base + kNaTileOff, tiles, sizeof(uint32_t) * (nseg + 1), hipMemcpyHostToDevice, st));
-    const int e = launch_segments(prof, radii, false, out_dtype, d_out, d_wire, segs, reinterpret_cast<const SegDev*>(base),
+    const int e = launch_segments(prof, radii, false, out_dtype, d_out, d_wire, segs,
+                                  reinterpret_cast<const SegDev*>(base),
                                   reinterpret_cast<const uint32_t*>(base + kNaTileOff), nseg, tiles[nseg], d_status,
                                   false, fanout, fanout_stride, 0, st);
     const hipError_t re = hipEventRecord(sc.ev, st);

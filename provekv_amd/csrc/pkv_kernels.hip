@@ -10,9 +10,12 @@
 //   * f32 rows: 16 lanes cover one 256 B row with 16 B loads/stores; each lane
 //     then reads its own row from LDS (row pitch dim+4 floats: conflict-free
 //     ds_read_b128);
-//   * wire bytes: a wave's 64 payloads are one contiguous byte range; it is
-//     moved with aligned dword accesses and v_alignbyte, independent of the
-//     38 B (TQB1) / 19 B (FB2) header offset.
+//   * wire bytes: a wave's payloads are one contiguous byte range; the encodes
+//     store it 16 bytes per lane at any byte alignment (the header is 38 B,
+//     TQB1, or 19 B, FB2), the head_dim-128 split decode and the table scoring
+//     load it so; the head_dim-64 split decode copies aligned dwords to LDS, the
+//     general decodes and scoring shift such dwords into place by v_alignbyte,
+//     the fib matrix-core decode loads a vector's 12 bytes per lane.
 //
 // Arithmetic follows the reference operation by operation (compiled with
 // -ffp-contract=off): the FWHT butterfly order of fwht_normalized
@@ -2128,14 +2131,14 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
         bool ok = true;
         float r[HP];
         if constexpr (!LOSSY) {
-    #pragma unroll
+#pragma unroll
             for (int i = 0; i < HP; ++i) {
                 r[i] = u2f(pw[(i < 8 ? 8 * q : 24 + 8 * q) + i]);
                 ok &= isfinite_f(r[i]) && !(r[i] < 0.0f);   // radius.rs:88-104
             }
         } else {
             uint32_t w[4];
-    #pragma unroll
+#pragma unroll
             for (int k = 0; k < 4; ++k) w[k] = pw[(k < 2 ? 2 * q : 6 + 2 * q) + k];
             radii_u8<HP>(w, u2f(pw[16]), u2f(pw[17]), exp_lds, r, ok);
         }
@@ -2145,7 +2148,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
         {
             const uint32_t nb = 8u * pbits;
             uint64_t run[2];
-    #pragma unroll
+#pragma unroll
             for (int half = 0; half < 2; ++half) {
                 const uint32_t bit0 = nb * (static_cast<uint32_t>(q) + 4u * half);
                 const uint32_t* aw = pw + rwords + (bit0 >> 5);
@@ -2158,7 +2161,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
         // bits to check (bitpack.rs:88-109); nor in the 32/64-bit QJL field
 
         float y[32];
-    #pragma unroll
+#pragma unroll
         for (int i = 0; i < HP; ++i) {
             const uint32_t bin = static_cast<uint32_t>(pk >> (static_cast<uint32_t>(i) * pbits)) & (levels - 1u);
             y[2 * i] = r[i] * cs_lds[2 * bin];
@@ -2173,7 +2176,7 @@ __global__ __launch_bounds__(TILE) void turbo_decode_split128_kernel(
         float* stage = reinterpret_cast<float*>(sw);
         {
             const uint32_t g0 = 16u * static_cast<uint32_t>(((q & 1) << 1) | (q >> 1)), g1 = 64u + g0;
-    #pragma unroll
+#pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const uint32_t e = (k < 4 ? g0 : g1) + 4u * (k & 3);
                 const float4 sg = *reinterpret_cast<const float4*>(signs + e);
@@ -3884,9 +3887,9 @@ int launch_turbo_encode(const LaunchCommon& lc, const TurboDev& td, const void* 
         if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 workgroups per tile
         const size_t vec_words = (lc.plen >> 2) + (lc.radii == PKV_RADII_F32 ? 0u : 32u);
         const size_t lds = static_cast<size_t>(WAVES) * (32 * vec_words + 4) * sizeof(uint32_t);
-#define PKV_QJL64(PB, DG, OW)                                                                                      \
-    launch_big_lds(turbo_encode_qjl_kernel<PB, DG, OW>, 2 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl, td.cs, \
-                   td.qa, td.qb, td.seed, td.pbits, td.proj)
+#define PKV_QJL64(PB, DG, OW)                                                                                  \
+    launch_big_lds(turbo_encode_qjl_kernel<PB, DG, OW>, 2 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl,  \
+                   td.cs, td.qa, td.qb, td.seed, td.pbits, td.proj)
         if (lc.diag) return td.pbits == 3 ? PKV_QJL64(3, true, false) : PKV_QJL64(0, true, false);
         if (lc.own_status) return td.pbits == 3 ? PKV_QJL64(3, false, true) : PKV_QJL64(0, false, true);
         return td.pbits == 3 ? PKV_QJL64(3, false, false) : PKV_QJL64(0, false, false);
@@ -3895,8 +3898,8 @@ int launch_turbo_encode(const LaunchCommon& lc, const TurboDev& td, const void* 
     if (td.dim == 128 && td.mode && td.qa && td.pbits <= 4) {
         if (nblocks > (1u << 29)) return hipErrorInvalidValue;   // 4 workgroups per tile
         const size_t lds = static_cast<size_t>(WAVES) * (16 * (lc.plen >> 2) + 4) * sizeof(uint32_t);
-#define PKV_QJL128(PB, DG, OW)                                                                                      \
-    launch_big_lds(turbo_encode_qjl128_kernel<PB, DG, OW>, 4 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl,   \
+#define PKV_QJL128(PB, DG, OW)                                                                                   \
+    launch_big_lds(turbo_encode_qjl128_kernel<PB, DG, OW>, 4 * nblocks, lds, st, lc, in, wire, td.signs, td.qjl, \
                    td.cs, td.qa, td.qb, td.seed, td.pbits, td.proj)
         if (lc.diag) return td.pbits == 3 ? PKV_QJL128(3, true, false) : PKV_QJL128(0, true, false);
         if (lc.own_status) return td.pbits == 3 ? PKV_QJL128(3, false, true) : PKV_QJL128(0, false, true);
@@ -3928,12 +3931,11 @@ int launch_turbo_decode(const LaunchCommon& lc, const TurboDev& td, const uint8_
 #define PKV_SPLIT64(PB, LO, OW)                                                                                  \
     launch_big_lds(turbo_decode_split_kernel<PB, LO, OW>, grid, lds, st, lc, wire, out, td.signs, td.cs, td.seed, \
                    td.pbits, td.proj, td.mode)
-        if (lc.own_status) {
-            if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT64(3, false, true) : PKV_SPLIT64(0, false, true);
-            return td.pbits == 3 ? PKV_SPLIT64(3, true, true) : PKV_SPLIT64(0, true, true);
-        }
-        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT64(3, false, false) : PKV_SPLIT64(0, false, false);
-        return td.pbits == 3 ? PKV_SPLIT64(3, true, false) : PKV_SPLIT64(0, true, false);
+        const bool lossy = lc.radii != PKV_RADII_F32;
+        if (lc.own_status && lossy) return td.pbits == 3 ? PKV_SPLIT64(3, true, true) : PKV_SPLIT64(0, true, true);
+        if (lc.own_status) return td.pbits == 3 ? PKV_SPLIT64(3, false, true) : PKV_SPLIT64(0, false, true);
+        if (lossy) return td.pbits == 3 ? PKV_SPLIT64(3, true, false) : PKV_SPLIT64(0, true, false);
+        return td.pbits == 3 ? PKV_SPLIT64(3, false, false) : PKV_SPLIT64(0, false, false);
 #undef PKV_SPLIT64
     }
     if (td.dim == 128 && td.pbits <= 4) {
@@ -3942,12 +3944,11 @@ int launch_turbo_decode(const LaunchCommon& lc, const TurboDev& td, const uint8_
 #define PKV_SPLIT128(PB, LO, OW)                                                                            \
     launch_big_lds(turbo_decode_split128_kernel<PB, LO, OW>, 4 * nblocks, lds, st, lc, wire, out, td.signs, \
                    td.cs, td.seed, td.pbits, td.proj)
-        if (lc.own_status) {
-            if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT128(3, false, true) : PKV_SPLIT128(0, false, true);
-            return td.pbits == 3 ? PKV_SPLIT128(3, true, true) : PKV_SPLIT128(0, true, true);
-        }
-        if (lc.radii == PKV_RADII_F32) return td.pbits == 3 ? PKV_SPLIT128(3, false, false) : PKV_SPLIT128(0, false, false);
-        return td.pbits == 3 ? PKV_SPLIT128(3, true, false) : PKV_SPLIT128(0, true, false);
+        const bool lossy = lc.radii != PKV_RADII_F32;
+        if (lc.own_status && lossy) return td.pbits == 3 ? PKV_SPLIT128(3, true, true) : PKV_SPLIT128(0, true, true);
+        if (lc.own_status) return td.pbits == 3 ? PKV_SPLIT128(3, false, true) : PKV_SPLIT128(0, false, true);
+        if (lossy) return td.pbits == 3 ? PKV_SPLIT128(3, true, false) : PKV_SPLIT128(0, true, false);
+        return td.pbits == 3 ? PKV_SPLIT128(3, false, false) : PKV_SPLIT128(0, false, false);
 #undef PKV_SPLIT128
     }
     if (td.dim == 64)
@@ -3993,10 +3994,10 @@ int launch_turbo_score(const LaunchCommon& lc, const TurboDev& td, const uint8_t
     (lc.radii == PKV_RADII_F32 ? (narrow ? PKV_SCORE(D, P, false, true) : PKV_SCORE(D, P, false, false))        \
                                : (narrow ? PKV_SCORE(D, P, true, true) : PKV_SCORE(D, P, true, false)))
     if ((td.pbits == 3 || td.pbits == 4) && proj <= 32) {   // table path: [pair][bin] terms in LDS
-#define PKV_LUT(D, P, PB)                                                                                      \
-    (lc.radii == PKV_RADII_F32                                                                                 \
+#define PKV_LUT(D, P, PB)                                                                                    \
+    (lc.radii == PKV_RADII_F32                                                                               \
          ? launch_big_lds(turbo_score_lut_kernel<D, P, false, PB>, nblocks, 0, st, lc, wire, prepared, nq,   \
-                          qstride, scores, ld, td.cs, td.seed, td.proj, qscale, post)                           \
+                          qstride, scores, ld, td.cs, td.seed, td.proj, qscale, post)                        \
          : launch_big_lds(turbo_score_lut_kernel<D, P, true, PB>, nblocks, 0, st, lc, wire, prepared, nq,    \
                           qstride, scores, ld, td.cs, td.seed, td.proj, qscale, post))
         if (td.dim == 64)
@@ -4010,9 +4011,12 @@ int launch_turbo_score(const LaunchCommon& lc, const TurboDev& td, const uint8_t
     }
     const bool narrow = td.dim == 128 && td.pbits <= 5;
     if (td.dim == 64) {
-        if (proj == 0) return lc.radii == PKV_RADII_F32 ? PKV_SCORE(64, 0, false, false) : PKV_SCORE(64, 0, true, false);
-        if (proj == 32) return lc.radii == PKV_RADII_F32 ? PKV_SCORE(64, 32, false, false) : PKV_SCORE(64, 32, true, false);
-        if (proj == 64) return lc.radii == PKV_RADII_F32 ? PKV_SCORE(64, 64, false, false) : PKV_SCORE(64, 64, true, false);
+        if (proj == 0)
+            return lc.radii == PKV_RADII_F32 ? PKV_SCORE(64, 0, false, false) : PKV_SCORE(64, 0, true, false);
+        if (proj == 32)
+            return lc.radii == PKV_RADII_F32 ? PKV_SCORE(64, 32, false, false) : PKV_SCORE(64, 32, true, false);
+        if (proj == 64)
+            return lc.radii == PKV_RADII_F32 ? PKV_SCORE(64, 64, false, false) : PKV_SCORE(64, 64, true, false);
     } else if (td.dim == 128) {
         if (proj == 0) return PKV_SCORE_R(128, 0);
         if (proj == 32) return PKV_SCORE_R(128, 32);

@@ -226,8 +226,9 @@ PKV_HD uint32_t octant_bin_m2(float a, float b, bool& near_line, bool& out_of_ra
 // instructions for the test on gfx950, |.| being a free source modifier):
 // g = |a| - |b|, unsafe = !(max(|a|, |b|, 2^-31) < min(|a|, |b|, |g|) * 2^16).
 // A pair it passes is one octant_bin_m2 passes, with the same bin, provided
-// fl(fl(a^2) + fl(b^2)) is finite (the kernels send every pair of a vector
-// whose radii do not sum to a finite value down the exact path):
+// fl(fl(a^2) + fl(b^2)) is finite (the kernels send every pair of a lane whose
+// squares do not sum to a finite value -- at head_dim 64 those of the vector
+// before its scale of 2^-3 -- down the exact path):
 //   * m3 * 2^16 is exact (no overflow: m3 <= mx < 2^64 when a^2, b^2 are
 //     finite), so m3 > mx 2^-16 = eps of octant_bin_m2 (exact for mx >
 //     2^-110), and m3 > 2^-47, so mx > 2^-47 > 1e-30; mx < 2^64 < 1e30;

@@ -19,7 +19,8 @@ def test_edges_of_the_fast_path(ctx, dim, bits, radii):
     one = np.zeros(dim)
     one[5] = 3.0
     rows += [one, -one, np.arange(dim) % 2]
-    for e in (-149, -140, -126, -100, -60, -48, -47, -46, -33, -32, -31, -30, -29, -28, -27, -16, 16, 40, 58, 59, 60, 61):
+    for e in (-149, -140, -126, -100, -60, -48, -47, -46, -33, -32, -31, -30, -29, -28, -27, -16, 16, 40, 58, 59, 60,
+              61):
         rows.append(rng.randn(dim) * 2.0 ** e)
         rows.append(rng.choice([-1.0, 1.0, 2.0], dim) * 2.0 ** e)
     rows += list(rng.randn(40, dim))

@@ -108,7 +108,8 @@ def test_blob_order_and_overlap(ctx):
     def encode(offsets):
         segs = segments([(k * n * 64, 0, 64, o, n, n) for k, o in enumerate(offsets)])
         prof.encode_segments(x.view(-1), segs, wire)
-    for offsets in ([0, blob, 2 * blob, 3 * blob], [3 * blob + 1, 0, 2 * blob + 1, blob], [7, 3 * blob, blob + 9, 4 * blob]):
+    for offsets in ([0, blob, 2 * blob, 3 * blob], [3 * blob + 1, 0, 2 * blob + 1, blob],
+                    [7, 3 * blob, blob + 9, 4 * blob]):
         encode(offsets)
         w = wire.cpu().numpy()
         for k, o in enumerate(offsets):
