@@ -3508,22 +3508,23 @@ __global__ __launch_bounds__(TILE) void fib_decode_mfma_kernel(LaunchCommon lc, 
     __syncthreads();
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t nhalf = 2u * tile_start[lc.nseg];
-    for (uint32_t hb = blockIdx.x; hb < nhalf; hb += gridDim.x) {
+    const uint64_t nhalf = 2ull * tile_start[lc.nseg];   // a bounded grid may walk 2^31 tiles
+    for (uint64_t hb = blockIdx.x; hb < nhalf; hb += gridDim.x) {
         // opaque per half-tile: the loop must not keep lane-derived addresses or
         // table reads live across half-tiles (register pressure)
         int zoff = 0, lane = threadIdx.x & 63;
         asm volatile("" : "+s"(zoff), "+v"(lane));
         const int h = lane >> 5, n = lane & 31;
-        const uint32_t sidx = segment_of(tile_seg, tile_start, lc.nseg, hb >> 1);
+        const uint32_t blk = static_cast<uint32_t>(hb >> 1);
+        const uint32_t sidx = segment_of(tile_seg, tile_start, lc.nseg, blk);
         const SegDev seg = segs[sidx];
         const uint8_t* blob = wire + seg.wire_offset;
         // Lane n's vector: two runs of 16, 32 apart -- when a blob holds 32 heads
         // (vector = token * H + head) the same 16 heads at consecutive tokens,
         // so the staged stores below write two adjacent rows per run.  Any
         // other layout is just another order.
-        const uint32_t r0 = ((hb >> 1) - tile_start[sidx]) * TILE + (hb & 1u) * (TILE / 2) + 64u * (wave >> 1) +
-                            16u * (wave & 1u);
+        const uint32_t r0 = (blk - tile_start[sidx]) * TILE + static_cast<uint32_t>(hb & 1u) * (TILE / 2) +
+                            64u * (wave >> 1) + 16u * (wave & 1u);
         const uint32_t vi = r0 + (static_cast<uint32_t>(n) & 15u) + 32u * (static_cast<uint32_t>(n) >> 4);
         const bool some = r0 < seg.n_vectors;   // wave-uniform
         const bool active = vi < seg.n_vectors;
@@ -4078,7 +4079,6 @@ int launch_fib_decode(const LaunchCommon& lc, const FibDev& fd, const uint8_t* w
                            fd.codebook);
         return hipGetLastError();
     }
-    if (nblocks > (1u << 30)) return hipErrorInvalidValue;   // 2 half-tiles per tile
     // The table of partial sums pays while the arithmetic is the bound; past
     // 12 output bytes per value the decode is bound by its writes and the
     // table's reads slow them down (a step of 1.2 M pool and 0.34 M shell

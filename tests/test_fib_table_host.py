@@ -1,7 +1,8 @@
 """The fib decode's table of partial sums as the host half keeps it, on the CPU
 with the HIP runtime replaced by tests/host_hip.cpp: a profile whose table cannot
 be allocated is created all the same and decodes by the kernel without one, and
-profiles with equal constants share a table."""
+profiles with equal constants share a table; a bounded decode walks any number of
+tiles a segment table may have."""
 import ctypes as C
 import os
 import subprocess
@@ -29,7 +30,7 @@ def _child(stub, name):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-@pytest.mark.parametrize("name", ["no_memory", "with_memory", "equal_constants"])
+@pytest.mark.parametrize("name", ["no_memory", "with_memory", "equal_constants", "many_tiles"])
 def test_profile_creation(stub, name):
     _child(stub, name)
 
@@ -104,6 +105,19 @@ def child_equal_constants(h):
     h.L.pkv_profile_destroy(b)
     h.L.pkv_profile_destroy(other)
     assert h.tables() == 0
+
+
+def child_many_tiles(h):
+    """More than 2^30 tiles of 256 vectors (one blob decoded again and again)."""
+    from provekv_amd.device import SEG_DTYPE
+    n, per = 1 << 24, 1 << 16   # vectors and tiles of a segment
+    segs = np.array([(0, 0, 0, 0, n, n)] * ((1 << 30) // per + 1), dtype=SEG_DTYPE)
+    status, buf = np.zeros(2 * len(segs), np.uint32), np.zeros(64, np.float32)
+    ptr = buf.ctypes.data + -buf.ctypes.data % 16
+    rc = h.L.pkv_decode_segments_bounded(h.ctx, h.profile(), 0, ptr, 19 + 12 * n, segs.ctypes.data, len(segs), ptr, 0,
+                                         64, 1, 0, 640, status.ctypes.data, None)
+    assert rc == 0, rc
+    assert "fib_decode_mfma_kernel" in h.hip.host_hip_launched().decode().split()[-1]
 
 
 if __name__ == "__main__":
